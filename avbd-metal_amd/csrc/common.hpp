@@ -22,6 +22,17 @@ constexpr float kPenaltyMaxT = 1.0e6f;   // tangential / soft normal cap
 constexpr float kStickThresh = 1.0e-5f;
 constexpr int kMaxColors = 64;
 constexpr int kMaxContacts = 8;
+constexpr uint32_t kColorPasses = 20;      // Jacobi passes of the dynamic coloring
+// Bodies of an island one workgroup colors / solves.  The solve crosses over
+// by contact density: one workgroup against the grid-wide persistent sweep
+// took 3.02 against 3.70 ms a frame on 125 cubes packed in a lattice, 4.08
+// against 3.73 on 216, but 0.55 against 0.72 on a loose heap of 300; the
+// line is where no density loses.  Coloring gains on all of these.
+constexpr uint32_t kIslandMax = 512;
+constexpr uint32_t kIslandSolveMax = 128;
+constexpr uint32_t kIslandFill = 64;       // bodies that small islands are gathered to in one workgroup
+constexpr uint32_t kIslandContacts = 2048; // contacts one island workgroup lists in LDS
+constexpr uint32_t kIslandThreads = 512;   // largest island workgroup
 constexpr uint32_t kWorld = 0xFFFFFFFFu;
 
 // force kinds packed in the top 4 bits of an adjacency entry

@@ -70,6 +70,8 @@ void launch_contact_adjacency(hipStream_t st, const DeviceState& S, const StepPa
 void launch_static_color_pass(hipStream_t st, const DeviceState& S, const StepParams& P, const uint32_t* in,
                               uint32_t* out);
 void launch_dynamic_coloring(hipStream_t st, const DeviceState& S, const StepParams& P);
+// colorStart / colorList of `colors` (CTR_COLOR_BASE counts zero on entry)
+void launch_color_buckets(hipStream_t st, const DeviceState& S, const StepParams& P, const uint32_t* colors);
 // primal specialisations of a color's bodies
 constexpr int kModeGeneral = 0;  // rigid bodies and particles, any entries
 constexpr int kModeTet = 1;      // particles whose static entries are all tets
@@ -82,13 +84,18 @@ void launch_primal_color(hipStream_t st, const DeviceState& S, const StepParams&
 void launch_primal_tail(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t first, int lanes);
 constexpr uint32_t kDynamicColorLaunches = 8;  // dynamic palette: colors launched one kernel each
 void launch_dual(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t gridCap);
-void launch_finalize(hipStream_t st, const DeviceState& S, const StepParams& P);
+// countColors: add the bodies of each color to CTR_COLOR_BASE
+void launch_finalize(hipStream_t st, const DeviceState& S, const StepParams& P, bool countColors);
 // guard: skip once a residual-terminated frame has ended its iterations
 void launch_residual(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t blocks, bool guard = false);
 void launch_residual_check(hipStream_t st, const DeviceState& S, uint32_t blocks, float tol, uint32_t maxIt,
                            uint32_t n, ConvHost* host);
 void launch_diag_error(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t* out, uint32_t gridCap);
 // persistent cooperative sweep: all iterations x colors x dual in one launch
+// island.hip: coloring (S.colorFlags zero on entry) and P.iterations sweeps, one workgroup of `threads` per island
+void launch_island_coloring(hipStream_t st, const DeviceState& S, uint32_t numIslands, uint32_t threads);
+void launch_island_solve(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t numIslands, int lanes,
+                         uint32_t threads);
 hipError_t launch_persistent_solve(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t numColors,
                                    int lanes, int mode, uint32_t gridBlocks, uint32_t barrierBase);
 int persistent_max_blocks(int lanes, int mode);

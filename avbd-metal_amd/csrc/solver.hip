@@ -16,6 +16,7 @@
 #include <mutex>
 #include <set>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/avbd.h"
@@ -92,6 +93,10 @@ struct avbd_solver {
   float elemCellSize = 0.0f, elemMargin = 0.0f, datQueryRadius = 0.0f, surfaceContactCellSize = 0.0f;
   float datQueryRadiusDerived = 0.0f;  // rq derived at create (a test hook may replace datQueryRadius)
   int lanes = 8, sweepMode = 1;
+  uint32_t numIslands = 0;       // island workgroups that color the dynamic palette (0: grid-wide coloring)
+  bool islandSolve = false;      // they also run the sweeps
+  uint32_t islandThreads = 64;   // their workgroup size
+  uint32_t largestIsland = 0;    // bodies of the largest
   int persistentBlocks = 0;
   uint32_t gridCap = 1024;
   hipStream_t stream = nullptr;
@@ -273,9 +278,10 @@ using StageFn = std::function<void(const char*)>;
 
 void enqueue_pre_solve(avbd_solver* s, const DeviceState& S, const StepParams& P, const StageFn& stage) {
   hipStream_t st = s->stream;
-  uint32_t* zp[5] = {S.counters, S.cellCount, S.cellRigid, S.dAdjCount, S.fineCount};
-  uint32_t zn[5] = {CTR_TOTAL, s->gridHashSize, s->gridHashSize, s->nb, s->fineCellSize > 0.0f ? s->gridHashSize : 0u};
-  launch_zero_multi(st, zp, zn, 5);
+  uint32_t* zp[6] = {S.counters, S.cellCount, S.cellRigid, S.dAdjCount, S.fineCount, S.colorFlags};
+  uint32_t zn[6] = {CTR_TOTAL, s->gridHashSize, s->gridHashSize, s->nb, s->fineCellSize > 0.0f ? s->gridHashSize : 0u,
+                    s->numIslands ? kColorPasses : 0u};
+  launch_zero_multi(st, zp, zn, 6);
   if (s->datOn) launch_fill_u32(st, S.datT, s->nb, 0x3F800000u);  // 1.0f: no pass has lowered a fraction
   if (!s->rateJoints.empty())
     launch_rate_motors(st, S, s->rateJointDev, s->rateValueDev, (uint32_t)s->rateJoints.size(), P.dt);
@@ -312,7 +318,10 @@ void enqueue_pre_solve(avbd_solver* s, const DeviceState& S, const StepParams& P
   }
   launch_contact_adjacency(st, S, P, s->gridCap);
   stage("adjacency");
-  if (s->dynamicColoring) launch_dynamic_coloring(st, S, P);
+  if (s->numIslands) {
+    launch_island_coloring(st, S, s->numIslands, s->islandThreads);
+    if (!s->islandSolve) launch_color_buckets(st, S, P, S.colors);
+  } else if (s->dynamicColoring) launch_dynamic_coloring(st, S, P);
   stage("coloring");
   // learned warm start: features, then (with a network) the learned start
   // and the residual comparison against the plain guess
@@ -348,6 +357,10 @@ hipError_t enqueue_iterations(avbd_solver* s, const DeviceState& S, const StepPa
   StepParams P = P0;
   P.iterations = iterations;
   if (iterations == 0) return hipSuccess;
+  if (s->islandSolve) {
+    launch_island_solve(st, S, P, s->numIslands, s->lanes, s->islandThreads);
+    return hipSuccess;
+  }
   if (s->sweepMode == 2) {
     if (clearBarrier) launch_fill_u32(st, S.counters + CTR_GBAR, 1, 0u);
     return launch_persistent_solve(st, S, P, s->dynamicColoring ? 0u : s->staticUsedColors, s->lanes, s->allMode,
@@ -379,7 +392,7 @@ void enqueue_post_solve(avbd_solver* s, const DeviceState& S, const StepParams& 
     launch_ws_target_rigid(s->stream, S, W);
   }
   launch_dat_restore(s->stream, S, P);
-  launch_finalize(s->stream, S, P);
+  launch_finalize(s->stream, S, P, s->islandSolve);
   launch_viscosity(s->stream, S, P);
   stage("finalize");
 }
@@ -1149,6 +1162,111 @@ void release_solver(avbd_solver* s) {
   delete s;
 }
 
+// Islands of a rigid scene: sets of dynamic bodies that no joint or spring
+// links and whose colliders never meet (40_solver's domain rule: colliders of
+// one nonzero group, group 0 with group 0, group 0 with the shared colliders
+// of any group).  The island kernels run when every island fits one
+// workgroup and the caller left the sweep mode open.
+avbd_status build_islands(avbd_solver* s, const avbd_scene_desc* d) {
+  if (!s->dynamicColoring || s->opts.sweep_mode != 0) return AVBD_OK;
+  std::vector<uint32_t> up(s->nb);
+  for (uint32_t b = 0; b < s->nb; b++) up[b] = b;
+  auto root = [&](uint32_t b) {
+    while (up[b] != b) b = up[b] = up[up[b]];
+    return b;
+  };
+  auto dynamic = [&](int64_t b) { return b >= 0 && s->mass[b] > 0.0f; };
+  auto join = [&](uint32_t a, uint32_t b) {
+    a = root(a);
+    b = root(b);
+    if (a != b) up[std::max(a, b)] = std::min(a, b);
+  };
+  for (uint32_t i = 0; i < s->nj; i++)
+    if (dynamic(d->joint_body_a[i]) && dynamic(d->joint_body_b[i])) join(d->joint_body_a[i], d->joint_body_b[i]);
+  for (uint32_t i = 0; i < s->ns; i++)
+    if (dynamic(d->spring_body_a[i]) && dynamic(d->spring_body_b[i])) join(d->spring_body_a[i], d->spring_body_b[i]);
+  std::unordered_map<uint32_t, uint32_t> first;  // collision group -> one of its dynamic bodies
+  std::vector<uint32_t> shared;                  // dynamic bodies that may meet group 0
+  for (uint32_t i = 0; i < d->num_colliders; i++) {
+    if (d->collider_enabled && !d->collider_enabled[i]) continue;
+    const uint32_t b = d->collider_body[i], g = d->collider_group ? d->collider_group[i] : 0u;
+    if (!dynamic(b)) continue;
+    const auto at = first.emplace(g, b);
+    if (!at.second) join(at.first->second, b);
+    if (g != 0u && (!d->collider_shared || d->collider_shared[i])) shared.push_back(b);
+  }
+  const auto zero = first.find(0u);
+  if (zero != first.end())
+    for (uint32_t b : shared) join(zero->second, b);
+  std::vector<uint32_t> size(s->nb, 0u), roots;
+  for (uint32_t b = 0; b < s->nb; b++)
+    if (dynamic(b) && size[root(b)]++ == 0u) roots.push_back(root(b));
+  if (roots.empty()) return AVBD_OK;
+  // similar islands next to each other: those with joints first (a wave of
+  // mixed islands runs both stamps' code), larger ones first
+  std::vector<uint8_t> jointed(s->nb, 0u);
+  for (uint32_t i = 0; i < s->nj; i++) {
+    if (dynamic(d->joint_body_a[i])) jointed[root(d->joint_body_a[i])] = 1u;
+    if (dynamic(d->joint_body_b[i])) jointed[root(d->joint_body_b[i])] = 1u;
+  }
+  std::stable_sort(roots.begin(), roots.end(), [&](uint32_t a, uint32_t b) {
+    return jointed[a] != jointed[b] ? jointed[a] > jointed[b] : size[a] > size[b];
+  });
+  uint32_t total = 0, widest = 0;
+  for (uint32_t r : roots) {
+    total += size[r];
+    widest = std::max(widest, size[r]);
+  }
+  if (widest > kIslandMax) return AVBD_OK;
+  // Small islands share a workgroup until it holds `fill` bodies, so that a
+  // color's lane groups fill its waves; with few bodies in all, every island
+  // keeps its own (the chip has room, and fewer bodies run fewer rounds).
+  const uint32_t fill = std::min<uint32_t>(kIslandFill, total / (2u * s->cus));
+  std::vector<uint32_t> id(s->nb, 0u), first_at(s->nb, 0u), start(1, 0u), local(s->nb, 0u);
+  uint32_t used = 0;
+  for (size_t k = 0; k < roots.size(); k++) {
+    const uint32_t r = roots[k];
+    if (k > 0 && (used - start.back() + size[r] > fill || jointed[r] != jointed[roots[k - 1]])) start.push_back(used);
+    id[r] = (uint32_t)start.size() - 1;
+    first_at[r] = used;
+    used += size[r];
+  }
+  start.push_back(used);
+  const uint32_t n = (uint32_t)start.size() - 1;
+  std::vector<uint32_t> jstart(n + 1, 0u), pstart(n + 1, 0u);
+  std::vector<uint32_t> body(total), jlist(std::max<uint32_t>(1, s->nj)), plist(std::max<uint32_t>(1, s->ns));
+  for (uint32_t b = 0; b < s->nb; b++) {
+    if (!dynamic(b)) continue;
+    const uint32_t r = root(b);
+    local[b] = first_at[r] - start[id[r]];
+    body[first_at[r]++] = b;
+  }
+  // a constraint follows its dynamic body; one without any goes to the first island
+  auto csr = [&](uint32_t count, auto owner, std::vector<uint32_t>& st, std::vector<uint32_t>& list) {
+    for (uint32_t i = 0; i < count; i++) st[owner(i) + 1]++;
+    for (uint32_t k = 0; k < n; k++) st[k + 1] += st[k];
+    std::vector<uint32_t> pos(st.begin(), st.end() - 1);
+    for (uint32_t i = 0; i < count; i++) list[pos[owner(i)]++] = i;
+  };
+  auto island = [&](int64_t a, int64_t b) { return dynamic(a) ? id[root((uint32_t)a)] : dynamic(b) ? id[root((uint32_t)b)] : 0u; };
+  csr(s->nj, [&](uint32_t i) { return island(d->joint_body_a[i], d->joint_body_b[i]); }, jstart, jlist);
+  csr(s->ns, [&](uint32_t i) { return island(d->spring_body_a[i], d->spring_body_b[i]); }, pstart, plist);
+  DeviceState& S = s->S;
+  if (dev_alloc(s, &S.islandStart, start.size()) || dev_alloc(s, &S.islandBody, body.size()) ||
+      dev_alloc(s, &S.islandLocal, local.size()) || dev_alloc(s, &S.islandJointStart, jstart.size()) ||
+      dev_alloc(s, &S.islandJoint, jlist.size()) || dev_alloc(s, &S.islandSpringStart, pstart.size()) ||
+      dev_alloc(s, &S.islandSpring, plist.size()))
+    return AVBD_ERR_ALLOC;
+  if (upload(S.islandStart, start) || upload(S.islandBody, body) || upload(S.islandLocal, local) ||
+      upload(S.islandJointStart, jstart) || upload(S.islandJoint, jlist) || upload(S.islandSpringStart, pstart) ||
+      upload(S.islandSpring, plist))
+    return AVBD_ERR_HIP;
+  s->numIslands = n;
+  s->islandSolve = widest <= kIslandSolveMax;
+  for (uint32_t k = 0; k < n; k++) s->largestIsland = std::max(s->largestIsland, start[k + 1] - start[k]);
+  return AVBD_OK;
+}
+
 avbd_status build_static_and_upload(avbd_solver* s, const avbd_scene_desc* d) {
   const uint32_t nb = d->num_bodies;
   s->nb = nb;
@@ -1797,7 +1915,9 @@ avbd_status build_static_and_upload(avbd_solver* s, const avbd_scene_desc* d) {
   s->gridCap = (uint32_t)std::max(256, 8 * cus);
   s->cus = (uint32_t)std::max(1, cus);
   create_phase(s, "runtime resources");
-  return AVBD_OK;
+  const avbd_status islands = build_islands(s, d);
+  create_phase(s, "islands");
+  return islands;
 }
 
 // Static palette: Jacobi fixed point of the greedy rule on the GPU, then
@@ -1913,6 +2033,15 @@ avbd_status static_coloring(avbd_solver* s) {
   return AVBD_OK;
 }
 
+// Workgroup size of the island kernels: enough lane groups for the larger
+// color of the largest island (two colors share a stack or chain about
+// evenly), at most kIslandThreads.
+constexpr int kIslandLanes = 4;
+uint32_t island_threads(const avbd_solver* s) {
+  const uint32_t want = (s->largestIsland + 1) / 2 * (uint32_t)kIslandLanes;
+  return std::min<uint32_t>(kIslandThreads, std::max<uint32_t>(64u, (want + 63u) / 64u * 64u));
+}
+
 // Times primal sweeps / iterations for each lane split and sweep mode on the
 // initial state, then restores every buffer the trials touched.
 void autotune(avbd_solver* s) {
@@ -1929,6 +2058,12 @@ void autotune(avbd_solver* s) {
   if (s->dynamicColoring && wantMode == 0) modeCands = {2, 1};
   // cloth: the Planar-DAT passes run between the colors' launches
   if (s->datOn || s->isoOn) modeCands = {1};
+  s->islandThreads = island_threads(s);
+  if (s->islandSolve) {
+    s->lanes = laneCands.size() == 1 ? laneCands[0] : kIslandLanes;
+    s->sweepMode = 2;
+    return;
+  }
   if (laneCands.size() == 1 && modeCands.size() == 1) {
     s->lanes = laneCands[0];
     s->sweepMode = modeCands[0];
@@ -2981,6 +3116,10 @@ extern "C" avbd_status avbd_time_primal(avbd_solver* s, int32_t reps, float* avg
       }
     }
   };
+  if (s->islandSolve) {  // the island kernels order their colors themselves: build the grid-wide lists
+    launch_fill_u32(s->stream, S.counters + CTR_COLOR_BASE, kMaxColors, 0u);
+    launch_color_buckets(s->stream, S, P, S.colors);
+  }
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipError_t he = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);

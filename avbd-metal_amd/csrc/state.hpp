@@ -69,6 +69,12 @@ struct DeviceState {
   // colors
   uint32_t *colors, *colorsB, *colorList, *colorStart, *bodySlot;
   U4* colorWork;              // static palette, color order: (body, static CSR start, count, 0)
+  // island workgroups of a dynamic-palette scene (null when the island path
+  // is off): islandStart[k] .. islandStart[k + 1] of islandBody, one or more
+  // whole islands each, a single island's bodies ascending; per body its
+  // position inside its workgroup; the joints and springs of each
+  uint32_t *islandStart, *islandBody, *islandLocal;
+  uint32_t *islandJointStart, *islandJoint, *islandSpringStart, *islandSpring;
   // start-of-iteration pose snapshot: contact partners that share the
   // body's color are read from here, so a same-color contact is a Jacobi
   // coupling with a schedule-independent result

@@ -210,7 +210,7 @@ void avbd_scene_free(avbd_scene_desc* d);
 typedef struct avbd_options {
     int32_t max_pairs_per_body;        /* 16; maxPairs = max(4096, colliders * this), negative -> 16 */
     int32_t lanes_per_body;            /* 0 = autotune; else 4, 8, 16 or 32 lanes per body in the primal sweep */
-    int32_t sweep_mode;                /* 0 = autotune, 1 = one launch per color, 2 = persistent cooperative sweep */
+    int32_t sweep_mode;                /* 0 = automatic, 1 = one launch per color, 2 = persistent cooperative sweep */
     int32_t use_graph;                 /* 1 = capture each step in a hipGraph (default), 0 = eager launches */
     int32_t pair_capacity_override;    /* test hook (planarDATPairCapacityForTesting analogue): >0 caps rigid pairs */
     int32_t dat_pair_capacity_override;  /* test hook, planarDATPairCapacityForTesting (GPUSolver.swift:2119): >0 caps the V-T/E-E stream */
@@ -321,7 +321,7 @@ typedef struct avbd_stats {
     int32_t color_conflicts;
     int32_t uses_dynamic_coloring;
     int32_t lanes_per_body;        /* primal lane split in use */
-    int32_t sweep_mode;            /* 1 per-color launches, 2 persistent */
+    int32_t sweep_mode;            /* 1 per-color launches, 2 persistent (the whole grid, or one workgroup per island) */
     int32_t dat_pairs;             /* lastPlanarDATPairs: V-T + E-E pair demand */
     int32_t dat_vt_pairs;          /* lastPlanarDATVertexTrianglePairs */
     int32_t dat_ee_pairs;          /* lastPlanarDATEdgeEdgePairs */
