@@ -185,13 +185,25 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 constexpr uint32_t kFineCap = 128;  // accepted candidates one wave sorts in LDS
 
+// The count pass keeps a producer's first kStash partners, slot-major, so
+// that emitting copies them instead of walking the cells again; producers
+// with more are listed and emitted by the wave path.
+__device__ __forceinline__ void bp_stash(const DeviceState& S, const StepParams& P, uint32_t producer, uint32_t k,
+                                         uint32_t partner) {
+  if (k < kStash) S.pairStash[k * (P.numHashed + P.numGlobals) + producer] = partner;
+}
+__device__ __forceinline__ void bp_count(const DeviceState& S, uint32_t producer, uint32_t count) {
+  S.pairCount[producer] = count;
+  if (count > kStash) S.bpBig[atomicAdd(&S.counters[CTR_BP_BIG], 1u)] = producer;
+}
+
 // One wave per producer (a hashed collider scanning its 27 neighbour cells
 // and the global list, or a global collider scanning the later globals).
 // Lanes split the producer's linearised candidate list; a ballot ranks the
 // accepted candidates so the emission order equals the serial order --
 // cells in (dz, dy, dx) order, each bucket in collider order, then globals.
-// Pass 1 (EMIT = false) writes the per-producer count, pass 2 emits at the
-// scanned offset.
+// Pass 1 (EMIT = false) writes the per-producer count and stashes the first
+// kStash partners; the emit pass runs only for producers with more.
 // With the candidate search grid (P.fineCellSize > 0: hash cells much larger
 // than the colliders), a hashed producer instead scans its 27 search cells,
 // applies the same filters, keys every accepted candidate by (position of
@@ -206,11 +218,12 @@ __device__ __forceinline__ void bp_producer(const DeviceState& S, const StepPara
   const uint64_t ltMask = lane ? ((~0ull) >> (64 - lane)) : 0ull;
   const uint32_t base = EMIT ? S.pairStart[producer] : 0u;
   uint32_t count = 0;
-  auto emitRanked = [&](bool accept, uint32_t a, uint32_t b) {
+  auto emitRanked = [&](bool accept, uint32_t a, uint32_t b) {  // a: the producer's collider
     uint64_t mask = __ballot(accept);
-    if (EMIT && accept) {
-      uint32_t slot = base + count + (uint32_t)__builtin_popcountll(mask & ltMask);
-      if (slot < P.maxPairs) S.pairs[slot] = U2{a, b};
+    if (accept) {
+      const uint32_t k = count + (uint32_t)__builtin_popcountll(mask & ltMask);
+      if (!EMIT) bp_stash(S, P, producer, k, b);
+      else if (base + k < P.maxPairs) S.pairs[base + k] = a < b ? U2{a, b} : U2{b, a};
     }
     count += (uint32_t)__builtin_popcountll(mask);
   };
@@ -372,7 +385,7 @@ __device__ __forceinline__ void bp_producer(const DeviceState& S, const StepPara
                              S.colliderShared[b], S.posLin[ownerB].w > 0.0f, collider_center(S, b),
                              fabsf(S.colliderShape[b].w));
       }
-      emitRanked(accept, a < b ? a : b, a < b ? b : a);
+      emitRanked(accept, a, b);
     }
   } else {
     const uint32_t gp = producer - P.numHashed;
@@ -395,53 +408,48 @@ __device__ __forceinline__ void bp_producer(const DeviceState& S, const StepPara
                              S.colliderShared[b], S.posLin[ownerB].w > 0.0f, collider_center(S, b),
                              fabsf(S.colliderShape[b].w));
       }
-      emitRanked(accept, a < b ? a : b, a < b ? b : a);
+      emitRanked(accept, a, b);
     }
   }
-  if (!EMIT && lane == 0) S.pairCount[producer] = count;
+  if (!EMIT && lane == 0) bp_count(S, producer, count);
 }
 
-// The wave path: one wave per producer of bpWave[0, bpWaveCount) -- the
+// The wave path: one wave per producer of bpWave -- the
 // producers not on the lane list (globals, hashed producers of small dense
 // packings), then those the lane path deferred this frame.
 template <bool EMIT>
 __global__ void __launch_bounds__(256) k_bp_pairs(DeviceState S, StepParams P) {
   __shared__ uint64_t fineKeys[4][2][kFineCap];
-  const uint32_t n = S.bpWaveCount[0];
+  const uint32_t n = EMIT ? S.counters[CTR_BP_BIG] : P.numBpWave + S.counters[CTR_BP_DEFER];
   for (uint32_t w = blockIdx.x * 4 + (threadIdx.x >> 6); w < n; w += gridDim.x * 4)
-    bp_producer<EMIT>(S, P, S.bpWave[w], fineKeys);
+    bp_producer<EMIT>(S, P, EMIT ? S.bpBig[w] : S.bpWave[w], fineKeys);
 }
 
 // Hashed producers on the lane path, one lane each, with the wave path's
-// filters and order: the 27 neighbour cells in (dz, dy, dx) order (a hash met
-// earlier in that order is not walked again), each bucket in collider order,
-// then the globals.  A soft-group particle with no hashed non-particle
-// collider in the scene skips the cells.  Under the candidate search grid the
-// lane gathers its accepted partners from the 27 search cells, keys each by
-// (position of its hash bucket in the visit order, collider id) and keeps up
-// to kLaneCap of them sorted in registers -- the walk's set and order, as on
-// the wave path.  A producer with more than kLaneCandidates candidates in its
-// cells, or more than kLaneCap accepted search-grid partners, goes to the
-// wave path: the count pass appends it to bpWave (one atomic per wave), the
-// emit pass reaches the same decision and leaves it there.  The lane list
-// (built at create) holds every hashed producer without the search grid or
-// when there are many of them (one lane each hides the walk's latency better
-// than one wave each), else the soft-group particles that scan only globals.
+// filters and order: the cells, then the globals.  Soft-group particles of a
+// scene with no hashed non-particle collider skip the cells.  Under the
+// candidate search grid the lane gathers its accepted partners from the 27
+// search cells, keys each by (position of its hash bucket in the visit
+// order, collider id) and keeps up to kLaneCap of them sorted in registers --
+// the walk's set and order, as on the wave path.  A producer with more than
+// kLaneCandidates candidates in its cells, or more than kLaneCap accepted
+// search-grid partners, goes to the wave path (one append per wave).
+// Without the search grid the cells are walked by eight lanes a producer,
+// k_bp_group.
 constexpr uint32_t kLaneCap = 8;
-constexpr uint32_t kLaneCandidates = 64;
+constexpr uint32_t kLaneCandidates = 64, kGroupCandidates = 128;
 
-__device__ __forceinline__ void bp_defer(const DeviceState& S, bool defer, uint32_t producer) {
+__device__ __forceinline__ void bp_defer(const DeviceState& S, const StepParams& P, bool defer, uint32_t producer) {
   const uint64_t m = __ballot(defer);
   if (m == 0ull) return;
   const uint32_t lane = __lane_id();
   const uint32_t leader = (uint32_t)(__ffsll((unsigned long long)__activemask()) - 1);
   uint32_t base = 0;
-  if (lane == leader) base = atomicAdd(S.bpWaveCount, (uint32_t)__popcll(m));
+  if (lane == leader) base = atomicAdd(&S.counters[CTR_BP_DEFER], (uint32_t)__popcll(m));
   base = __shfl(base, (int)leader, 64);
-  if (defer) S.bpWave[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = producer;
+  if (defer) S.bpWave[P.numBpWave + base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = producer;
 }
 
-template <bool EMIT>
 __global__ void __launch_bounds__(256) k_bp_lane(DeviceState S, StepParams P) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= P.numBpLane) return;
@@ -453,100 +461,71 @@ __global__ void __launch_bounds__(256) k_bp_lane(DeviceState S, StepParams P) {
   const bool aDyn = (ma.z & 2u) != 0;
   const V3 pa = xyz(ca);
   const float ra = ca.w;
-  const bool cells = !(ga != 0 && P.numHashedRigid == 0);
-  const bool fine = P.fineCellSize > 0.0f;
-  // the 27 cells walked (hash cells, or search cells under the search grid)
-  // and their ranges, duplicates and skipped cells empty
-  uint32_t h[27], cs[27], cc[27];
-  uint32_t total = 0;
-  int cx = 0, cy = 0, cz = 0;
-  if (cells) {
+  uint32_t count = 0;
+  if (P.fineCellSize > 0.0f && !(ga != 0 && P.numHashedRigid == 0)) {
+    // the 27 search cells and their ranges, duplicates and skipped cells empty
+    uint32_t h[27], cs[27], cc[27];
+    uint32_t total = 0;
+    int cx, cy, cz, wx, wy, wz;
     cell_coord(pa, P.cellSize, cx, cy, cz);
 #pragma unroll
     for (int q = 0; q < 27; q++)
       h[q] = cell_hash(cx + q % 3 - 1, cy + (q / 3) % 3 - 1, cz + q / 9 - 1, grpA, P.gridHashSize);
-    int wx = cx, wy = cy, wz = cz;
-    if (fine) cell_coord(pa, P.fineCellSize, wx, wy, wz);
+    cell_coord(pa, P.fineCellSize, wx, wy, wz);
 #pragma unroll
     for (int q = 0; q < 27; q++) {
-      const uint32_t hq =
-          fine ? cell_hash(wx + q % 3 - 1, wy + (q / 3) % 3 - 1, wz + q / 9 - 1, grpA, P.gridHashSize) : h[q];
+      const uint32_t hq = cell_hash(wx + q % 3 - 1, wy + (q / 3) % 3 - 1, wz + q / 9 - 1, grpA, P.gridHashSize);
       bool dup = false;
 #pragma unroll
       for (int j = 0; j < q; j++)
-        dup |= (fine ? cell_hash(wx + j % 3 - 1, wy + (j / 3) % 3 - 1, wz + j / 9 - 1, grpA, P.gridHashSize) : h[j]) ==
-               hq;
-      const bool skip = dup || (!fine && ga != 0 && S.cellRigid[hq] == 0);
-      cs[q] = skip ? 0u : (fine ? S.fineStart[hq] : S.cellStart[hq]);
-      cc[q] = skip ? 0u : (fine ? S.fineCount[hq] : S.cellCount[hq]);
+        dup |= cell_hash(wx + j % 3 - 1, wy + (j / 3) % 3 - 1, wz + j / 9 - 1, grpA, P.gridHashSize) == hq;
+      cs[q] = dup ? 0u : S.fineStart[hq];
+      cc[q] = dup ? 0u : S.fineCount[hq];
       total += cc[q];
     }
-  }
-  bool defer = total > kLaneCandidates;
-  uint64_t keys[kLaneCap];
-  uint32_t nAcc = 0;
-  if (!defer && cells && fine) {
+    bool defer = total > kLaneCandidates;
+    uint64_t keys[kLaneCap];
 #pragma unroll
     for (uint32_t k = 0; k < kLaneCap; k++) keys[k] = ~0ull;
+    if (!defer) {
 #pragma unroll
-    for (int q = 0; q < 27; q++) {
-      for (uint32_t k = cs[q]; k < cs[q] + cc[q]; k++) {
-        const uint32_t g = S.fineBodies[k];
-        const uint32_t b = S.hashedIdx[g];
-        if (b <= a) continue;
-        const U4 mb = S.hashMeta[g];
-        const F4 cb = S.hashCenter[g];
-        if ((ga != 0 && mb.w != 0) ||
-            !pair_accept(S, P, ownerA, grpA, shA, aDyn, pa, ra, mb.x, mb.y, mb.z & 1u, (mb.z & 2u) != 0, xyz(cb),
-                         cb.w))
-          continue;
-        int bx, by, bz;
-        cell_coord(xyz(cb), P.cellSize, bx, by, bz);
-        const uint32_t hb = cell_hash(bx, by, bz, S.colliderGroup[b], P.gridHashSize);
-        if (ga != 0 && S.cellRigid[hb] == 0) continue;
-        uint32_t pos = 27;
+      for (int q = 0; q < 27; q++) {
+        for (uint32_t k = cs[q]; k < cs[q] + cc[q]; k++) {
+          const uint32_t g = S.fineBodies[k];
+          const uint32_t b = S.hashedIdx[g];
+          if (b <= a) continue;
+          const U4 mb = S.hashMeta[g];
+          const F4 cb = S.hashCenter[g];
+          if ((ga != 0 && mb.w != 0) ||
+              !pair_accept(S, P, ownerA, grpA, shA, aDyn, pa, ra, mb.x, mb.y, mb.z & 1u, (mb.z & 2u) != 0, xyz(cb),
+                           cb.w))
+            continue;
+          int bx, by, bz;
+          cell_coord(xyz(cb), P.cellSize, bx, by, bz);
+          const uint32_t hb = cell_hash(bx, by, bz, S.colliderGroup[b], P.gridHashSize);
+          if (ga != 0 && S.cellRigid[hb] == 0) continue;
+          uint32_t pos = 27;
 #pragma unroll
-        for (int j = 26; j >= 0; j--) pos = h[j] == hb ? (uint32_t)j : pos;
-        if (pos == 27) continue;
-        // sorted insertion (ascending keys; static register indices)
-        uint64_t x = ((uint64_t)pos << 32) | b;
+          for (int j = 26; j >= 0; j--) pos = h[j] == hb ? (uint32_t)j : pos;
+          if (pos == 27) continue;
+          // sorted insertion (ascending keys; static register indices)
+          uint64_t x = ((uint64_t)pos << 32) | b;
 #pragma unroll
-        for (uint32_t m = 0; m < kLaneCap; m++) {
-          const uint64_t lo = keys[m] < x ? keys[m] : x, hi = keys[m] < x ? x : keys[m];
-          keys[m] = lo;
-          x = hi;
+          for (uint32_t m = 0; m < kLaneCap; m++) {
+            const uint64_t lo = keys[m] < x ? keys[m] : x, hi = keys[m] < x ? x : keys[m];
+            keys[m] = lo;
+            x = hi;
+          }
+          count++;
         }
-        nAcc++;
       }
+      defer = count > kLaneCap;
     }
-    defer = nAcc > kLaneCap;
-  }
-  if (!EMIT) bp_defer(S, defer, producer);
-  if (defer) return;
-  const uint32_t base = EMIT ? S.pairStart[producer] : 0u;
-  uint32_t count = 0;
-  auto emit = [&](uint32_t x, uint32_t y) {
-    if (EMIT && base + count < P.maxPairs) S.pairs[base + count] = U2{x, y};
-    count++;
-  };
-  if (cells && fine) {
+    bp_defer(S, P, defer, producer);
+    if (defer) return;
 #pragma unroll
     for (uint32_t k = 0; k < kLaneCap; k++)
-      if (k < nAcc) emit(a, (uint32_t)(keys[k] & 0xFFFFFFFFull));
-  } else if (cells) {
-#pragma unroll
-    for (int q = 0; q < 27; q++) {
-      for (uint32_t k = cs[q]; k < cs[q] + cc[q]; k++) {
-        const uint32_t b = S.cellBodies[k];
-        if (b <= a) continue;
-        const U4 mb = S.cellMeta[k];
-        const F4 cb = S.cellPos[k];
-        if (!(ga != 0 && mb.w != 0) &&
-            pair_accept(S, P, ownerA, grpA, shA, aDyn, pa, ra, mb.x, mb.y, mb.z & 1u, (mb.z & 2u) != 0, xyz(cb),
-                        cb.w))
-          emit(a, b);
-      }
-    }
+      if (k < count) bp_stash(S, P, producer, k, (uint32_t)(keys[k] & 0xFFFFFFFFull));
   }
   for (uint32_t g = 0; g < P.numGlobals; g++) {
     const uint32_t b = S.globalIdx[g];
@@ -554,17 +533,126 @@ __global__ void __launch_bounds__(256) k_bp_lane(DeviceState S, StepParams P) {
     if (!(ga != 0 && S.clothGroup[ownerB] == ga) &&
         pair_accept(S, P, ownerA, grpA, shA, aDyn, pa, ra, ownerB, S.colliderGroup[b], S.colliderShared[b],
                     S.posLin[ownerB].w > 0.0f, collider_center(S, b), fabsf(S.colliderShape[b].w)))
-      emit(a < b ? a : b, a < b ? b : a);
+      bp_stash(S, P, producer, count++, b);
   }
-  if (!EMIT) S.pairCount[producer] = count;
+  bp_count(S, producer, count);
 }
 
-__global__ void k_bp_finalize(DeviceState S, StepParams P) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  uint32_t producers = P.numHashed + P.numGlobals;
-  uint32_t n = producers == 0 ? 0 : S.pairStart[producers - 1] + S.pairCount[producers - 1];
-  S.counters[CTR_PAIR_CANDIDATES] = n;
-  S.counters[CTR_PAIRS] = n < P.maxPairs ? n : P.maxPairs;
+// The cell walk without the search grid, eight lanes per hashed producer:
+// each lane takes three or four consecutive cells of the 27, so lane order
+// is visit order and a scan of the lanes' counts gives every partner its
+// place.  One lane per producer was a chain of 27 dependent walks: 64 us for
+// 300 producers, 133 us for 94000, and the same again to emit; this takes 26
+// and 97 us, the stash copy 3 us.
+constexpr uint32_t kGroupLanes = 8;
+constexpr uint32_t kGroupCells = 4;
+__global__ void __launch_bounds__(256) k_bp_group(DeviceState S, StepParams P) {
+  __shared__ uint32_t found[kStash][256];  // each lane's first partners
+  const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / kGroupLanes;
+  const uint32_t lane = threadIdx.x % kGroupLanes;
+  if (i >= P.numBpLane) return;
+  const uint32_t producer = S.bpLane[i];
+  const uint32_t a = S.hashedIdx[producer];
+  const U4 ma = S.hashMeta[producer];
+  const F4 ca = S.hashCenter[producer];
+  const uint32_t ownerA = ma.x, grpA = ma.y, shA = ma.z & 1u, ga = ma.w;
+  const bool aDyn = (ma.z & 2u) != 0;
+  const V3 pa = xyz(ca);
+  const float ra = ca.w;
+  uint32_t count = 0;
+  if (!(ga != 0 && P.numHashedRigid == 0)) {
+    int cx, cy, cz;
+    cell_coord(pa, P.cellSize, cx, cy, cz);
+    auto hash = [&](int q) {
+      return cell_hash(cx + q % 3 - 1, cy + (q / 3) % 3 - 1, cz + q / 9 - 1, grpA, P.gridHashSize);
+    };
+    const uint32_t q0 = lane * 27u / kGroupLanes, q1 = (lane + 1u) * 27u / kGroupLanes;
+    uint32_t h[kGroupCells], cs[kGroupCells], cc[kGroupCells];
+    bool dup[kGroupCells];
+#pragma unroll
+    for (uint32_t k = 0; k < kGroupCells; k++) {
+      h[k] = hash((int)(q0 + k));
+      dup[k] = q0 + k >= q1;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 26; j++) {  // a bucket met earlier in the visit order is not walked again
+      const uint32_t hj = hash((int)j);
+#pragma unroll
+      for (uint32_t k = 0; k < kGroupCells; k++) dup[k] |= j < q0 + k && hj == h[k];
+    }
+    uint32_t total = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kGroupCells; k++) {
+      const bool skip = dup[k] || (ga != 0 && S.cellRigid[h[k]] == 0);
+      cs[k] = skip ? 0u : S.cellStart[h[k]];
+      cc[k] = skip ? 0u : S.cellCount[h[k]];
+      total += cc[k];
+    }
+#pragma unroll
+    for (uint32_t d = 1; d < kGroupLanes; d <<= 1) total += __shfl_xor(total, (int)d, 64);
+    const bool defer = total > kGroupCandidates;
+    bp_defer(S, P, defer && lane == 0, producer);
+    if (defer) return;
+    uint32_t n = 0;
+#pragma unroll
+    for (uint32_t c = 0; c < kGroupCells; c++) {
+      for (uint32_t k = cs[c]; k < cs[c] + cc[c]; k++) {
+        const uint32_t b = S.cellBodies[k];
+        if (b <= a) continue;
+        const U4 mb = S.cellMeta[k];
+        const F4 cb = S.cellPos[k];
+        if (!(ga != 0 && mb.w != 0) &&
+            pair_accept(S, P, ownerA, grpA, shA, aDyn, pa, ra, mb.x, mb.y, mb.z & 1u, (mb.z & 2u) != 0, xyz(cb),
+                        cb.w)) {
+          if (n < kStash) found[n][threadIdx.x] = b;
+          n++;
+        }
+      }
+    }
+    uint32_t incl = n;
+#pragma unroll
+    for (uint32_t d = 1; d < kGroupLanes; d <<= 1) {
+      const uint32_t y = __shfl_up(incl, d, kGroupLanes);
+      if (lane >= d) incl += y;
+    }
+    for (uint32_t k = 0; k < n && k < kStash; k++) bp_stash(S, P, producer, incl - n + k, found[k][threadIdx.x]);
+    count = __shfl(incl, kGroupLanes - 1, kGroupLanes);
+  }
+  const uint32_t shift = (threadIdx.x & 63u) - lane;  // the group's bits of a wave ballot
+  for (uint32_t g0 = 0; g0 < P.numGlobals; g0 += kGroupLanes) {
+    const uint32_t g = g0 + lane;
+    bool accept = false;
+    uint32_t b = 0;
+    if (g < P.numGlobals) {
+      b = S.globalIdx[g];
+      const uint32_t ownerB = S.colliderOwner[b];
+      accept = !(ga != 0 && S.clothGroup[ownerB] == ga) &&
+               pair_accept(S, P, ownerA, grpA, shA, aDyn, pa, ra, ownerB, S.colliderGroup[b], S.colliderShared[b],
+                           S.posLin[ownerB].w > 0.0f, collider_center(S, b), fabsf(S.colliderShape[b].w));
+    }
+    const uint32_t mask = (uint32_t)(__ballot(accept) >> shift) & ((1u << kGroupLanes) - 1u);
+    if (accept) bp_stash(S, P, producer, count + (uint32_t)__popc(mask & ((1u << lane) - 1u)), b);
+    count += (uint32_t)__popc(mask);
+  }
+  if (lane == 0) bp_count(S, producer, count);
+}
+
+// Copies the stashed partners to their places and sets the pair counters;
+// every pair is (smaller, larger collider).
+__global__ void __launch_bounds__(256) k_bp_emit(DeviceState S, StepParams P) {
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x, producers = P.numHashed + P.numGlobals;
+  if (p >= producers) return;
+  const uint32_t n = S.pairCount[p], base = S.pairStart[p];
+  if (p == producers - 1) {
+    S.counters[CTR_PAIR_CANDIDATES] = base + n;
+    S.counters[CTR_PAIRS] = base + n < P.maxPairs ? base + n : P.maxPairs;
+  }
+  if (n == 0 || n > kStash) return;
+  const uint32_t a = p < P.numHashed ? S.hashedIdx[p] : S.globalIdx[p - P.numHashed];
+  for (uint32_t k = 0; k < n && base + k < P.maxPairs; k++) {
+    const uint32_t b = S.pairStash[k * producers + p];
+    S.pairs[base + k] = a < b ? U2{a, b} : U2{b, a};
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -629,16 +717,18 @@ void launch_broadphase(hipStream_t st, const DeviceState& S, const StepParams& P
     // deferred lane producers (the kernel loops over its list)
     const uint32_t deferred = blocks_for(P.numBpLane, 4);
     const uint32_t waveBlocks = blocks_for(P.numBpWave, 4) + (deferred < 1024u ? deferred : 1024u);
-    launch_fill_u32(st, S.bpWaveCount, 1u, P.numBpWave);
-    if (P.numBpLane > 0)
-      hipLaunchKernelGGL(k_bp_lane<false>, dim3(blocks_for(P.numBpLane, 256)), dim3(256), 0, st, S, P);
+    if (P.numBpLane > 0) {
+      if (P.bpGroup)
+        hipLaunchKernelGGL(k_bp_group, dim3(blocks_for(P.numBpLane * kGroupLanes, 256)), dim3(256), 0, st, S, P);
+      else
+        hipLaunchKernelGGL(k_bp_lane, dim3(blocks_for(P.numBpLane, 256)), dim3(256), 0, st, S, P);
+    }
     if (waveBlocks > 0) hipLaunchKernelGGL(k_bp_pairs<false>, dim3(waveBlocks), dim3(256), 0, st, S, P);
     launch_exclusive_scan(st, S.pairCount, S.pairStart, producers, S.scanScratch);
-    if (P.numBpLane > 0)
-      hipLaunchKernelGGL(k_bp_lane<true>, dim3(blocks_for(P.numBpLane, 256)), dim3(256), 0, st, S, P);
-    if (waveBlocks > 0) hipLaunchKernelGGL(k_bp_pairs<true>, dim3(waveBlocks), dim3(256), 0, st, S, P);
+    hipLaunchKernelGGL(k_bp_emit, dim3(blocks_for(producers, 256)), dim3(256), 0, st, S, P);
+    const uint32_t bigBlocks = blocks_for(producers, 4);
+    hipLaunchKernelGGL(k_bp_pairs<true>, dim3(bigBlocks < 1024u ? bigBlocks : 1024u), dim3(256), 0, st, S, P);
   }
-  hipLaunchKernelGGL(k_bp_finalize, dim3(1), dim3(64), 0, st, S, P);
 }
 
 void launch_map_rebuild(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t gridCap) {

@@ -102,6 +102,8 @@ enum Counter : uint32_t {
   CTR_OGC_ARRIVE,          // workgroups of the running refresh check that have read CTR_OGC
   CTR_OGC_TRUNC,           // truncations this frame
   CTR_OGC_REFRESH,         // refreshes fired this frame
+  CTR_BP_DEFER,            // pair producers the lane / group paths passed to the wave path
+  CTR_BP_BIG,              // producers with more partners than the stash holds
   CTR_TOTAL = 16 + 2 * kMaxColors + 24
 };
 
@@ -429,6 +431,7 @@ struct StepParams {
   uint32_t numBodies, numColliders, numJoints, numSprings, numTets;
   uint32_t mapCapacity, maxPairs, gridHashSize, numHashed, numGlobals, numHashedRigid;
   uint32_t numBpLane, numBpWave;  // pair producers on the lane / wave paths
+  uint32_t bpGroup;               // lane producers walk the hash cells: eight lanes each
   // 1 in the iterate-to-residual chunks: sweep kernels first read the
   // frame's end flag (CTR_CONV_DONE) and exit once it is set; 0 elsewhere,
   // where the flag is never set, so the kernels skip that dependent load

@@ -15,6 +15,7 @@ void launch_exclusive_scan_dev(hipStream_t st, const uint32_t* in, uint32_t* out
                                uint32_t cap, uint32_t* scratch);
 
 // collide.hip
+constexpr uint32_t kStash = 8;  // partners kept per pair producer
 void launch_broadphase(hipStream_t st, const DeviceState& S, const StepParams& P);
 void launch_narrowphase(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t gridCap);
 void launch_map_rebuild(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t gridCap);

@@ -52,6 +52,7 @@ struct avbd_solver {
   uint32_t nb = 0, nc = 0, nj = 0, ns = 0, nt = 0;
   uint32_t nHashed = 0, nGlobal = 0, nHashedRigid = 0, nExcl = 0;
   uint32_t numBpLane = 0, numBpWave = 0;  // pair producers on the lane / wave paths
+  bool bpGroup = false;                   // lane producers walk the hash cells (no search grid)
   uint32_t maxPairs = 0, mapCapacity = 0, gridHashSize = 0;
   float cellSize = 0.1f;
   float fineCellSize = 0.0f;  // candidate search grid (0 = off)
@@ -234,6 +235,7 @@ StepParams make_params(const avbd_solver* s) {
   P.numHashedRigid = s->nHashedRigid;
   P.numBpLane = s->numBpLane;
   P.numBpWave = s->numBpWave;
+  P.bpGroup = s->bpGroup ? 1u : 0u;
   P.frictionCombineMode = s->settings.friction_combine_mode;
   P.numExclusions = s->nExcl;
   P.iterations = (uint32_t)std::max(0, s->settings.iterations);
@@ -1733,23 +1735,24 @@ avbd_status build_static_and_upload(avbd_solver* s, const avbd_scene_desc* d) {
     ALLOC(S.largeCells, hashed.size() / 33 + 1)
   }
   uint32_t producers = s->nHashed + s->nGlobal;
-  // pair producers: one lane each where that walk is short or hides its
-  // latency -- every hashed producer without the search grid (small
-  // buckets) or when there are many (kLaneMany), else the soft-group
-  // particles of scenes with no hashed non-particle collider (globals
-  // only); one wave each for the rest and the globals
+  // pair producers: one lane each (eight where they walk hash cells) for
+  // every hashed producer without the search grid (small buckets) or when
+  // there are many (kLaneMany), else the soft-group particles of scenes with
+  // no hashed non-particle collider (globals only); one wave each for the
+  // rest and the globals
   constexpr size_t kLaneMany = 32768;
   std::vector<uint32_t> bpLane, bpWave;
   for (size_t k = 0; k < hashed.size(); k++) {
-    const bool lane = s->fineCellSize <= 0.0f || hashed.size() >= kLaneMany ||
-                      (clothGroup[co[hashed[k]]] != 0u && s->nHashedRigid == 0);
+    const bool globalsOnly = clothGroup[co[hashed[k]]] != 0u && s->nHashedRigid == 0;
+    const bool lane = s->fineCellSize <= 0.0f || hashed.size() >= kLaneMany || globalsOnly;
     (lane ? bpLane : bpWave).push_back((uint32_t)k);
+    s->bpGroup |= s->fineCellSize <= 0.0f && !globalsOnly;
   }
   for (uint32_t g = 0; g < s->nGlobal; g++) bpWave.push_back(s->nHashed + g);
   s->numBpLane = (uint32_t)bpLane.size();
   s->numBpWave = (uint32_t)bpWave.size();
   ALLOC(S.bpLane, std::max<size_t>(1, bpLane.size())) ALLOC(S.bpWave, std::max<uint32_t>(1, producers))
-  ALLOC(S.bpWaveCount, 1)
+  ALLOC(S.pairStash, std::max<size_t>(1, (size_t)kStash * producers)) ALLOC(S.bpBig, std::max<uint32_t>(1, producers))
   ALLOC(S.pairCount, std::max<uint32_t>(1, producers)) ALLOC(S.pairStart, std::max<uint32_t>(1, producers))
   ALLOC(S.pairs, s->maxPairs) ALLOC(S.exclusions, std::max<size_t>(1, exr.size()))
   ALLOC(S.manifolds, s->maxPairs) ALLOC(S.prevManifolds, s->maxPairs)

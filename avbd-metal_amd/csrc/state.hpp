@@ -49,10 +49,11 @@ struct DeviceState {
   U2* fineSlot;
   uint32_t* largeCells;       // buckets of more than 32 colliders (sorted by a workgroup each)
   uint32_t *pairCount, *pairStart;
-  // pair producers by path: bpLane one lane each; bpWave one wave each,
-  // its static part (built at create) followed by the lane producers
-  // deferred this frame, bpWaveCount[0] entries in all
-  uint32_t *bpLane, *bpWave, *bpWaveCount;
+  // pair producers by path: bpLane one lane (or eight) each; bpWave one wave
+  // each, its static part (built at create) followed by the lane producers
+  // deferred this frame; pairStash the first partners of every producer,
+  // slot-major; bpBig the producers with more
+  uint32_t *bpLane, *bpWave, *pairStash, *bpBig;
   U2* pairs;
   U2* exclusions;
   // contacts
