@@ -31,6 +31,9 @@ constexpr uint32_t kColorPasses = 20;      // Jacobi passes of the dynamic color
 constexpr uint32_t kIslandMax = 512;
 constexpr uint32_t kIslandSolveMax = 128;
 constexpr uint32_t kIslandFill = 64;       // bodies that small islands are gathered to in one workgroup
+constexpr uint32_t kTileThreads = 512;     // largest tile workgroup
+constexpr uint32_t kTileLocal = 1024;      // own and halo bodies of a tile
+constexpr uint32_t kTileOwn = 128;         // own bodies of a tile
 constexpr uint32_t kIslandContacts = 2048; // contacts one island workgroup lists in LDS
 constexpr uint32_t kIslandThreads = 512;   // largest island workgroup
 constexpr uint32_t kWorld = 0xFFFFFFFFu;
@@ -104,6 +107,7 @@ enum Counter : uint32_t {
   CTR_OGC_REFRESH,         // refreshes fired this frame
   CTR_BP_DEFER,            // pair producers the lane / group paths passed to the wave path
   CTR_BP_BIG,              // producers with more partners than the stash holds
+  CTR_DYN_CONTACT,         // some contact this frame joins two dynamic bodies (or is an element contact)
   CTR_TOTAL = 16 + 2 * kMaxColors + 24
 };
 

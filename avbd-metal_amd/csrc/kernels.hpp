@@ -93,6 +93,11 @@ void launch_residual_check(hipStream_t st, const DeviceState& S, uint32_t blocks
                            uint32_t n, ConvHost* host);
 void launch_diag_error(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t* out, uint32_t gridCap);
 // persistent cooperative sweep: all iterations x colors x dual in one launch
+// tile.hip: P.iterations sweeps of the tiles
+hipError_t launch_tile_solve(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t tiles,
+                             uint32_t colors, uint32_t threads, bool cooperative);
+// two workgroups of `threads` fit a CU
+bool tile_fits(uint32_t threads);
 // island.hip: coloring (S.colorFlags zero on entry) and P.iterations sweeps, one workgroup of `threads` per island
 void launch_island_coloring(hipStream_t st, const DeviceState& S, uint32_t numIslands, uint32_t threads);
 void launch_island_solve(hipStream_t st, const DeviceState& S, const StepParams& P, uint32_t numIslands, int lanes,

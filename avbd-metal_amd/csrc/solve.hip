@@ -6,32 +6,6 @@
 
 namespace avbd {
 
-// Grid barrier for cooperative launches (every workgroup co-resident).
-// Every wait is bounded: past the spin bound a block records CTR_GBAR_FAIL
-// and proceeds, and once any block has given up later barriers do not wait,
-// so the grid always drains.
-// One release (cache write-back) before arriving, relaxed polling of the
-// arrival counter, and one acquire (cache invalidate) once it is reached:
-// an acquire load inside the spin would invalidate the L2 on every poll.
-__device__ __forceinline__ void grid_barrier(uint32_t* bar, uint32_t* fail, uint32_t target) {
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t spins = 0;
-    while (__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target &&
-           __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
-      __builtin_amdgcn_s_sleep(1);
-      if (++spins > (1u << 20)) {
-        atomicAdd(fail, 1u);
-        break;
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  }
-  __syncthreads();
-}
-
 // ---------------------------------------------------------------------------
 // per-frame contact adjacency: count / scan / scatter / sort of active
 // manifolds into a second CSR beside the static topology CSR
@@ -45,6 +19,7 @@ __global__ void __launch_bounds__(256) k_cadj_count(DeviceState S, StepParams P)
       // element contact: one entry per dynamic participant
       U4 ids = S.soft[m - n].ids;
       uint32_t v[4] = {ids.x, ids.y, ids.z, ids.w};
+      S.counters[CTR_DYN_CONTACT] = 1u;
       for (int k = 0; k < 4; k++)
         if (body_dynamic(S, v[k])) atomicAdd(&S.dAdjCount[v[k]], 1u);
       continue;
@@ -52,8 +27,10 @@ __global__ void __launch_bounds__(256) k_cadj_count(DeviceState S, StepParams P)
     U4 h = S.manifolds[m].header;
     if (h.z == 0) continue;
     active++;
-    if (body_dynamic(S, h.x)) atomicAdd(&S.dAdjCount[h.x], 1u);
-    if (body_dynamic(S, h.y)) atomicAdd(&S.dAdjCount[h.y], 1u);
+    const bool dx = body_dynamic(S, h.x), dy = body_dynamic(S, h.y);
+    if (dx) atomicAdd(&S.dAdjCount[h.x], 1u);
+    if (dy) atomicAdd(&S.dAdjCount[h.y], 1u);
+    if (dx && dy) S.counters[CTR_DYN_CONTACT] = 1u;
   }
   if (active) atomicAdd(&S.counters[CTR_ACTIVE_MANIFOLDS], active);
 }
@@ -364,16 +341,6 @@ void launch_color_buckets(hipStream_t st, const DeviceState& S, const StepParams
   hipLaunchKernelGGL(k_color_starts, dim3(1), dim3(64), 0, st, S, P);
 }
 
-// XCD-aware block order: the hardware deals consecutive workgroups to the
-// 8 XCDs round-robin; remapping gives each XCD one contiguous slice of the
-// color list so neighbour gathers of adjacent bodies share that XCD's L2.
-__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t n) {
-  const uint32_t X = 8;
-  uint32_t per = (n + X - 1) / X;
-  uint32_t r = (b % X) * per + b / X;
-  return r;
-}
-
 template <int L, int MODE>
 __global__ void __launch_bounds__(256) k_primal(DeviceState S, StepParams P, uint32_t color, uint32_t count,
                                                 uint32_t base) {
@@ -674,41 +641,7 @@ template <int L, int MODE>
 __global__ void __launch_bounds__(256) k_persistent(DeviceState S, StepParams P, uint32_t numColors,
                                                     uint32_t barrierBase) {
   if (P.convCheck && S.counters[CTR_CONV_DONE] != 0u) return;  // uniform across the grid: no barrier is entered
-  const uint32_t groupsPerBlock = 256 / L;
-  const uint32_t lane = threadIdx.x & (L - 1);
-  const uint32_t gslot = xcd_block(blockIdx.x, gridDim.x) * groupsPerBlock + threadIdx.x / L;
-  const uint32_t ngroups = gridDim.x * groupsPerBlock;
-  uint32_t* bar = &S.counters[CTR_GBAR];
-  uint32_t* fail = &S.counters[CTR_GBAR_FAIL];
-  uint32_t epoch = barrierBase;
-  const uint32_t colorsUsed = numColors ? numColors : S.colorStart[kMaxColors + 1];
-  const uint32_t numPairs = S.counters[CTR_PAIRS];
-  const uint32_t dualTotal = P.numJoints + P.numSprings + numPairs * kMaxContacts + S.counters[CTR_SOFT];
-  const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x, nthreads = gridDim.x * blockDim.x;
-  for (uint32_t it = 0; it < P.iterations; it++) {
-    for (uint32_t c = 0; c < colorsUsed; c++) {
-      uint32_t s = S.colorStart[c], e = S.colorStart[c + 1];
-      uint32_t count = e - s;
-      uint32_t rounds = (count + ngroups - 1) / ngroups;
-      for (uint32_t r = 0; r < rounds; r++) {
-        uint32_t slot = r * ngroups + gslot;
-        bool active = slot < count;
-        primal_group<L, MODE>(S, P, active,
-                              numColors ? (active ? S.colorWork[s + slot] : U4{0u, 0u, 0u, 0u})
-                                        : body_work(S, active, active ? S.colorList[s + slot] : 0u),
-                              lane, c);
-      }
-      epoch += gridDim.x;
-      grid_barrier(bar, fail, epoch);
-    }
-    for (uint32_t g = tid; g < dualTotal; g += nthreads) dual_item(S, P, g, numPairs);
-    for (uint32_t b = tid; b < P.numBodies; b += nthreads) {
-      S.posLinSnap[b] = S.posLin[b];
-      S.posAngSnap[b] = S.posAng[b];
-    }
-    epoch += gridDim.x;
-    grid_barrier(bar, fail, epoch);
-  }
+  grid_sweeps<L, MODE>(S, P, numColors, barrierBase);
 }
 
 template <int MODE>

@@ -9,6 +9,7 @@
 #include <string.h>
 #include <stdio.h>
 #include <algorithm>
+#include <atomic>
 #include <array>
 #include <functional>
 #include <map>
@@ -16,6 +17,7 @@
 #include <mutex>
 #include <set>
 #include <string>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -94,6 +96,10 @@ struct avbd_solver {
   float elemCellSize = 0.0f, elemMargin = 0.0f, datQueryRadius = 0.0f, surfaceContactCellSize = 0.0f;
   float datQueryRadiusDerived = 0.0f;  // rq derived at create (a test hook may replace datQueryRadius)
   int lanes = 8, sweepMode = 1;
+  uint32_t numTiles = 0;         // tiles of a tetrahedral scene (0: no tile path)
+  uint32_t tileThreads = 0;
+  int tileHold = 0;              // frames the tile path still stays off after contacts between dynamic bodies
+  bool dynContact[2] = {false, false};  // per frame slot: the retired frame had contacts between dynamic bodies
   uint32_t numIslands = 0;       // island workgroups that color the dynamic palette (0: grid-wide coloring)
   bool islandSolve = false;      // they also run the sweeps
   uint32_t islandThreads = 64;   // their workgroup size
@@ -117,10 +123,17 @@ struct avbd_solver {
   bool slotBusy[2] = {false, false};
   int64_t frameIndex = 0;
   // graphs (even / odd frame: manifold buffers alternate)
-  hipGraphExec_t graphs[2] = {nullptr, nullptr};
-  bool graphsValid = false;
+  // one pair for ordinary launches, one with the waiting kernels launched
+  // cooperatively (scenes on the tile path only)
+  hipGraphExec_t graphs[2][2] = {};
+  bool graphsValid[2] = {false, false};
   bool graphsDisabled = false;
-  int64_t graphBaseFrame = 1;  // frame that replays graphs[0]
+  int64_t graphBaseFrame[2] = {1, 1};  // frame that replays the pair's first graph
+  // kernels that wait for their other workgroups (tiles, grid barriers)
+  bool waits = false;          // this solver's frames may hold such kernels
+  bool cooperative = true;     // how the next frame launches its tile kernel
+  std::atomic<bool> frameOpen{false};          // a frame is being submitted (or iterated to a residual)
+  std::atomic<bool> waitBusy[2] = {false, false};  // per frame slot: submitted and not retired
   // failure latch
   avbd_failure failure{};
   bool failed = false;
@@ -145,7 +158,7 @@ struct avbd_solver {
   // even and odd frame roles, for one (chunk, tolerance, cap) key
   ConvHost* convHost = nullptr;
   ConvHost* convDev = nullptr;
-  hipGraphExec_t resPre[2] = {nullptr, nullptr}, resChunk[2] = {nullptr, nullptr}, resPost[2] = {nullptr, nullptr};
+  hipGraphExec_t resPre[2] = {nullptr, nullptr}, resChunk[2][2] = {}, resPost[2] = {nullptr, nullptr};
   bool resValid = false;
   int32_t resCheck = 0, resMax = 0;
   float resTol = 0.0f;
@@ -359,6 +372,9 @@ hipError_t enqueue_iterations(avbd_solver* s, const DeviceState& S, const StepPa
   StepParams P = P0;
   P.iterations = iterations;
   if (iterations == 0) return hipSuccess;
+  if (s->numTiles && s->tileHold == 0) {
+    return launch_tile_solve(st, S, P, s->numTiles, s->staticUsedColors, s->tileThreads, s->cooperative);
+  }
   if (s->islandSolve) {
     launch_island_solve(st, S, P, s->numIslands, s->lanes, s->islandThreads);
     return hipSuccess;
@@ -415,14 +431,13 @@ hipError_t enqueue_frame(avbd_solver* s, const DeviceState& S, const StageFn& ma
 
 void invalidate_graphs(avbd_solver* s) {
   for (int i = 0; i < 2; i++) {
-    if (s->graphs[i]) hipGraphExecDestroy(s->graphs[i]);
-    s->graphs[i] = nullptr;
-    for (hipGraphExec_t* g : {&s->resPre[i], &s->resChunk[i], &s->resPost[i]}) {
+    for (hipGraphExec_t* g : {&s->graphs[0][i], &s->graphs[1][i], &s->resPre[i], &s->resChunk[0][i], &s->resChunk[1][i],
+                              &s->resPost[i]}) {
       if (*g) hipGraphExecDestroy(*g);
       *g = nullptr;
     }
   }
-  s->graphsValid = false;
+  s->graphsValid[0] = s->graphsValid[1] = false;
   s->resValid = false;
 }
 
@@ -444,7 +459,7 @@ hipError_t capture_graph(avbd_solver* s, const std::function<hipError_t()>& body
 }
 
 hipError_t build_graphs(avbd_solver* s) {
-  invalidate_graphs(s);
+  const int v = s->cooperative ? 1 : 0;
   DeviceState S = s->S;
   for (int p = 0; p < 2; p++) {
     hipGraph_t g = nullptr;
@@ -454,20 +469,103 @@ hipError_t build_graphs(avbd_solver* s) {
     e = hipStreamEndCapture(s->stream, &g);
     if (eq != hipSuccess) { if (g) hipGraphDestroy(g); return eq; }
     if (e != hipSuccess) return e;
-    e = hipGraphInstantiate(&s->graphs[p], g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&s->graphs[v][p], g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
     if (e != hipSuccess) return e;
     std::swap(S.manifolds, S.prevManifolds);
     std::swap(S.soft, S.prevSoft);
   }
-  s->graphsValid = true;
-  s->graphBaseFrame = s->frameIndex + 1;
+  s->graphsValid[v] = true;
+  s->graphBaseFrame[v] = s->frameIndex + 1;
   return hipSuccess;
 }
+
+avbd_status sync_all(avbd_solver* s);
+
+// Kernels that wait for their other workgroups need all of them resident.
+// Cooperative launches are kept apart by the runtime; an ordinary launch of
+// the tile kernel is only safe beside kernels that end by themselves (or one
+// tile kernel more: two of its workgroups fit a CU).  So each solver whose
+// frames hold such kernels announces them here, per process, and a tile frame
+// is launched the ordinary way only while no other solver's is in flight;
+// other waiting kernels hold back until an ordinary tile frame has ended.
+struct WaitingSolvers {
+  std::mutex m;
+  std::vector<avbd_solver*> list;
+};
+WaitingSolvers& waiting_solvers() {
+  static WaitingSolvers* w = new WaitingSolvers();  // outlives every handle
+  return *w;
+}
+void leave_waiting(avbd_solver* s) {
+  WaitingSolvers& w = waiting_solvers();
+  std::lock_guard<std::mutex> lock(w.m);
+  w.list.erase(std::remove(w.list.begin(), w.list.end(), s), w.list.end());
+}
+bool frame_in_flight(avbd_solver* o) {
+  if (o->frameOpen) return true;
+  for (int k = 0; k < 2; k++)
+    if (o->waitBusy[k]) {
+      const hipError_t e = hipEventQuery(o->frameDone[k]);
+      if (e == hipErrorNotReady) {
+        (void)hipGetLastError();
+        return true;
+      }
+    }
+  return false;
+}
+// held from the choice of the launch to the record of the frame's event
+struct FrameTurn {
+  avbd_solver* s;
+  explicit FrameTurn(avbd_solver* solver) : s(solver) {
+    if (!s->waits) return;
+    WaitingSolvers& w = waiting_solvers();
+    for (;;) {
+      bool others = false, tile = false;
+      {
+        std::lock_guard<std::mutex> lock(w.m);
+        for (avbd_solver* o : w.list)
+          if (o != s && o->device == s->device && frame_in_flight(o)) {
+            others = true;
+            tile |= o->numTiles && !o->cooperative;
+          }
+        if (s->numTiles || !tile) {
+          s->cooperative = others || !s->numTiles;
+          s->frameOpen = true;
+          return;
+        }
+      }
+      std::this_thread::yield();
+    }
+  }
+  ~FrameTurn() { s->frameOpen = false; }
+  FrameTurn(const FrameTurn&) = delete;
+  FrameTurn& operator=(const FrameTurn&) = delete;
+};
+
+// Which path the next frame takes: after a frame with contacts between
+// dynamic bodies, which the tile kernel leaves to the grid-wide sweep, the
+// next kTileHold frames run one launch per color.  Frame f decides for frame
+// f + 2, whose submission has always seen f retired, so the choice does not
+// depend on when the caller synchronizes.
+constexpr int kTileHold = 120;
+void choose_tile_path(avbd_solver* s, int slot) {
+  if (!s->numTiles) return;
+  const bool was = s->tileHold == 0;
+  if (s->dynContact[slot]) s->tileHold = kTileHold;
+  else if (s->tileHold > 0) s->tileHold--;
+  if (was == (s->tileHold == 0)) return;
+  sync_all(s);  // the graphs of the other path may be running
+  invalidate_graphs(s);
+}
+// Bodies a tile is filled to before a further CU takes some: 8, 16 and 36
+// measured 0.59, 0.61 and 0.63 ms a frame on 125 vertices (9261: no difference).
+constexpr uint32_t kTileFill = 8;
 
 avbd_status retire_slot(avbd_solver* s, int slot) {
   if (!s->slotBusy[slot]) return AVBD_OK;
   s->slotBusy[slot] = false;
+  s->waitBusy[slot] = false;
   int64_t frame = s->slotFrame[slot];
   hipError_t e = hipEventSynchronize(s->frameDone[slot]);
   if (e != hipSuccess) {
@@ -504,6 +602,7 @@ avbd_status retire_slot(avbd_solver* s, int slot) {
   s->lastOgcTrunc = c[CTR_OGC_TRUNC];
   s->lastOgcRefresh = c[CTR_OGC_REFRESH];
   s->stats.color_conflicts = (int32_t)c[CTR_COLOR_CONFLICTS];
+  s->dynContact[slot] = c[CTR_DYN_CONTACT] != 0u;
   if (s->dynamicColoring) {
     int maxUsed = -1;
     for (int k = 0; k < kMaxColors; k++) {
@@ -1135,10 +1234,18 @@ extern "C" avbd_status avbd_create(const avbd_scene_desc* d, const avbd_options*
     *out = nullptr;
     return st;
   }
+  s->waits = true;  // the trials may launch grid-wide sweeps
+  {
+    std::lock_guard<std::mutex> lock(waiting_solvers().m);
+    waiting_solvers().list.push_back(s);
+  }
   autotune(s);
   create_phase(s, "autotune");
   s->stats.lanes_per_body = s->lanes;
-  s->stats.sweep_mode = s->sweepMode;
+  s->waits = s->numTiles || (s->dynamicColoring && !s->numIslands) || (s->sweepMode == 2 && !s->islandSolve);
+  s->cooperative = !s->numTiles;
+  if (!s->waits) leave_waiting(s);
+  s->stats.sweep_mode = s->numTiles ? 2 : s->sweepMode;
   s->stats.uses_dynamic_coloring = s->dynamicColoring ? 1 : 0;
   return AVBD_OK;
 }
@@ -1153,6 +1260,7 @@ namespace {
 void release_solver(avbd_solver* s) {
   if (!s) return;
   if (s->stream) hipStreamSynchronize(s->stream);
+  leave_waiting(s);
   invalidate_graphs(s);
   for (void* p : s->allocs) hipFree(p);
   for (int i = 0; i < 2; i++)
@@ -1923,6 +2031,115 @@ avbd_status build_static_and_upload(avbd_solver* s, const avbd_scene_desc* d) {
   return islands;
 }
 
+// Tiles of a scene whose dynamic bodies are all particles of tets only:
+// bodies in Morton order of their positions, an equal share each, one
+// workgroup per tile and at most one per CU (all of them resident).  Scenes
+// past kTileOwn bodies a CU stay with one launch per color, which by then is
+// bound by memory and not by the launches.
+avbd_status build_tiles(avbd_solver* s, const std::vector<uint32_t>& colors, const std::vector<uint32_t>& sStart) {
+  DeviceState& S = s->S;
+  if (s->dynamicColoring || s->allMode != kModeTet || s->datOn || s->isoOn || s->opts.sweep_mode != 0 ||
+      (s->opts.lanes_per_body != 0 && s->opts.lanes_per_body != 32))
+    return AVBD_OK;
+  std::vector<uint32_t> order;
+  for (uint32_t b = 0; b < s->nb; b++)
+    if (s->mass[b] > 0.0f) order.push_back(b);
+  const uint32_t nd = (uint32_t)order.size(), C = s->staticUsedColors;
+  if (nd == 0 || nd > kTileOwn * s->cus) return AVBD_OK;
+  std::vector<F4> pos(s->nb);
+  if (hipMemcpy(pos.data(), S.posLin, 16 * (size_t)s->nb, hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
+  V3 lo = xyz(pos[order[0]]), hi = lo;
+  for (uint32_t b : order) {
+    lo = v3(fminf(lo.x, pos[b].x), fminf(lo.y, pos[b].y), fminf(lo.z, pos[b].z));
+    hi = v3(fmaxf(hi.x, pos[b].x), fmaxf(hi.y, pos[b].y), fmaxf(hi.z, pos[b].z));
+  }
+  const float side = fmaxf(fmaxf(hi.x - lo.x, hi.y - lo.y), fmaxf(hi.z - lo.z, 1e-20f));
+  auto spread = [](uint32_t v) {  // 10 bits, two zeros after each
+    v = (v | v << 16) & 0x030000FFu;
+    v = (v | v << 8) & 0x0300F00Fu;
+    v = (v | v << 4) & 0x030C30C3u;
+    return (v | v << 2) & 0x09249249u;
+  };
+  std::vector<uint32_t> code(s->nb, 0u);
+  for (uint32_t b : order) {
+    const float f[3] = {(pos[b].x - lo.x) / side, (pos[b].y - lo.y) / side, (pos[b].z - lo.z) / side};
+    for (int k = 0; k < 3; k++) code[b] |= spread((uint32_t)fminf(fmaxf(f[k], 0.0f) * 1023.0f, 1023.0f)) << k;
+  }
+  std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return code[a] < code[b]; });
+  const uint32_t T = std::min<uint32_t>(s->cus, (nd + kTileFill - 1) / kTileFill);
+  std::vector<uint32_t> own((size_t)T * (C + 1)), halo((size_t)T * (C + 2)), torder(T), mark(s->nb, 0xFFFFFFFFu), local(s->nb);
+  std::vector<U4> work;
+  std::vector<U2> hb;
+  std::vector<TileSlotIdx> idx(std::max<size_t>(1, s->sAdjListHost.size()), TileSlotIdx{{0, 0, 0, 0}});
+  uint32_t widest = 1;
+  for (uint32_t t = 0; t < T; t++) {
+    const uint32_t a = (uint32_t)((uint64_t)nd * t / T), e = (uint32_t)((uint64_t)nd * (t + 1) / T);
+    std::vector<std::vector<uint32_t>> mine(C), other(C + 1);
+    for (uint32_t i = a; i < e; i++) mine[colors[order[i]]].push_back(order[i]);
+    uint32_t n = 0;
+    for (uint32_t c = 0; c < C; c++) {
+      own[(size_t)t * (C + 1) + c] = (uint32_t)work.size();
+      widest = std::max(widest, (uint32_t)mine[c].size());
+      for (uint32_t b : mine[c]) {
+        mark[b] = t;
+        local[b] = n;
+        work.push_back(U4{b, sStart[b], s->sAdjCount[b], n++});
+      }
+    }
+    own[(size_t)t * (C + 1) + C] = (uint32_t)work.size();
+    auto partners = [&](uint32_t b, uint32_t k, uint32_t* o) {  // as the slots hold them: the other ids in tet order
+      const U4 id = s->tetIdsHost[s->sAdjListHost[sStart[b] + k] & kAdjIndexMask];
+      const uint32_t v[4] = {id.x, id.y, id.z, id.w};
+      int m = 0;
+      o[0] = o[1] = o[2] = 0u;
+      for (int q = 0; q < 4; q++)
+        if (v[q] != b && m < 3) o[m++] = v[q];
+    };
+    uint32_t o[3];
+    for (uint32_t i = a; i < e; i++)
+      for (uint32_t k = 0; k < s->sAdjCount[order[i]]; k++) {
+        partners(order[i], k, o);
+        for (uint32_t v : o)
+          if (mark[v] != t) {
+            mark[v] = t;
+            other[s->mass[v] > 0.0f ? colors[v] : C].push_back(v);
+          }
+      }
+    for (uint32_t c = 0; c <= C; c++) {
+      halo[(size_t)t * (C + 2) + c] = (uint32_t)hb.size();
+      for (uint32_t v : other[c]) {
+        local[v] = n;
+        hb.push_back(U2{v, n++});
+      }
+    }
+    halo[(size_t)t * (C + 2) + C + 1] = (uint32_t)hb.size();
+    if (n > kTileLocal) return AVBD_OK;  // no spatial locality in the mesh
+    for (uint32_t i = a; i < e; i++)
+      for (uint32_t k = 0; k < s->sAdjCount[order[i]]; k++) {
+        partners(order[i], k, o);
+        TileSlotIdx& q = idx[sStart[order[i]] + k];
+        for (int m = 0; m < 3; m++) q.o[m] = (uint16_t)local[o[m]];
+      }
+  }
+  // consecutive workgroups go to the 8 XCDs in turn: neighbouring tiles to one XCD
+  uint32_t next = 0;
+  for (uint32_t x = 0; x < 8; x++)
+    for (uint32_t b = x; b < T; b += 8) torder[b] = next++;
+  const uint32_t threads = std::min<uint32_t>(kTileThreads, std::max<uint32_t>(64u, widest * 32u));
+  if (!tile_fits(threads)) return AVBD_OK;
+  if (hb.empty()) hb.push_back(U2{0u, 0u});
+  if (dev_alloc(s, &S.tileOrder, T) || dev_alloc(s, &S.tileOwn, own.size()) || dev_alloc(s, &S.tileHalo, halo.size()) ||
+      dev_alloc(s, &S.tileWork, work.size()) || dev_alloc(s, &S.tileHaloBody, hb.size()) ||
+      dev_alloc(s, &S.tileIdx, idx.size()) || dev_alloc(s, &S.tileX, 6 * (size_t)s->nb) || dev_alloc(s, &S.tileEpoch, 2))
+    return AVBD_ERR_ALLOC;
+  if (upload(S.tileOrder, torder) || upload(S.tileOwn, own) || upload(S.tileHalo, halo) || upload(S.tileWork, work) ||
+      upload(S.tileHaloBody, hb) || upload(S.tileIdx, idx))
+    return AVBD_ERR_HIP;
+  s->numTiles = T;
+  s->tileThreads = (threads + 63u) / 64u * 64u;
+  return AVBD_OK;
+}
+
 // Static palette: Jacobi fixed point of the greedy rule on the GPU, then
 // stable index-ordered buckets (GPUSolver.swift:1956-2050).
 avbd_status static_coloring(avbd_solver* s) {
@@ -2033,7 +2250,7 @@ avbd_status static_coloring(avbd_solver* s) {
   }
   s->stats.max_color_used = (int32_t)s->staticUsedColors - 1;
   s->stats.num_colors = (int32_t)s->staticUsedColors;
-  return AVBD_OK;
+  return build_tiles(s, colors, sStart);
 }
 
 // Workgroup size of the island kernels: enough lane groups for the larger
@@ -2061,16 +2278,6 @@ void autotune(avbd_solver* s) {
   if (s->dynamicColoring && wantMode == 0) modeCands = {2, 1};
   // cloth: the Planar-DAT passes run between the colors' launches
   if (s->datOn || s->isoOn) modeCands = {1};
-  s->islandThreads = island_threads(s);
-  if (s->islandSolve) {
-    s->lanes = laneCands.size() == 1 ? laneCands[0] : kIslandLanes;
-    s->sweepMode = 2;
-    return;
-  }
-  if (laneCands.size() == 1 && modeCands.size() == 1) {
-    s->lanes = laneCands[0];
-    s->sweepMode = modeCands[0];
-  }
   // persistent grid size per lane count
   auto pblocks = [&](int L) {
     int maxB = persistent_max_blocks(L, s->allMode);
@@ -2083,11 +2290,27 @@ void autotune(avbd_solver* s) {
     if (maxB <= 0) return 0;
     return (int)std::min<uint32_t>(want, (uint32_t)maxB);
   };
+  s->islandThreads = island_threads(s);
+  if (s->numTiles) {
+    s->lanes = 32;
+    s->sweepMode = 1;  // while the tile path is off
+    return;
+  }
+  if (s->islandSolve) {
+    s->lanes = laneCands.size() == 1 ? laneCands[0] : kIslandLanes;
+    s->sweepMode = 2;
+    return;
+  }
+  if (laneCands.size() == 1 && modeCands.size() == 1) {
+    s->lanes = laneCands[0];
+    s->sweepMode = modeCands[0];
+  }
   if (laneCands.size() == 1 && modeCands.size() == 1) {
     s->persistentBlocks = pblocks(s->lanes);
     if (s->sweepMode == 2 && s->persistentBlocks <= 0) s->sweepMode = 1;
     return;
   }
+  FrameTurn turn(s);
   // backup
   std::vector<std::pair<void*, size_t>> bufs = {
       {S.posLin, nb * 16}, {S.posLo, nb * 16}, {S.posAng, nb * 16}, {S.initLin, nb * 16}, {S.initAng, nb * 16},
@@ -2200,8 +2423,10 @@ extern "C" avbd_status avbd_submit_step(avbd_solver* s) {
       return latch(s, AVBD_FAIL_STAGE_DENIED, frame, 0, 0, 0, m);
     }
   }
+  choose_tile_path(s, slot);
   bool useGraph = s->opts.use_graph && !s->graphsDisabled && !s->profiling;
-  if (useGraph && !s->graphsValid) {
+  FrameTurn turn(s);
+  if (useGraph && !s->graphsValid[s->cooperative]) {
     hipError_t e = build_graphs(s);
     if (e != hipSuccess) {
       hipGetLastError();
@@ -2211,8 +2436,9 @@ extern "C" avbd_status avbd_submit_step(avbd_solver* s) {
     }
   }
   if (useGraph) {
-    // graphs[0] was captured with the buffer roles of frame graphBaseFrame
-    HIP_OR_LATCH(s, hipGraphLaunch(s->graphs[(frame - s->graphBaseFrame) & 1], s->stream), frame);
+    // the pair's first graph was captured with the buffer roles of frame graphBaseFrame
+    const int v = s->cooperative ? 1 : 0;
+    HIP_OR_LATCH(s, hipGraphLaunch(s->graphs[v][(frame - s->graphBaseFrame[v]) & 1], s->stream), frame);
   } else if (s->profiling) {
     // eager, with per-stage events
     hipStream_t st = s->stream;
@@ -2243,6 +2469,7 @@ extern "C" avbd_status avbd_submit_step(avbd_solver* s) {
                frame);
   HIP_OR_LATCH(s, hipEventRecord(s->frameDone[slot], s->stream), frame);
   s->slotBusy[slot] = true;
+  s->waitBusy[slot] = s->waits;
   s->slotFrame[slot] = frame;
   s->frameIndex = frame;
   return AVBD_OK;
@@ -2279,7 +2506,7 @@ hipError_t enqueue_chunk(avbd_solver* s, const DeviceState& S, const StepParams&
 
 hipError_t build_residual_graphs(avbd_solver* s, float tol, int32_t maxIt, int32_t check) {
   for (int i = 0; i < 2; i++)
-    for (hipGraphExec_t* g : {&s->resPre[i], &s->resChunk[i], &s->resPost[i]}) {
+    for (hipGraphExec_t* g : {&s->resPre[i], &s->resChunk[0][i], &s->resChunk[1][i], &s->resPost[i]}) {
       if (*g) hipGraphExecDestroy(*g);
       *g = nullptr;
     }
@@ -2290,9 +2517,14 @@ hipError_t build_residual_graphs(avbd_solver* s, float tol, int32_t maxIt, int32
   for (int p = 0; p < 2; p++) {
     hipError_t e = capture_graph(s, [&]() { enqueue_pre_solve(s, S, P, none); return hipGetLastError(); },
                                  &s->resPre[p]);
-    if (e == hipSuccess)
+    const bool now = s->cooperative;
+    for (int v = 0; v < 2 && e == hipSuccess; v++) {
+      if (v != (now ? 1 : 0) && !s->numTiles) continue;
+      s->cooperative = v == 1;
       e = capture_graph(s, [&]() { return enqueue_chunk(s, S, P, (uint32_t)check, tol, (uint32_t)maxIt); },
-                        &s->resChunk[p]);
+                        &s->resChunk[v][p]);
+    }
+    s->cooperative = now;
     if (e == hipSuccess)
       e = capture_graph(s, [&]() { enqueue_post_solve(s, S, P, none); return hipGetLastError(); }, &s->resPost[p]);
     if (e != hipSuccess) return e;
@@ -2317,7 +2549,9 @@ extern "C" avbd_status avbd_step_to_residual(avbd_solver* s, float tol, int32_t 
   const int64_t frame = s->frameIndex + 1;
   const int slot = (int)(frame & 1);
   hipStream_t st = s->stream;
+  choose_tile_path(s, slot);
   bool useGraph = s->opts.use_graph && !s->graphsDisabled && !s->profiling;
+  FrameTurn turn(s);
   if (useGraph && !(s->resValid && s->resCheck == check_every && s->resMax == max_iterations && s->resTol == tol)) {
     if (build_residual_graphs(s, tol, max_iterations, check_every) != hipSuccess) {
       (void)hipGetLastError();
@@ -2341,7 +2575,7 @@ extern "C" avbd_status avbd_step_to_residual(avbd_solver* s, float tol, int32_t 
   for (;;) {
     while (launched < total && launched - seen < kChunksInFlight) {
       if (launched < full && useGraph) {
-        HIP_OR_LATCH(s, hipGraphLaunch(s->resChunk[parity], st), frame);
+        HIP_OR_LATCH(s, hipGraphLaunch(s->resChunk[s->cooperative][parity], st), frame);
       } else {
         const uint32_t n = launched < full ? (uint32_t)check_every : tail;
         HIP_OR_LATCH(s, enqueue_chunk(s, S, P, n, tol, (uint32_t)max_iterations), frame);
@@ -2378,6 +2612,7 @@ extern "C" avbd_status avbd_step_to_residual(avbd_solver* s, float tol, int32_t 
                frame);
   HIP_OR_LATCH(s, hipEventRecord(s->frameDone[slot], st), frame);
   s->slotBusy[slot] = true;
+  s->waitBusy[slot] = s->waits;
   s->slotFrame[slot] = frame;
   s->frameIndex = frame;
   avbd_status out = sync_all(s);
@@ -2770,7 +3005,7 @@ extern "C" avbd_status avbd_get_stats(avbd_solver* s, avbd_stats* out) {
   if (!s || !out) return AVBD_ERR_INVALID_ARGUMENT;
   sync_all(s);
   s->stats.lanes_per_body = s->lanes;
-  s->stats.sweep_mode = s->sweepMode;
+  s->stats.sweep_mode = s->numTiles ? 2 : s->sweepMode;
   s->stats.uses_dynamic_coloring = s->dynamicColoring ? 1 : 0;
   *out = s->stats;
   return AVBD_OK;

@@ -157,7 +157,8 @@ __device__ __forceinline__ V3 contact_force(const ManifoldRec& m, int ci, V3 dqA
 // displacement from the step start)
 // contacts first, first + stride, ... of the manifold (a lane's share when a
 // body's lanes split one manifold)
-__device__ __forceinline__ void stamp_manifold(const ManifoldRec& m, uint32_t self, bool rigidSelf, const PoseView& pv,
+template <typename Pose>
+__device__ __forceinline__ void stamp_manifold(const ManifoldRec& m, uint32_t self, bool rigidSelf, const Pose& pv,
                                                const F4* initLin, const F4* initAng, float alpha, Acc& acc,
                                                V3 loSelf, uint32_t first = 0u, uint32_t stride = 1u) {
   uint32_t a = m.header.x, b = m.header.y, n = m.header.z;

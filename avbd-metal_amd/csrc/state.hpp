@@ -9,6 +9,10 @@ struct alignas(8) U2 {
   uint32_t x, y;
 };
 
+struct TileSlotIdx {
+  uint16_t o[4];  // a tet slot's three partners as positions in the tile's LDS arrays
+};
+
 struct DeviceState {
   // bodies (one F4 per body, each field its own array)
   F4 *posLin, *posAng, *initLin, *initAng, *inertLin, *inertAng;
@@ -76,6 +80,17 @@ struct DeviceState {
   // position inside its workgroup; the joints and springs of each
   uint32_t *islandStart, *islandBody, *islandLocal;
   uint32_t *islandJointStart, *islandJoint, *islandSpringStart, *islandSpring;
+  // tiles of a tetrahedral scene (null when the tile path is off): per tile
+  // and color the own bodies (body, static CSR start, count, local index) and
+  // the halo bodies (body, local index), static neighbours last; per tet slot
+  // the partners' local indices; the exchanged positions, six (version, float)
+  // words per body; {version base, workgroups finished}
+  uint32_t *tileOrder, *tileOwn, *tileHalo;
+  U4* tileWork;
+  U2* tileHaloBody;
+  TileSlotIdx* tileIdx;
+  uint64_t* tileX;
+  uint32_t* tileEpoch;
   // start-of-iteration pose snapshot: contact partners that share the
   // body's color are read from here, so a same-color contact is a Jacobi
   // coupling with a schedule-independent result

@@ -418,4 +418,82 @@ __device__ __forceinline__ void dual_item(const DeviceState& S, const StepParams
   dual_soft(S, P, mi - numPairs * kMaxContacts);
 }
 
+// Grid barrier (every workgroup resident).
+// Every wait is bounded: past the spin bound a block records CTR_GBAR_FAIL
+// and proceeds, and once any block has given up later barriers do not wait,
+// so the grid always drains.
+// One release (cache write-back) before arriving, relaxed polling of the
+// arrival counter, and one acquire (cache invalidate) once it is reached:
+// an acquire load inside the spin would invalidate the L2 on every poll.
+__device__ __forceinline__ void grid_barrier(uint32_t* bar, uint32_t* fail, uint32_t target) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __hip_atomic_fetch_add(bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t spins = 0;
+    while (__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target &&
+           __hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
+      __builtin_amdgcn_s_sleep(1);
+      if (++spins > (1u << 20)) {
+        atomicAdd(fail, 1u);
+        break;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+}
+
+// XCD-aware block order: the hardware deals consecutive workgroups to the
+// 8 XCDs round-robin; remapping gives each XCD one contiguous slice of the
+// color list so neighbour gathers of adjacent bodies share that XCD's L2.
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t n) {
+  const uint32_t X = 8;
+  uint32_t per = (n + X - 1) / X;
+  uint32_t r = (b % X) * per + b / X;
+  return r;
+}
+
+// Every sweep of the whole grid, a grid barrier after each color and each dual
+template <int L, int MODE>
+__device__ __forceinline__ void grid_sweeps(const DeviceState& S, const StepParams& P, uint32_t numColors,
+                                            uint32_t barrierBase) {
+  const uint32_t groupsPerBlock = blockDim.x / L;
+  const uint32_t lane = threadIdx.x & (L - 1);
+  const uint32_t block = gridDim.x % 8u ? blockIdx.x : xcd_block(blockIdx.x, gridDim.x);
+  const uint32_t gslot = block * groupsPerBlock + threadIdx.x / L;
+  const uint32_t ngroups = gridDim.x * groupsPerBlock;
+  uint32_t* bar = &S.counters[CTR_GBAR];
+  uint32_t* fail = &S.counters[CTR_GBAR_FAIL];
+  uint32_t epoch = barrierBase;
+  const uint32_t colorsUsed = numColors ? numColors : S.colorStart[kMaxColors + 1];
+  const uint32_t numPairs = S.counters[CTR_PAIRS];
+  const uint32_t dualTotal = P.numJoints + P.numSprings + numPairs * kMaxContacts + S.counters[CTR_SOFT];
+  const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x, nthreads = gridDim.x * blockDim.x;
+  for (uint32_t it = 0; it < P.iterations; it++) {
+    for (uint32_t c = 0; c < colorsUsed; c++) {
+      uint32_t s = S.colorStart[c], e = S.colorStart[c + 1];
+      uint32_t count = e - s;
+      uint32_t rounds = (count + ngroups - 1) / ngroups;
+      for (uint32_t r = 0; r < rounds; r++) {
+        uint32_t slot = r * ngroups + gslot;
+        bool active = slot < count;
+        primal_group<L, MODE>(S, P, active,
+                              numColors ? (active ? S.colorWork[s + slot] : U4{0u, 0u, 0u, 0u})
+                                        : body_work(S, active, active ? S.colorList[s + slot] : 0u),
+                              lane, c);
+      }
+      epoch += gridDim.x;
+      grid_barrier(bar, fail, epoch);
+    }
+    for (uint32_t g = tid; g < dualTotal; g += nthreads) dual_item(S, P, g, numPairs);
+    for (uint32_t b = tid; b < P.numBodies; b += nthreads) {
+      S.posLinSnap[b] = S.posLin[b];
+      S.posAngSnap[b] = S.posAng[b];
+    }
+    epoch += gridDim.x;
+    grid_barrier(bar, fail, epoch);
+  }
+}
+
 }  // namespace avbd

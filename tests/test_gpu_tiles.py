@@ -1,0 +1,117 @@
+"""The tile kernel (all sweeps of a tetrahedral scene in one launch, tiles
+exchanging versioned positions) against one launch per color at the same 32
+lanes, over frames of fall, landing and rest and iterated to a residual: one
+tile, a few, an odd number and one per CU; with pinned vertices, with particles
+on two static bodies at once, and with particles of the block in contact with
+each other, where the frames run the grid-wide sweep.
+
+The two paths evaluate the same expressions in the same order, but the
+compiler fuses multiply-adds differently in each: an update may differ by one
+rounding, 2^-24 of its step, which Gauss-Seidel contracts.  The bound is eight
+units in the last place of the scene's extent on positions, and sixty times
+that (1 / dt) on velocities."""
+import numpy as np
+import pytest
+
+from avbd_amd import GPUSolver, demos
+from conftest import flush_print
+
+pytestmark = pytest.mark.gpu
+
+
+def _pinned(cells):
+    s = demos.soft_block_scene(cells=cells, bottom=0.3)
+    for b in s.bodies[1:1 + (cells + 1)]:
+        b["density"] = 0.0
+    return s
+
+
+def _pair(**kw):
+    return demos.soft_block_scene(**kw)
+
+
+def _corner(cells):
+    s = demos.soft_block_scene(cells=cells, bottom=0.02)
+    s.addBody((0.2, 4.0, 4.0), 0.0, 0.7, (0.61, 0.0, 1.0))
+    return s
+
+
+def _close(a, b):
+    pa, ra, va, wa = a.bodyStates()
+    pb, rb, vb, wb = b.bodyStates()
+    ulp = float(np.abs(pb[1:]).max()) * 2.0 ** -23
+    assert np.array_equal(ra, rb) and np.array_equal(wa, wb)
+    assert np.abs(pa - pb).max() <= 8 * ulp
+    assert np.abs(va - vb).max() <= 8 * ulp * 60
+
+
+SCENES = {
+    "block_1": lambda: _pair(cells=1, bottom=0.02), "block_3": lambda: _pair(cells=3, bottom=0.02),
+    "block_4": lambda: _pair(cells=4, bottom=0.02), "block_5": lambda: _pair(cells=5, bottom=0.02, iterations=3),
+    "block_9": lambda: _pair(cells=9, bottom=0.02), "block_20": lambda: _pair(cells=20, bottom=0.02),
+    "pinned_6": lambda: _pinned(6), "corner_4": lambda: _corner(4),
+    "self_contact_7": lambda: _pair(cells=7, bottom=0.02, radius_factor=0.7),
+    "too_large_33": lambda: _pair(cells=33, bottom=0.02, iterations=3),
+}
+
+
+@pytest.mark.parametrize("name", list(SCENES))
+def test_tiles_equal_the_color_launches(name):
+    flush_print(f"[gpu case] tiles vs per-color launches: {name}")
+    scene = SCENES[name]()
+    with GPUSolver(scene, lanesPerBody=32) as a, GPUSolver(scene, lanesPerBody=32, sweepMode=1) as b:
+        p, r, v, w = a.bodyStates()
+        v[1:, 2] -= 1.5
+        idx = np.arange(len(p), dtype=np.uint32)
+        a.setBodyStates(idx, p, r, v, w)
+        b.setBodyStates(idx, p, r, v, w)
+        for _ in range(6):
+            a.step()
+            b.step()
+        _close(a, b)
+        for tol, count in ((0.5, None), (1e-9, 45)):
+            (na, xa), (nb, xb) = a.stepToResidual(tol, 45, 10), b.stepToResidual(tol, 45, 10)
+            # a converged residual is the rounding of element forces of about 100 m g: 100 * 2^-23 = 1.2e-5
+            assert na == nb and (count is None or na == count) and abs(xa - xb) <= 0.01 * xb + 1.2e-5
+        a.step(3)
+        b.step(3)
+        _close(a, b)
+        flush_print(f"  {a.stats().num_active_manifolds} contacts")
+
+
+def test_tiles_beside_other_solvers():
+    """Tile solvers of one, 2 and 256 tiles a scene, a scene swept grid-wide and
+    one of islands stepped from threads of their own at once: each ends where it
+    ends alone."""
+    import threading
+
+    flush_print("[gpu case] tile solvers in threads")
+
+    def solvers():
+        rigid = demos.stack_scene(height=140)
+        return [GPUSolver(_pair(cells=1, bottom=0.02)), GPUSolver(_pair(cells=2, bottom=0.02)),
+                GPUSolver(_pair(cells=14, bottom=0.02)), GPUSolver(rigid), GPUSolver(rigid, sweepMode=2),
+                GPUSolver(demos.stack_scene(height=6))]
+
+    alone = []
+    for g in solvers():
+        with g:
+            g.step(24)
+            alone.append(g.bodyStates())
+    together = solvers()
+
+    def run(g):
+        for _ in range(4):
+            g.step(6)
+            g.synchronize()
+
+    threads = [threading.Thread(target=run, args=(g,)) for g in together]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g, want in zip(together, alone):
+        with g:
+            assert g.runtimeFailure is None
+            for x, y in zip(g.bodyStates(), want):
+                assert np.array_equal(x, y)
