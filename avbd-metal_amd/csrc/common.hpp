@@ -108,6 +108,7 @@ enum Counter : uint32_t {
   CTR_BP_DEFER,            // pair producers the lane / group paths passed to the wave path
   CTR_BP_BIG,              // producers with more partners than the stash holds
   CTR_DYN_CONTACT,         // some contact this frame joins two dynamic bodies (or is an element contact)
+  CTR_LONG_ADJ,            // bodies whose contact segment a wave sorts
   CTR_TOTAL = 16 + 2 * kMaxColors + 24
 };
 

@@ -32,7 +32,14 @@ __global__ void __launch_bounds__(256) k_cadj_count(DeviceState S, StepParams P)
     if (dy) atomicAdd(&S.dAdjCount[h.y], 1u);
     if (dx && dy) S.counters[CTR_DYN_CONTACT] = 1u;
   }
-  if (active) atomicAdd(&S.counters[CTR_ACTIVE_MANIFOLDS], active);
+  // one atomic per workgroup: per thread they serialised on the one counter
+  // (33 us for 162759 pairs)
+  __shared__ uint32_t sum;
+  if (threadIdx.x == 0) sum = 0u;
+  __syncthreads();
+  if (active) atomicAdd(&sum, active);
+  __syncthreads();
+  if (threadIdx.x == 0 && sum) atomicAdd(&S.counters[CTR_ACTIVE_MANIFOLDS], sum);
 }
 __global__ void __launch_bounds__(256) k_cadj_cursor(DeviceState S, StepParams P) {
   uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -73,19 +80,60 @@ __global__ void __launch_bounds__(256) k_cadj_scatter(DeviceState S, StepParams 
   }
 }
 // Sorting each (short) segment makes the accumulation order a function of
-// the manifold indices only, which are themselves deterministic.
-__global__ void __launch_bounds__(256) k_cadj_sort(DeviceState S, StepParams P) {
-  uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= P.numBodies) return;
-  uint32_t s = S.dAdjStart[gid], n = S.dAdjCount[gid];
+// the manifold indices only, which are themselves deterministic.  One lane
+// sorts up to kCadjLane entries by insertion and lists the bodies with more
+// (in the cursors, free by now); a wave takes each of those, every lane
+// ranking up to four entries against all.  Two cloth layers in contact give a
+// particle tens of entries: 200 us by insertion alone for 9216 of them, 20 us
+// this way.  Past 256 entries one lane inserts.
+constexpr uint32_t kCadjLane = 8, kCadjWave = 256;
+__device__ __forceinline__ void cadj_insertion(uint32_t* a, uint32_t n) {
   for (uint32_t i = 1; i < n; i++) {
-    uint32_t v = S.dAdjList[s + i];
+    uint32_t v = a[i];
     uint32_t j = i;
-    while (j > 0 && S.dAdjList[s + j - 1] > v) {
-      S.dAdjList[s + j] = S.dAdjList[s + j - 1];
+    while (j > 0 && a[j - 1] > v) {
+      a[j] = a[j - 1];
       j--;
     }
-    S.dAdjList[s + j] = v;
+    a[j] = v;
+  }
+}
+__global__ void __launch_bounds__(256) k_cadj_sort(DeviceState S, StepParams P) {
+  const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63u;
+  const uint32_t n = gid < P.numBodies ? S.dAdjCount[gid] : 0u;
+  const bool longer = n > kCadjLane;
+  if (n > 1 && !longer) cadj_insertion(S.dAdjList + S.dAdjStart[gid], n);
+  const uint64_t m = __ballot(longer);
+  if (m == 0ull) return;
+  uint32_t at = 0;
+  if (lane == 0) at = atomicAdd(&S.counters[CTR_LONG_ADJ], (uint32_t)__popcll(m));
+  at = __shfl(at, 0, 64);
+  if (longer) S.dAdjCursor[at + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = gid;
+}
+__global__ void __launch_bounds__(256) k_cadj_sort_long(DeviceState S) {
+  const uint32_t lane = threadIdx.x & 63u, count = S.counters[CTR_LONG_ADJ];
+  for (uint32_t q = blockIdx.x * 4u + (threadIdx.x >> 6); q < count; q += gridDim.x * 4u) {
+    const uint32_t body = S.dAdjCursor[q], n = S.dAdjCount[body];
+    uint32_t* a = S.dAdjList + S.dAdjStart[body];
+    if (n > kCadjWave) {
+      if (lane == 0) cadj_insertion(a, n);
+      continue;
+    }
+    uint32_t v[4], rank[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) v[k] = lane + 64u * k < n ? a[lane + 64u * k] : 0xFFFFFFFFu;
+#pragma unroll
+    for (uint32_t b = 0; b < 4; b++) {
+      const uint32_t m = n > 64u * b ? (n - 64u * b < 64u ? n - 64u * b : 64u) : 0u;
+      for (uint32_t j = 0; j < m; j++) {
+        const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)v[b], (int)j), at = 64u * b + j;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) rank[k] += x < v[k] || (x == v[k] && at < lane + 64u * k) ? 1u : 0u;
+      }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++)
+      if (lane + 64u * k < n) a[rank[k]] = v[k];
   }
 }
 
@@ -100,6 +148,8 @@ void launch_contact_adjacency(hipStream_t st, const DeviceState& S, const StepPa
   hipLaunchKernelGGL(k_cadj_cursor, dim3(bb), dim3(256), 0, st, S, P);
   hipLaunchKernelGGL(k_cadj_scatter, dim3(blocks), dim3(256), 0, st, S, P);
   hipLaunchKernelGGL(k_cadj_sort, dim3(bb), dim3(256), 0, st, S, P);
+  const uint32_t lb = (P.numBodies + 3) / 4;
+  hipLaunchKernelGGL(k_cadj_sort_long, dim3(lb < 2048u ? lb : 2048u), dim3(256), 0, st, S);
 }
 
 // Static palette: c_v = lowest color unused by lower-index dynamic clique

