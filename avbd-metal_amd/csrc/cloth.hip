@@ -21,6 +21,7 @@ constexpr uint32_t kRtMaxPerTri = 4u;
 constexpr float kEeInteriorEps = 0.02f;
 constexpr float kDatGeometryEps = 1.0e-8f;
 constexpr uint32_t kDatLdsCap = 512u;  // per-producer sorted-emission buffer (LDS)
+constexpr uint32_t kDatStash = kDatStashSlots;      // partners the count pass keeps for the emit pass
 
 // Ericson, Real-Time Collision Detection 5.1.5 (25_cloth.metal:26-61)
 __device__ __forceinline__ V3 closest_pt_triangle(V3 p, V3 a, V3 b, V3 c, V3& bary) {
@@ -134,11 +135,30 @@ __device__ __forceinline__ CellRange range_of(V3 lo, V3 hi, float cs) {
   return r;
 }
 __device__ __forceinline__ int cell_add(int c, int i) { return (int)((uint32_t)c + (uint32_t)i); }
-__device__ __forceinline__ bool axis_in(int c, int c0, int s) {
-  return (long long)c >= c0 && (long long)c <= (long long)c0 + s;
-}
+// a cover ends at or below INT_MAX, so the wrapped difference is in [0, s]
+// only for the cover's own cells
+__device__ __forceinline__ bool axis_in(int c, int c0, int s) { return (uint32_t)c - (uint32_t)c0 <= (uint32_t)s; }
 __device__ __forceinline__ bool in_range(const CellRange& r, Cell3 c) {
   return axis_in(c.x, r.c0.x, r.sx) && axis_in(c.y, r.c0.y, r.sy) && axis_in(c.z, r.c0.z, r.sz);
+}
+
+// An element's cover as the binning wrote it: the queries' owner tests read
+// these 16 bytes instead of dividing the box by the cell size again.
+__device__ __forceinline__ U4 cover_pack(const CellRange& r) {
+  return U4{(uint32_t)r.c0.x, (uint32_t)r.c0.y, (uint32_t)r.c0.z, (uint32_t)(r.sx | (r.sy << 2) | (r.sz << 4))};
+}
+__device__ __forceinline__ CellRange cover_of(U4 c) {
+  CellRange r;
+  r.c0 = Cell3{(int)c.x, (int)c.y, (int)c.z};
+  r.sx = (int)(c.w & 3u);
+  r.sy = (int)((c.w >> 2) & 3u);
+  r.sz = (int)(c.w >> 4);
+  r.over = false;
+  return r;
+}
+// the low ten bits of a cell's coordinates, x in the lowest
+__device__ __forceinline__ uint32_t cell_low(Cell3 c) {
+  return ((uint32_t)c.x & 1023u) | (((uint32_t)c.y & 1023u) << 10) | (((uint32_t)c.z & 1023u) << 20);
 }
 
 }  // namespace
@@ -234,8 +254,10 @@ __global__ void __launch_bounds__(256) k_el_bin(DeviceState S, StepParams P) {
         ge = S.clothGroup[e.x];
         if (S.clothGroup[e.y] != ge) ge = 0u;
       }
+      if (finite3(lo) && finite3(hi)) r = range_of(lo, hi, P.elemCellSize);
       S.elemBox[2 * gid] = f4(lo, as_float(ge));
-      S.elemBox[2 * gid + 1] = f4(hi, 0.0f);
+      S.elemBox[2 * gid + 1] = f4(hi, as_float(cell_low(r.c0)));
+      S.elemCover[gid] = cover_pack(r);
     }
     if (!finite3(lo) || !finite3(hi)) {
       if (!SCATTER) {
@@ -244,7 +266,7 @@ __global__ void __launch_bounds__(256) k_el_bin(DeviceState S, StepParams P) {
       }
       live = false;
     } else {
-      r = range_of(lo, hi, P.elemCellSize);
+      if (SCATTER) r = cover_of(S.elemCover[gid]);
       if (!SCATTER && r.over) atomicAdd(&S.counters[CTR_DAT_OVERFLOW], 1u);
     }
   }
@@ -321,8 +343,7 @@ __device__ __forceinline__ bool vt_rest(const DeviceState& S, const StepParams& 
                                         uint32_t ns, uint32_t ne, uint32_t entry, float q2) {
   U4 t = S.tris[entry];
   if (t.x == v || t.y == v || t.z == v) return false;
-  const F4 blo = S.elemBox[2 * entry], bhi = S.elemBox[2 * entry + 1];
-  if (!in_range(range_of(xyz(blo), xyz(bhi), P.elemCellSize), cell)) return false;
+  if (!in_range(cover_of(S.elemCover[entry]), cell)) return false;
   V3 bary;
   V3 q = closest_pt_triangle(p, P3(S, t.x), P3(S, t.y), P3(S, t.z), bary);
   V3 d = p - q;
@@ -341,13 +362,18 @@ __device__ __forceinline__ bool vt_accept(const DeviceState& S, const StepParams
   return vt_box(S, P, p, entry, noSelf) && vt_rest(S, P, v, p, cell, ns, ne, entry, q2);
 }
 
+// `mask`, `want`: the axes on which the visited cell lies past the producer's
+// first cell, and the cell's low bits there.  On those axes the owner cell is
+// the partner's first cell, so any other partner fails the owner test; most
+// of a producer's repeated meetings with one partner end here.
 __device__ __forceinline__ bool ee_box(const DeviceState& S, const StepParams& P, uint32_t gid, V3 a0, V3 a1,
-                                       uint32_t entry, uint32_t noSelf) {
+                                       uint32_t entry, uint32_t noSelf, uint32_t mask, uint32_t want) {
   if ((entry & kElemEdgeBit) == 0u) return false;
   uint32_t other = entry & ~kElemEdgeBit;
   if (other <= gid || other >= P.numEdges) return false;
   const F4 blo = S.elemBox[2 * (P.numTris + other)], bhi = S.elemBox[2 * (P.numTris + other) + 1];
   if (noSelf != 0u && as_uint(blo.w) == noSelf) return false;
+  if (((as_uint(bhi.w) ^ want) & mask) != 0u) return false;
   return !boxes_apart(vmin(a0, a1), vmax(a0, a1), blo, bhi, kBoxSlack);
 }
 
@@ -356,8 +382,7 @@ __device__ __forceinline__ bool ee_rest(const DeviceState& S, const StepParams& 
                                         Cell3 cell, uint32_t other, float q2) {
   U2 b = S.edges[other];
   if (b.x == a.x || b.x == a.y || b.y == a.x || b.y == a.y) return false;
-  const F4 blo = S.elemBox[2 * (P.numTris + other)], bhi = S.elemBox[2 * (P.numTris + other) + 1];
-  CellRange br = range_of(xyz(blo), xyz(bhi), P.elemCellSize);
+  const CellRange br = cover_of(S.elemCover[P.numTris + other]);
   // owned by the minimum cell of tight(A) x padded(B)
   Cell3 o0{max(ar.c0.x, br.c0.x), max(ar.c0.y, br.c0.y), max(ar.c0.z, br.c0.z)};
   if (!in_range(ar, o0) || !in_range(br, o0)) return false;
@@ -379,7 +404,7 @@ __device__ __forceinline__ bool ee_rest(const DeviceState& S, const StepParams& 
 __device__ __forceinline__ bool ee_accept(const DeviceState& S, const StepParams& P, uint32_t gid, U2 a, V3 a0, V3 a1,
                                           const CellRange& ar, uint32_t ns0, uint32_t ne0, uint32_t ns1, uint32_t ne1,
                                           Cell3 cell, uint32_t entry, float q2, uint32_t noSelf) {
-  return ee_box(S, P, gid, a0, a1, entry, noSelf) &&
+  return ee_box(S, P, gid, a0, a1, entry, noSelf, 0u, 0u) &&
          ee_rest(S, P, a, a0, a1, ar, ns0, ne0, ns1, ne1, cell, entry & ~kElemEdgeBit, q2);
 }
 
@@ -451,67 +476,102 @@ __device__ __forceinline__ U4 dat_record(const StepParams& P, uint32_t prod, uin
 
 }  // namespace
 
-// Emit pass: one wave (64 lanes) per producer with pairs, four producers
-// per block; the accepted partners are gathered in LDS and written ranked by
-// partner index at datStart[prod] (k_dat_count below is the count pass).
-__global__ void __launch_bounds__(256) k_dat_pairs(DeviceState S, StepParams P) {
-  __shared__ uint32_t buf[4][kDatLdsCap];
-  const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-  const uint32_t prod = blockIdx.x * 4u + wv;
+// Emit pass.  The count pass left the first kDatStash partners of every
+// producer; one lane looks at each producer, and the wave then takes two of
+// its producers with pairs at a time, 32 lanes ranking the stashed partners
+// and writing their records at datStart[prod].  Producers with more partners
+// are listed for k_dat_pairs.  Two folded layers of 96^2 particles: 33 us
+// where walking every producer's buckets again took 157 us (16 kept partners:
+// 17 us, and 53 us for the listed producers).
+__global__ void __launch_bounds__(256) k_dat_emit(DeviceState S, StepParams P) {
+  const uint32_t lane = threadIdx.x & 63u, sub = lane & (kDatStash - 1u), grp = lane / kDatStash;
   const uint32_t nProd = P.numParticles + P.numEdges;
-  const bool valid = prod < nProd;
+  const uint32_t prod = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t start = 0, want = 0;
-  if (valid) {
+  if (prod < nProd) {
     start = S.datStart[prod];
     want = S.datStart[prod + 1] - start;
   }
-  const bool big = want > kDatLdsCap;
-  uint32_t n = 0;
-  if (valid && want != 0u && !big) {
-    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    dat_visit(S, P, prod, lane, 64u, false, [&](bool acc, uint32_t other) {
-      uint64_t m = __ballot(acc);
-      if (acc) {
-        uint32_t r = n + (uint32_t)__popcll(m & below);
-        if (r < kDatLdsCap) buf[wv][r] = other;
+  if (want > kDatStash) S.datBig[atomicAdd(&S.counters[CTR_DAT_BIG], 1u)] = prod;
+  uint64_t m = __ballot(want != 0u && want <= kDatStash);
+  while (m != 0ull) {
+    // the group's producer: the grp-th of the next 64 / kDatStash
+    uint64_t mine = m;
+    for (uint32_t g = 0; g < 64u / kDatStash; g++) {
+      if (g < grp) mine &= mine - 1ull;
+      m &= m - 1ull;
+    }
+    const int src = mine != 0ull ? __ffsll((unsigned long long)mine) - 1 : 0;
+    // every lane takes part in the shuffles: the source lane may be in a group without a producer
+    const uint32_t has = (uint32_t)__shfl((int)want, src), at = (uint32_t)__shfl((int)start, src);
+    const uint32_t n = mine != 0ull ? has : 0u, p = (prod - lane) + (uint32_t)src;
+    const uint32_t x = sub < n ? S.datStash[(uint64_t)p * kDatStash + sub] : 0xFFFFFFFFu;
+    uint32_t rank = 0;
+    for (int j = 0; j < (int)kDatStash; j++) rank += (uint32_t)__shfl((int)x, j, (int)kDatStash) < x ? 1u : 0u;
+    if (sub < n && at + rank < P.maxDatPairs) {
+      U4 r = dat_record(P, p, x);
+      if (r.x == kDatVT) r.y = S.particleIdx[p];
+      S.datPairs[at + rank] = r;
+    }
+  }
+}
+
+// The listed producers: one wave (64 lanes) walks a producer's buckets again,
+// gathers the accepted partners in LDS and writes them ranked by index.
+__global__ void __launch_bounds__(256) k_dat_pairs(DeviceState S, StepParams P) {
+  __shared__ uint32_t buf[4][kDatLdsCap];
+  const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const uint32_t nBig = S.counters[CTR_DAT_BIG];
+  for (uint32_t item = blockIdx.x * 4u + wv; item < nBig; item += gridDim.x * 4u) {
+    const uint32_t prod = S.datBig[item];
+    const uint32_t start = S.datStart[prod], want = S.datStart[prod + 1] - start;
+    const uint32_t wo = prod < P.numParticles ? S.particleIdx[prod] : 0u;
+    if (want <= kDatLdsCap) {
+      uint32_t n = 0;
+      dat_visit(S, P, prod, lane, 64u, false, [&](bool acc, uint32_t other) {
+        uint64_t m = __ballot(acc);
+        if (acc) {
+          uint32_t r = n + (uint32_t)__popcll(m & below);
+          if (r < kDatLdsCap) buf[wv][r] = other;
+        }
+        n += (uint32_t)__popcll(m);
+      });
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const uint32_t cnt = n < want ? n : want;
+      for (uint32_t i = lane; i < cnt; i += 64u) {
+        uint32_t x = buf[wv][i], rank = 0;
+        for (uint32_t j = 0; j < cnt; j++) rank += buf[wv][j] < x ? 1u : 0u;
+        uint32_t slot = start + rank;
+        if (slot < P.maxDatPairs) {
+          U4 r = dat_record(P, prod, x);
+          if (r.x == kDatVT) r.y = wo;
+          S.datPairs[slot] = r;
+        }
       }
-      n += (uint32_t)__popcll(m);
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
+    // more partners than the LDS buffer holds: one lane inserts in order
+    if (lane != 0) continue;
+    uint32_t cnt = 0;
+    dat_visit(S, P, prod, 0u, 1u, false, [&](bool acc, uint32_t other) {
+      if (!acc || cnt >= want) return;
+      uint32_t j = cnt;
+      while (j > 0 && start + j - 1 < P.maxDatPairs && S.datPairs[start + j - 1].z > other) {
+        if (start + j < P.maxDatPairs) S.datPairs[start + j] = S.datPairs[start + j - 1];
+        j--;
+      }
+      if (start + j < P.maxDatPairs) {
+        U4 r = dat_record(P, prod, other);
+        if (r.x == kDatVT) r.y = wo;
+        S.datPairs[start + j] = r;
+      }
+      cnt++;
     });
   }
-  __syncthreads();
-  if (!valid || want == 0u) return;
-  const uint32_t wo = prod < P.numParticles ? S.particleIdx[prod] : 0u;
-  if (!big) {
-    uint32_t cnt = n < want ? n : want;
-    for (uint32_t i = lane; i < cnt; i += 64u) {
-      uint32_t x = buf[wv][i], rank = 0;
-      for (uint32_t j = 0; j < cnt; j++) rank += buf[wv][j] < x ? 1u : 0u;
-      uint32_t slot = start + rank;
-      if (slot < P.maxDatPairs) {
-        U4 r = dat_record(P, prod, x);
-        if (r.x == kDatVT) r.y = wo;
-        S.datPairs[slot] = r;
-      }
-    }
-    return;
-  }
-  // more partners than the LDS buffer holds: one lane inserts in order
-  if (lane != 0) return;
-  uint32_t cnt = 0;
-  dat_visit(S, P, prod, 0u, 1u, false, [&](bool acc, uint32_t other) {
-    if (!acc || cnt >= want) return;
-    uint32_t j = cnt;
-    while (j > 0 && start + j - 1 < P.maxDatPairs && S.datPairs[start + j - 1].z > other) {
-      if (start + j < P.maxDatPairs) S.datPairs[start + j] = S.datPairs[start + j - 1];
-      j--;
-    }
-    if (start + j < P.maxDatPairs) {
-      U4 r = dat_record(P, prod, other);
-      if (r.x == kDatVT) r.y = wo;
-      S.datPairs[start + j] = r;
-    }
-    cnt++;
-  });
 }
 
 // Count pass: 16 lanes per producer, four producers per wave.  The groups
@@ -521,7 +581,8 @@ __global__ void __launch_bounds__(256) k_dat_pairs(DeviceState S, StepParams P) 
 // the queue holds 64 of them the remaining tests run on the full wave.  The
 // accepted count is the same as the emit pass's walk (both evaluate the same
 // predicate on the same candidates); the queue only keeps the long tests off
-// lanes the box filter already emptied.
+// lanes the box filter already emptied.  The first kDatStash accepted partners
+// of a producer are kept for the emit pass.
 namespace {
 
 constexpr uint32_t kDatQueue = 128u;  // < 64 held + up to 64 added per step
@@ -540,18 +601,17 @@ __device__ __forceinline__ Cell3 cover_cell(const CellRange& r, uint32_t ci) {
 
 }  // namespace
 
-// Six waves per SIMD (80 VGPRs, four spilled) measured 1 % faster on the
-// 256^2 cloth step than the compiler's choice of five (85 VGPRs); eight
-// spill 36 registers.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k_dat_count(DeviceState S, StepParams P) {
+// Five waves per SIMD (95 VGPRs); six would spill 18 registers.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_dat_count(DeviceState S, StepParams P) {
   __shared__ DatProducer ctx[16];
-  __shared__ uint32_t qEntry[4][kDatQueue], qTag[4][kDatQueue];
+  __shared__ uint32_t qEntry[4][kDatQueue], qTag[4][kDatQueue], cnt[16];
   const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6, sub = threadIdx.x & 15u, grp = lane >> 4;
   const uint32_t slot = threadIdx.x >> 4;
   const uint32_t prod = blockIdx.x * 16u + slot;
   const uint32_t nProd = P.numParticles + P.numEdges;
   const float q2 = P.datQueryRadius * P.datQueryRadius;
   const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  if (threadIdx.x < 16u) cnt[threadIdx.x] = 0u;
   // producer set-up: every lane of a group computes the same values
   const bool vt = prod < P.numParticles;
   bool live = prod < nProd;
@@ -612,16 +672,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 
   // a V-T producer reads its cell's triangles, an E-E producer each cover
   // cell's edges (the buckets lay out triangles, then edges)
+  uint32_t mask = 0u, want = 0u;
   auto bucket = [&](uint32_t ci, uint32_t& bs, uint32_t& be) {
     const Cell3 c = cover_cell(ar, ci);
+    mask = (c.x != ar.c0.x ? 1023u : 0u) | (c.y != ar.c0.y ? 1023u << 10 : 0u) | (c.z != ar.c0.z ? 1023u << 20 : 0u);
+    want = cell_low(c);
     const uint32_t h = cell_hash(c.x, c.y, c.z, 0u, P.elemHashSize);
     const uint32_t o = vt ? 0u : 1u;
     bs = S.elemCellStart[2u * h + o];
     be = S.elemCellStart[2u * h + o + 1u];
   };
   // the remaining tests on queue items [0, n), then the queue's tail moves
-  // to its head; `count` gathers the accepted items of this lane's producer
-  uint32_t qn = 0, count = 0;
+  // to its head; `cnt` counts the accepted items of each producer
+  uint32_t qn = 0;
   auto drain = [&](uint32_t n) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -647,9 +710,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
                       entry & ~kElemEdgeBit, q2);
       }
     }
-    for (uint32_t gg = 0; gg < 4u; gg++) {
-      const uint64_t m = __ballot(acc && g == gg);
-      if (gg == grp) count += (uint32_t)__popcll(m);
+    if (acc) {
+      const uint32_t at = atomicAdd(&cnt[wv * 4u + g], 1u);
+      if (at < kDatStash)
+        S.datStash[(uint64_t)(blockIdx.x * 16u + wv * 4u + g) * kDatStash + at] = entry & ~kElemEdgeBit;
     }
     if (qn > n) {
       const bool mv = lane < qn - n;
@@ -677,7 +741,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
     bool surv = false;
     if (more && k < ke) {
       entry = S.elemCells[k];
-      surv = vt ? vt_box(S, P, p0, entry, noSelf) : ee_box(S, P, gid, p0, p1, entry, noSelf);
+      surv = vt ? vt_box(S, P, p0, entry, noSelf) : ee_box(S, P, gid, p0, p1, entry, noSelf, mask, want);
     }
     k0 += 16u;
     const uint64_t m = __ballot(surv);
@@ -690,7 +754,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
     if (qn >= 64u) drain(64u);
   }
   if (qn > 0u) drain(qn);
-  if (prod < nProd && sub == 0) S.datCount[prod] = count;
+  __syncthreads();
+  if (prod < nProd && sub == 0) S.datCount[prod] = cnt[slot];
 }
 
 // The frame's demand counters keep the larger of its two queries (step
@@ -703,6 +768,7 @@ __global__ void k_dat_finalize(DeviceState S, StepParams P) {
   atomicMax(&S.counters[CTR_DAT_PAIRS], total);
   atomicMax(&S.counters[CTR_DAT_VT], vt);
   atomicMax(&S.counters[CTR_DAT_EE], total - vt);
+  S.counters[CTR_DAT_BIG] = 0u;  // the frame queries twice
 }
 
 // ---------------------------------------------------------------------------
@@ -2056,10 +2122,10 @@ void launch_dat_pairs(hipStream_t st, const DeviceState& S, const StepParams& P,
                      S.elemCellStart, slots);
   hipLaunchKernelGGL(k_el_bin<true>, dim3(eb), dim3(256), 0, st, S, P);
   uint32_t nProd = P.numParticles + P.numEdges;
-  uint32_t pb = (nProd + 3) / 4;
   hipLaunchKernelGGL(k_dat_count, dim3((nProd + 15) / 16), dim3(256), 0, st, S, P);
   launch_exclusive_scan(st, S.datCount, S.datStart, nProd + 1, S.scanScratch);
-  hipLaunchKernelGGL(k_dat_pairs, dim3(pb), dim3(256), 0, st, S, P);
+  hipLaunchKernelGGL(k_dat_emit, dim3((nProd + 255) / 256), dim3(256), 0, st, S, P);
+  hipLaunchKernelGGL(k_dat_pairs, dim3(cap_blocks(64ull * nProd, gridCap)), dim3(256), 0, st, S, P);
   hipLaunchKernelGGL(k_dat_finalize, dim3(1), dim3(1), 0, st, S, P);
 }
 

@@ -21,6 +21,7 @@ constexpr float kPenaltyMax = 1.0e10f;
 constexpr float kPenaltyMaxT = 1.0e6f;   // tangential / soft normal cap
 constexpr float kStickThresh = 1.0e-5f;
 constexpr int kMaxColors = 64;
+constexpr uint32_t kDatStashSlots = 32;  // partners of a surface pair producer kept between its two passes
 constexpr int kMaxContacts = 8;
 constexpr uint32_t kColorPasses = 20;      // Jacobi passes of the dynamic coloring
 // Bodies of an island one workgroup colors / solves.  The solve crosses over
@@ -109,6 +110,7 @@ enum Counter : uint32_t {
   CTR_BP_BIG,              // producers with more partners than the stash holds
   CTR_DYN_CONTACT,         // some contact this frame joins two dynamic bodies (or is an element contact)
   CTR_LONG_ADJ,            // bodies whose contact segment a wave sorts
+  CTR_DAT_BIG,             // surface pair producers with more partners than the stash holds
   CTR_TOTAL = 16 + 2 * kMaxColors + 24
 };
 

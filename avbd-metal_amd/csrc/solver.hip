@@ -1903,9 +1903,10 @@ avbd_status build_static_and_upload(avbd_solver* s, const avbd_scene_desc* d) {
     ALLOC(S.selfCollision, cl ? nb : 1u)
     ALLOC(S.elemCellCount, cl ? 2 * s->elemHashSize + 1 : 1u) ALLOC(S.elemCellStart, cl ? 2 * s->elemHashSize + 1 : 1u)
     ALLOC(S.elemCellCursor, cl ? 2 * s->elemHashSize : 1u) ALLOC(S.elemCells, std::max<uint64_t>(1, 64ull * nElem))
-    ALLOC(S.elemBox, std::max<uint32_t>(2, 2 * nElem))
+    ALLOC(S.elemBox, std::max<uint32_t>(2, 2 * nElem)) ALLOC(S.elemCover, std::max<uint32_t>(1, nElem))
     ALLOC(S.datAnchor, cl ? nb : 1u) ALLOC(S.datT, cl ? nb : 1u)
     ALLOC(S.datCount, nProd + 1) ALLOC(S.datStart, nProd + 1)
+    ALLOC(S.datStash, (uint64_t)kDatStashSlots * nProd) ALLOC(S.datBig, nProd)
     ALLOC(S.datPairs, cl ? s->maxDatPairs : 1u)
     uint32_t flagN = cl ? std::max(std::max(s->nTris, s->maxDatPairs), s->nParticles + s->numContactEdges) + 1 : 1u;
     ALLOC(S.softFlag, flagN) ALLOC(S.softStart, flagN)

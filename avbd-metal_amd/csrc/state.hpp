@@ -104,10 +104,12 @@ struct DeviceState {
   uint32_t* selfCollision;    // per body: its surface self-collides
   // element grid: counts / starts / cursors per (bucket, triangles | edges), interleaved
   uint32_t *elemCellCount, *elemCellStart, *elemCellCursor, *elemCells;
-  F4* elemBox;                // per element (triangles, then edges): padded box lo, hi; lo.w = surface group bits (0: mixed)
+  F4* elemBox;                // per element (triangles, then edges): padded box lo, hi; lo.w = surface group bits (0: mixed), hi.w = low cover bits
+  U4* elemCover;              // per element: first cell and spans of its cover
   F4* datAnchor;              // Planar-DAT anchor pose of the color passes (accepted predictor pose)
   uint32_t* datT;             // per body: step fraction of the running pass (f32 bits, 1.0 between passes)
   uint32_t *datCount, *datStart;  // per producer: surface particles, then edges (+1 total)
+  uint32_t *datStash, *datBig;    // per producer: its first kDatStashSlots partners; producers with more
   U4* datPairs;               // (kind, owner, other, 0), producer-major, other ascending
   uint32_t *softFlag, *softStart;  // emission counts / offsets (RT per triangle, DAT per pair)
   SoftRec *soft, *prevSoft;
