@@ -28,9 +28,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 namespace {
 
 constexpr int kIn = kMlpIn, kInPad = kMlpInPad, kHid = kMlpHidden, kOutPad = kMlpOutPad;
-// LDS row strides (bf16 elements): 80 B / 272 B / 48 B rows put the 16 rows
+// LDS row strides (bf16 elements): 80 B / 272 B rows put the 16 rows
 // of one operand fetch on 16 distinct 4-bank groups
-constexpr int kS1 = 40, kSH = 136, kS3 = 24, kSD = 40;
+constexpr int kS1 = 40, kSH = 136, kSD = 40;
 
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -61,11 +61,6 @@ struct LdsFwd {
   bf16 w2t[kHid * kSH];
   bf16 w3t[kOutPad * kSH];
 };
-struct LdsBack {
-  bf16 w2[kHid * kSH];
-  bf16 w3[kHid * kS3];
-};
-
 // copy a dense [rows][cols] bf16 matrix into LDS rows of `stride` (16-byte chunks)
 __device__ void stage(bf16* dst, const bf16* src, int rows, int cols, int stride) {
   const int chunks = cols / 8;
@@ -80,11 +75,6 @@ __device__ void load_fwd(const MlpDevice& M, LdsFwd& L) {
   stage(L.w2t, M.w2t, kHid, kHid, kSH);
   stage(L.w3t, M.w3t, kOutPad, kHid, kSH);
 }
-__device__ void load_back(const MlpDevice& M, LdsBack& L) {
-  stage(L.w2, M.w2, kHid, kHid, kSH);
-  stage(L.w3, M.w3, kHid, kOutPad, kS3);
-}
-
 // Forward of one 16-row tile by one wave.  h1, h2: the wave's [16][kSH] LDS
 // rows, left holding the bf16 activations.  Returns the layer-3 accumulator
 // (D layout) plus bias.
@@ -123,20 +113,17 @@ __device__ f32x4 tile_forward(const MlpDevice& M, const LdsFwd& W, const bf16* X
   return acc;
 }
 
-// 16 rows of a wave's LDS rows, feature-major into dst[f * P + r0 ..]:
-// lane l writes features l, l + 64, ... as 32 contiguous bytes each
-__device__ void store_transposed(const bf16* h, int stride, int features, bf16* dst, size_t P, uint32_t r0,
-                                 uint32_t lane) {
-  for (int f = lane; f < features; f += 64) {
-    bf16x8 lo, hi;
+// one feature of 16 LDS rows, 32 contiguous bytes of its row in dst[f * P + r0 ..]
+__device__ __forceinline__ void store_transposed(const bf16* h, int stride, uint32_t f, bf16* dst, size_t P,
+                                                 uint32_t r0) {
+  bf16x8 lo, hi;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      lo[j] = h[j * stride + f];
-      hi[j] = h[(8 + j) * stride + f];
-    }
-    *(bf16x8*)(dst + (size_t)f * P + r0) = lo;
-    *(bf16x8*)(dst + (size_t)f * P + r0 + 8) = hi;
+  for (int j = 0; j < 8; j++) {
+    lo[j] = h[j * stride + f];
+    hi[j] = h[(8 + j) * stride + f];
   }
+  *(bf16x8*)(dst + (size_t)f * P + r0) = lo;
+  *(bf16x8*)(dst + (size_t)f * P + r0 + 8) = hi;
 }
 
 }  // namespace
@@ -171,106 +158,140 @@ __global__ void __launch_bounds__(64 * kFwdWaves) k_mlp_forward(MlpDevice M, con
 // ---------------------------------------------------------------------------
 // training, pass 1: forward + activation gradients of
 // L = sum_r |y_r - t_r|^2 * lossScale over every 16-row tile of the padded
-// batch (rows >= `rows` carry zero gradient); writes the feature-major
-// operands of the weight-gradient GEMMs and adds the bias gradients and
-// sum |y - t|^2 atomically
+// batch (rows >= `rows` carry zero gradient; row r is dataset row perm[r], or
+// r without perm); writes the feature-major operands of the weight-gradient
+// GEMMs and adds the bias gradients and sum |y - t|^2 atomically.
+//
+// A workgroup owns a tile and each of its four waves two of the eight column
+// tiles of every layer, so the weights a wave multiplies fit its registers:
+// they are read once, all loads in flight together, straight from the L2.
+// One wave per tile needs every weight, staged through 86 KB of LDS: at 4096
+// rows that filled 64 CUs, was bound by the staging, and took 21 us (15 us
+// now).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_mlp_act_grad(MlpDevice M, MlpTrain T, const bf16* X, const float* Tgt,
-                                                      uint32_t rows, float lossScale) {
-  __shared__ LdsFwd W;
-  __shared__ LdsBack B;
-  __shared__ bf16 hbuf[4][2][16 * kSH];
-  __shared__ bf16 dzbuf[4][16 * kSD];
-  load_fwd(M, W);
-  load_back(M, B);
-  __syncthreads();
-  const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+                                                      const uint32_t* perm, uint32_t rows, float lossScale) {
+  __shared__ bf16 h1[16 * kSH], h2[16 * kSH], dz[16 * kSD];
+  const uint32_t tid = threadIdx.x, wv = tid >> 6, lane = tid & 63u;
   const uint32_t ar = lane & 15u, ak = 8u * (lane >> 4), dr = 4u * (lane >> 4);
-  bf16 *h1 = hbuf[wv][0], *h2 = hbuf[wv][1], *dz = dzbuf[wv];
-  float db1[kHid / 16], db2[kHid / 16], db3 = 0.0f, loss = 0.0f;
+  constexpr int kN = 2, kK = kHid / 32;  // column tiles of a wave, k steps of a hidden layer
+  bf16x8 w1[kN], w2[kN][kK], w3[kK], v3t[kN], v2[kN][kK];
+  float b1[kN], b2[kN], db1[kN], db2[kN], db3 = 0.0f, loss = 0.0f;
 #pragma unroll
-  for (int i = 0; i < kHid / 16; i++) db1[i] = db2[i] = 0.0f;
+  for (int c = 0; c < kN; c++) {
+    const uint32_t col = (kN * wv + c) * 16 + ar;
+    w1[c] = ld8(M.w1t + col * kInPad + ak);
+    v3t[c] = lane < 32 ? ld8(M.w3 + col * kOutPad + ak) : zero8();  // k = outputs, zero beyond 16
+#pragma unroll
+    for (int kt = 0; kt < kK; kt++) {
+      w2[c][kt] = ld8(M.w2t + col * kHid + kt * 32 + ak);
+      v2[c][kt] = ld8(M.w2 + col * kHid + kt * 32 + ak);
+    }
+    b1[c] = M.b1[col];
+    b2[c] = M.b2[col];
+    db1[c] = db2[c] = 0.0f;
+  }
+#pragma unroll
+  for (int kt = 0; kt < kK; kt++) w3[kt] = ld8(M.w3t + ar * kHid + kt * 32 + ak);
+  const float b3 = M.b3[ar];
   const size_t P = T.rowsPad;
   const uint32_t tiles = T.rowsPad / 16;
-  for (uint32_t t = blockIdx.x * 4 + wv; t < tiles; t += gridDim.x * 4) {
-    const uint32_t r0 = t * 16;
-    f32x4 y = tile_forward(M, W, X, rows, r0, h1, h2, lane);
-    // dY = 2 (y - t) lossScale (D layout; columns >= nOut and padded rows are zero)
+  for (uint32_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const uint32_t r0 = t * 16, row = r0 + ar;
+    const uint32_t src = row >= rows ? 0u : perm ? perm[row] : row;
+    const bf16x8 a1 = row < rows ? ld8(X + (size_t)src * kInPad + ak) : zero8();
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      uint32_t r = r0 + dr + i;
-      float g = 0.0f;
-      if (r < rows && ar < M.nOut) {
-        float e = y[i] - Tgt[(size_t)r * M.nOut + ar];
-        loss += e * e;
-        g = 2.0f * e * lossScale;
-      }
-      db3 += g;
-      dz[(dr + i) * kSD + ar] = (bf16)g;
-      dz[(dr + i) * kSD + 16 + ar] = (bf16)0.0f;
+    for (int c = 0; c < kN; c++) {
+      const f32x4 acc = mfma(a1, w1[c], zero4());
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        h1[(dr + i) * kSH + (kN * wv + c) * 16 + ar] = (bf16)fmaxf(acc[i] + b1[c], 0.0f);
     }
-    // feature-major copy of X: lane = 16 rows x 4 groups of 8 features
-    {
-      const uint32_t r = r0 + (lane & 15u), f0 = 8u * (lane >> 4);
-      bf16x8 xv = r < rows ? ld8(X + (size_t)r * kInPad + f0) : zero8();
+    if (wv == 3u) {  // feature-major copy of X: a lane's operand is one row's 8 features
 #pragma unroll
-      for (int j = 0; j < 8; j++) T.xt[(size_t)(f0 + j) * P + r] = xv[j];
+      for (int j = 0; j < 8; j++) T.xt[(size_t)(ak + j) * P + row] = a1[j];
     }
-    wave_sync();
-    store_transposed(h1, kSH, kHid, T.h1t, P, r0, lane);
-    store_transposed(h2, kSH, kHid, T.h2t, P, r0, lane);
-    store_transposed(dz, kSD, kOutPad, T.dyt, P, r0, lane);
-    wave_sync();  // the transposed reads of h2 precede its in-place update
-    // dH2 = dY W3^T (k = outputs, zero beyond 16); dZ2 = dH2 (h2 > 0) replaces h2 in place
-    const bf16x8 ady = ld8(dz + ar * kSD + ak);
+    __syncthreads();
 #pragma unroll
-    for (int nt = 0; nt < kHid / 16; nt++) {
-      bf16x8 bw = (lane < 32) ? ld8(B.w3 + (nt * 16 + ar) * kS3 + ak) : zero8();
-      f32x4 acc = mfma(ady, bw, zero4());
-      const uint32_t col = nt * 16 + ar;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const uint32_t rr = dr + i;
-        float g = ((float)h2[rr * kSH + col] > 0.0f && r0 + rr < rows) ? acc[i] : 0.0f;
-        db2[nt] += g;
-        h2[rr * kSH + col] = (bf16)g;  // each (row, col) is read and written by this lane only
-      }
-    }
-    wave_sync();
-    store_transposed(h2, kSH, kHid, T.dz2t, P, r0, lane);
-    // dH1 = dZ2 W2^T; dZ1 = dH1 (h1 > 0), then replaces h1
-#pragma unroll
-    for (int nt = 0; nt < kHid / 16; nt++) {
+    for (int c = 0; c < kN; c++) {
       f32x4 acc = zero4();
 #pragma unroll
-      for (int kt = 0; kt < kHid / 32; kt++)
-        acc = mfma(ld8(h2 + ar * kSH + kt * 32 + ak), ld8(B.w2 + (nt * 16 + ar) * kSH + kt * 32 + ak), acc);
-      const uint32_t col = nt * 16 + ar;
+      for (int kt = 0; kt < kK; kt++) acc = mfma(ld8(h1 + ar * kSH + kt * 32 + ak), w2[c][kt], acc);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        h2[(dr + i) * kSH + (kN * wv + c) * 16 + ar] = (bf16)fmaxf(acc[i] + b2[c], 0.0f);
+    }
+    __syncthreads();
+    if (wv == 0u) {
+      f32x4 y = zero4();
+#pragma unroll
+      for (int kt = 0; kt < kK; kt++) y = mfma(ld8(h2 + ar * kSH + kt * 32 + ak), w3[kt], y);
+      // dY = 2 (y - t) lossScale (D layout; columns >= nOut and padded rows are zero)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const uint32_t rr = dr + i;
-        float g = ((float)h1[rr * kSH + col] > 0.0f && r0 + rr < rows) ? acc[i] : 0.0f;
-        db1[nt] += g;
-        h1[rr * kSH + col] = (bf16)g;  // h1 is not an operand of this product
+        const uint32_t from = (uint32_t)__shfl((int)src, (int)(dr + i));
+        float g = 0.0f;
+        if (r0 + dr + i < rows && ar < M.nOut) {
+          float e = y[i] + b3 - Tgt[(size_t)from * M.nOut + ar];
+          loss += e * e;
+          g = 2.0f * e * lossScale;
+        }
+        db3 += g;
+        dz[(dr + i) * kSD + ar] = (bf16)g;
+        dz[(dr + i) * kSD + 16 + ar] = (bf16)0.0f;
       }
     }
-    wave_sync();
-    store_transposed(h1, kSH, kHid, T.dz1t, P, r0, lane);
-    wave_sync();  // the next tile overwrites h1 / h2 / dz
-  }
-  // bias gradients: the four row groups of each column, then one atomic per column and wave
+    if (tid < (uint32_t)kHid) store_transposed(h1, kSH, tid, T.h1t, P, r0);
+    else store_transposed(h2, kSH, tid - kHid, T.h2t, P, r0);
+    __syncthreads();  // dY is written, and the transposed reads of h2 precede its in-place update
+    if (tid < (uint32_t)kOutPad) store_transposed(dz, kSD, tid, T.dyt, P, r0);
+    // dH2 = dY W3^T; dZ2 = dH2 (h2 > 0) replaces h2 in place
+    const bf16x8 ady = ld8(dz + ar * kSD + ak);
 #pragma unroll
-  for (int nt = 0; nt < kHid / 16; nt++) {
-    float a = db1[nt], b = db2[nt];
+    for (int c = 0; c < kN; c++) {
+      const f32x4 acc = mfma(ady, v3t[c], zero4());
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        bf16& h = h2[(dr + i) * kSH + (kN * wv + c) * 16 + ar];
+        const float g = ((float)h > 0.0f && r0 + dr + i < rows) ? acc[i] : 0.0f;
+        db2[c] += g;
+        h = (bf16)g;  // each (row, col) is read and written by this lane only
+      }
+    }
+    __syncthreads();
+    if (tid < (uint32_t)kHid) store_transposed(h2, kSH, tid, T.dz2t, P, r0);
+    // dH1 = dZ2 W2^T; dZ1 = dH1 (h1 > 0), then replaces h1
+#pragma unroll
+    for (int c = 0; c < kN; c++) {
+      f32x4 acc = zero4();
+#pragma unroll
+      for (int kt = 0; kt < kK; kt++) acc = mfma(ld8(h2 + ar * kSH + kt * 32 + ak), v2[c][kt], acc);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        bf16& h = h1[(dr + i) * kSH + (kN * wv + c) * 16 + ar];
+        const float g = ((float)h > 0.0f && r0 + dr + i < rows) ? acc[i] : 0.0f;
+        db1[c] += g;
+        h = (bf16)g;  // h1 is not an operand of this product
+      }
+    }
+    __syncthreads();
+    if (tid >= (uint32_t)kHid) store_transposed(h1, kSH, tid - kHid, T.dz1t, P, r0);
+    __syncthreads();  // the next tile overwrites h1 / h2 / dz
+  }
+  // bias gradients: the four row groups of each column, then one atomic per column and workgroup
+#pragma unroll
+  for (int c = 0; c < kN; c++) {
+    float a = db1[c], b = db2[c];
     a += __shfl_xor(a, 16, 64);
     a += __shfl_xor(a, 32, 64);
     b += __shfl_xor(b, 16, 64);
     b += __shfl_xor(b, 32, 64);
     if (lane < 16) {
-      atomicAdd(&T.gb1[nt * 16 + lane], a);
-      atomicAdd(&T.gb2[nt * 16 + lane], b);
+      atomicAdd(&T.gb1[(kN * wv + c) * 16 + lane], a);
+      atomicAdd(&T.gb2[(kN * wv + c) * 16 + lane], b);
     }
   }
+  if (wv != 0u) return;
   db3 += __shfl_xor(db3, 16, 64);
   db3 += __shfl_xor(db3, 32, 64);
   if (lane < 16) atomicAdd(&T.gb3[lane], db3);
@@ -303,7 +324,18 @@ __global__ void __launch_bounds__(256) k_mlp_wgrad(MlpTrain T, uint32_t samplesP
   const bf16* ap = At + (size_t)(mt * 16 + ar) * P + ak;
   const bf16* bp = Bt + (size_t)(nt * 16 + ar) * P + ak;
   f32x4 acc = zero4();
-  for (uint32_t k = k0; k < k1; k += 32) acc = mfma(ld8(ap + k), ld8(bp + k), acc);
+  uint32_t k = k0;
+  for (; k + 128 <= k1; k += 128) {  // eight loads in flight
+    bf16x8 a[4], b[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      a[j] = ld8(ap + k + 32 * j);
+      b[j] = ld8(bp + k + 32 * j);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc = mfma(a[j], b[j], acc);
+  }
+  for (; k < k1; k += 32) acc = mfma(ld8(ap + k), ld8(bp + k), acc);
 #pragma unroll
   for (int i = 0; i < 4; i++) atomicAdd(&G[(mt * 16 + dr + i) * ldG + nt * 16 + ar], acc[i]);
 }
@@ -341,16 +373,53 @@ __global__ void __launch_bounds__(256) k_mlp_zero(MlpTrain T) {
   }
 }
 
-// Adam (beta1 0.9, beta2 0.999, eps 1e-8) on the f32 master parameters
-__global__ void __launch_bounds__(256) k_mlp_adam(MlpDevice M, MlpTrain T, float lr, float b1c, float b2c) {
+// One training step's tail: Adam (beta1 0.9, beta2 0.999, eps 1e-8) on the f32
+// master parameters, the bf16 operand layouts and f32 biases of the updated
+// values, the batch's share of the epoch's mean loss, and zeros where the
+// next batch adds its gradients.  20099 parameters (3 outputs) are nothing
+// but launches: five of 2.3 to 4.2 us each, one of 3.3 us now.
+__global__ void __launch_bounds__(256) k_mlp_update(MlpDevice M, MlpTrain T, float lr, float b1c, float b2c,
+                                                    float* lossDst, float lossScale) {
   const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < M.nParams; i += gridDim.x * blockDim.x) {
-    float g = T.grad[i];
-    float m = beta1 * T.m[i] + (1.0f - beta1) * g;
-    float v = beta2 * T.v[i] + (1.0f - beta2) * g * g;
-    T.m[i] = m;
-    T.v[i] = v;
-    M.params[i] -= lr * (m / b1c) / (sqrtf(v / b2c) + eps);
+  const uint32_t nOut = M.nOut, offB3 = (uint32_t)mlp_off_b3((int)nOut);
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0u) {
+    lossDst[0] += T.loss[0] * lossScale;
+    T.loss[0] = 0.0f;
+  }
+  if (i >= M.nParams) return;
+  float* gp;
+  if (i < (uint32_t)kMlpOffB1) gp = &T.gw1[i];  // rows 0..23 of gw1 [32][128]
+  else if (i < (uint32_t)kMlpOffW2) gp = &T.gb1[i - kMlpOffB1];
+  else if (i < (uint32_t)kMlpOffB2) gp = &T.gw2[i - kMlpOffW2];
+  else if (i < (uint32_t)kMlpOffW3) gp = &T.gb2[i - kMlpOffB2];
+  else if (i < offB3) gp = &T.gw3[((i - kMlpOffW3) / nOut) * kOutPad + (i - kMlpOffW3) % nOut];
+  else gp = &T.gb3[i - offB3];
+  const float g = *gp;
+  *gp = 0.0f;
+  const float m = beta1 * T.m[i] + (1.0f - beta1) * g;
+  const float v = beta2 * T.v[i] + (1.0f - beta2) * g * g;
+  T.m[i] = m;
+  T.v[i] = v;
+  const float p = M.params[i] - lr * (m / b1c) / (sqrtf(v / b2c) + eps);
+  M.params[i] = p;
+  // the padding of the operand layouts is zero since k_mlp_pack
+  if (i < (uint32_t)kMlpOffB1) {
+    M.w1t[(i % kHid) * kInPad + i / kHid] = (bf16)p;
+  } else if (i < (uint32_t)kMlpOffW2) {
+    M.b1[i - kMlpOffB1] = p;
+  } else if (i < (uint32_t)kMlpOffB2) {
+    const uint32_t q = i - kMlpOffW2;  // W2[in][out]
+    M.w2[q] = (bf16)p;
+    M.w2t[(q % kHid) * kHid + q / kHid] = (bf16)p;
+  } else if (i < (uint32_t)kMlpOffW3) {
+    M.b2[i - kMlpOffB2] = p;
+  } else if (i < offB3) {
+    const uint32_t a = (i - kMlpOffW3) / nOut, b = (i - kMlpOffW3) % nOut;
+    M.w3[a * kOutPad + b] = (bf16)p;
+    M.w3t[b * kHid + a] = (bf16)p;
+  } else {
+    M.b3[i - offB3] = p;
   }
 }
 
@@ -387,21 +456,6 @@ __global__ void __launch_bounds__(256) k_mlp_pack_input(const float* Xf, uint32_
   }
 }
 
-// batch rows by a permutation: four 16-byte chunks of X and the nOut targets per row
-__global__ void __launch_bounds__(256) k_mlp_gather_batch(const bf16* Xall, const float* Tall, const uint32_t* perm,
-                                                          uint32_t n, uint32_t nOut, bf16* X, float* T) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 4 * n; i += gridDim.x * blockDim.x) {
-    const uint32_t r = i >> 2, c = i & 3u, src = perm[r];
-    *(bf16x8*)(X + (size_t)r * kInPad + 8 * c) = *(const bf16x8*)(Xall + (size_t)src * kInPad + 8 * c);
-    for (uint32_t k = c; k < nOut; k += 4) T[(size_t)r * nOut + k] = Tall[(size_t)src * nOut + k];
-  }
-}
-
-// dst += loss * scale (one thread; per-epoch mean of the batch losses)
-__global__ void k_mlp_accum_loss(const float* loss, float* dst, float scale) {
-  if (threadIdx.x == 0) dst[0] += loss[0] * scale;
-}
-
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
@@ -417,12 +471,6 @@ void launch_mlp_pack_input(hipStream_t st, const float* Xf, uint32_t n, void* X)
   if (n == 0) return;
   hipLaunchKernelGGL(k_mlp_pack_input, dim3(grid_for(n * kInPad, 2048)), dim3(256), 0, st, Xf, n, (bf16*)X);
 }
-void launch_mlp_gather_batch(hipStream_t st, const void* Xall, const float* Tall, const uint32_t* perm, uint32_t n,
-                             uint32_t nOut, void* X, float* T) {
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_mlp_gather_batch, dim3(grid_for(4 * n, 2048)), dim3(256), 0, st, (const bf16*)Xall, Tall,
-                     perm, n, nOut, (bf16*)X, T);
-}
 void launch_mlp_forward(hipStream_t st, const MlpDevice& M, const void* X, uint32_t rows, float* Y, uint32_t cus) {
   if (rows == 0) return;
   const uint32_t tiles = (rows + 15) / 16;
@@ -430,30 +478,31 @@ void launch_mlp_forward(hipStream_t st, const MlpDevice& M, const void* X, uint3
   if (blocks > cus) blocks = cus;  // one 8-wave block per CU (LDS), tiles strided over the grid
   hipLaunchKernelGGL(k_mlp_forward, dim3(blocks), dim3(64 * kFwdWaves), 0, st, M, (const bf16*)X, rows, Y);
 }
-void launch_mlp_grad(hipStream_t st, const MlpDevice& M, const MlpTrain& T, const void* X, const float* Tgt,
-                     uint32_t rows, uint32_t cus) {
+void launch_mlp_zero(hipStream_t st, const MlpTrain& T) {
   hipLaunchKernelGGL(k_mlp_zero, dim3(96), dim3(256), 0, st, T);
-  const uint32_t tiles = T.rowsPad / 16;
-  uint32_t blocks = (tiles + 3) / 4;
-  if (blocks > cus) blocks = cus;
+}
+void launch_mlp_backprop(hipStream_t st, const MlpDevice& M, const MlpTrain& T, const void* X, const float* Tgt,
+                         const uint32_t* perm, uint32_t rows, uint32_t cus) {
+  const uint32_t P = T.rowsPad, tiles = P / 16;
   const float scale = 1.0f / ((float)M.nOut * (float)(rows > 0 ? rows : 1));
-  hipLaunchKernelGGL(k_mlp_act_grad, dim3(blocks), dim3(256), 0, st, M, T, (const bf16*)X, Tgt, rows, scale);
-  // split-K: at least 1024 samples per block, about one block per CU and tile group
-  const uint32_t P = T.rowsPad;
+  hipLaunchKernelGGL(k_mlp_act_grad, dim3(std::min(tiles, 2u * cus)), dim3(256), 0, st, M, T, (const bf16*)X, Tgt, perm,
+                     rows, scale);
+  // split-K: at least 256 samples per block, about one block per CU and tile group; 4096 rows take 5.7 us on
+  // 352 workgroups, with eight loads in flight a wave (11 us on 88 of 1024 samples, two at a time)
   uint32_t spb = (P + cus - 1) / cus;
   spb = (spb + 31) / 32 * 32;
-  if (spb < 1024) spb = 1024;
+  if (spb < 256) spb = 256;
   const uint32_t kb = (P + spb - 1) / spb;
   hipLaunchKernelGGL(k_mlp_wgrad, dim3(kb, (kGradTiles + 3) / 4), dim3(256), 0, st, T, spb);
+}
+void launch_mlp_gather_grad(hipStream_t st, const MlpDevice& M, const MlpTrain& T) {
   hipLaunchKernelGGL(k_mlp_gather_grad, dim3(grid_for(M.nParams, 256)), dim3(256), 0, st, T, M.nOut);
 }
-void launch_mlp_accum_loss(hipStream_t st, const float* loss, float* dst, float scale) {
-  hipLaunchKernelGGL(k_mlp_accum_loss, dim3(1), dim3(64), 0, st, loss, dst, scale);
-}
-void launch_mlp_adam(hipStream_t st, const MlpDevice& M, const MlpTrain& T, float lr, int step) {
+void launch_mlp_update(hipStream_t st, const MlpDevice& M, const MlpTrain& T, float lr, int step, float* lossDst,
+                       float lossScale) {
   const float b1c = 1.0f - powf(0.9f, (float)step), b2c = 1.0f - powf(0.999f, (float)step);
-  hipLaunchKernelGGL(k_mlp_adam, dim3(grid_for(M.nParams, 256)), dim3(256), 0, st, M, T, lr, b1c, b2c);
-  launch_mlp_pack(st, M);
+  hipLaunchKernelGGL(k_mlp_update, dim3((M.nParams + 255) / 256), dim3(256), 0, st, M, T, lr, b1c, b2c, lossDst,
+                     lossScale);
 }
 
 }  // namespace avbd

@@ -73,15 +73,18 @@ struct WarmState {
 void launch_mlp_pack(hipStream_t st, const MlpDevice& M);
 void launch_mlp_pack_input(hipStream_t st, const float* Xf, uint32_t n, void* X);
 void launch_mlp_forward(hipStream_t st, const MlpDevice& M, const void* X, uint32_t rows, float* Y, uint32_t cus);
-// zeroes the gradient buffers, then forward + activation gradients + weight
-// gradients of L = sum |y - t|^2 / (nOut rows) into T.grad (master layout) and T.loss
-void launch_mlp_grad(hipStream_t st, const MlpDevice& M, const MlpTrain& T, const void* X, const float* Tgt,
-                     uint32_t rows, uint32_t cus);
-void launch_mlp_adam(hipStream_t st, const MlpDevice& M, const MlpTrain& T, float lr, int step);
-void launch_mlp_accum_loss(hipStream_t st, const float* loss, float* dst, float scale);
-// rows of a dataset gathered by a permutation: X bf16 [n][32], T f32 [n][nOut]
-void launch_mlp_gather_batch(hipStream_t st, const void* Xall, const float* Tall, const uint32_t* perm,
-                             uint32_t n, uint32_t nOut, void* X, float* T);
+// gradient sums and the batch loss to zero
+void launch_mlp_zero(hipStream_t st, const MlpTrain& T);
+// adds the gradients of L = sum |y - t|^2 / (nOut rows) to T's sums and sum
+// |y - t|^2 to T.loss; row r is row perm[r] of X and Tgt (r without perm)
+void launch_mlp_backprop(hipStream_t st, const MlpDevice& M, const MlpTrain& T, const void* X, const float* Tgt,
+                         const uint32_t* perm, uint32_t rows, uint32_t cus);
+// T's sums in the master layout, T.grad
+void launch_mlp_gather_grad(hipStream_t st, const MlpDevice& M, const MlpTrain& T);
+// Adam step number `step` from T's sums, the operand layouts of the new
+// values, lossDst += T.loss lossScale; T's sums and loss are zero afterwards
+void launch_mlp_update(hipStream_t st, const MlpDevice& M, const MlpTrain& T, float lr, int step, float* lossDst,
+                       float lossScale);
 
 // learned stage of a step (learned.hip)
 void launch_ws_features(hipStream_t st, const DeviceState& S, const StepParams& P, const WarmState& W);

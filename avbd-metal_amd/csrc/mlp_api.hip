@@ -210,7 +210,9 @@ extern "C" avbd_status avbd_mlp_loss_grad(avbd_mlp* m, const float* x, const flo
     return AVBD_ERR_HIP;
   MlpTrain T = m->T;
   T.rowsPad = P;
-  launch_mlp_grad(m->stream, m->M, T, m->xb, m->tf, n, m->cus);
+  launch_mlp_zero(m->stream, T);
+  launch_mlp_backprop(m->stream, m->M, T, m->xb, m->tf, nullptr, n, m->cus);
+  launch_mlp_gather_grad(m->stream, m->M, T);
   float l = 0.0f;
   if (hipMemcpyAsync(&l, T.loss, 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
       (grad && hipMemcpyAsync(grad, T.grad, (size_t)m->M.nParams * 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess) ||
@@ -229,8 +231,8 @@ extern "C" avbd_status avbd_mlp_train(avbd_mlp* m, const float* x, const float* 
   if (ensure_train(m, P) != hipSuccess) return AVBD_ERR_ALLOC;
   // the dataset (bf16 rows) and the targets stay resident for the whole run
   std::vector<void*> local;
-  float *xf = nullptr, *tAll = nullptr, *tb = nullptr, *losses = nullptr;
-  __bf16 *xAll = nullptr, *xbat = nullptr;
+  float *xf = nullptr, *tAll = nullptr, *losses = nullptr;
+  __bf16* xAll = nullptr;
   uint32_t* perm = nullptr;
   auto done = [&](avbd_status st) {
     hipStreamSynchronize(m->stream);
@@ -239,9 +241,7 @@ extern "C" avbd_status avbd_mlp_train(avbd_mlp* m, const float* x, const float* 
   };
   const uint32_t no = m->M.nOut;
   if (grab(local, &xf, (size_t)n * kMlpIn) || grab(local, &xAll, (size_t)n * kMlpInPad) ||
-      grab(local, &tAll, (size_t)n * no) || grab(local, &xbat, (size_t)P * kMlpInPad) ||
-      grab(local, &tb, (size_t)P * no) || grab(local, &losses, (size_t)epochs) ||
-      grab(local, &perm, (size_t)epochs * n))
+      grab(local, &tAll, (size_t)n * no) || grab(local, &losses, (size_t)epochs) || grab(local, &perm, (size_t)epochs * n))
     return done(AVBD_ERR_ALLOC);
   // one shuffle per epoch (Fisher-Yates on SplitMix64), uploaded at once
   std::vector<uint32_t> order((size_t)epochs * n);
@@ -261,13 +261,12 @@ extern "C" avbd_status avbd_mlp_train(avbd_mlp* m, const float* x, const float* 
   launch_mlp_pack_input(m->stream, xf, n, xAll);
   MlpTrain T = m->T;
   T.rowsPad = P;
+  launch_mlp_zero(m->stream, T);
   const float meanScale = 1.0f / ((float)no * (float)B * (float)batches);
   for (int32_t e = 0; e < epochs; e++) {
     for (uint32_t k = 0; k < batches; k++) {
-      launch_mlp_gather_batch(m->stream, xAll, tAll, perm + (size_t)e * n + (size_t)k * B, B, no, xbat, tb);
-      launch_mlp_grad(m->stream, m->M, T, xbat, tb, B, m->cus);
-      launch_mlp_accum_loss(m->stream, T.loss, losses + e, meanScale);
-      launch_mlp_adam(m->stream, m->M, T, lr, ++m->adamStep);
+      launch_mlp_backprop(m->stream, m->M, T, xAll, tAll, perm + (size_t)e * n + (size_t)k * B, B, m->cus);
+      launch_mlp_update(m->stream, m->M, T, lr, ++m->adamStep, losses + e, meanScale);
     }
   }
   if (hipGetLastError() != hipSuccess) return done(AVBD_ERR_HIP);
