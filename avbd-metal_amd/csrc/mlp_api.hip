@@ -243,7 +243,15 @@ extern "C" avbd_status avbd_mlp_train(avbd_mlp* m, const float* x, const float* 
   if (grab(local, &xf, (size_t)n * kMlpIn) || grab(local, &xAll, (size_t)n * kMlpInPad) ||
       grab(local, &tAll, (size_t)n * no) || grab(local, &losses, (size_t)epochs) || grab(local, &perm, (size_t)epochs * n))
     return done(AVBD_ERR_ALLOC);
-  // one shuffle per epoch (Fisher-Yates on SplitMix64), uploaded at once
+  if (hipMemcpyAsync(xf, x, (size_t)n * kMlpIn * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
+      hipMemcpyAsync(tAll, t, (size_t)n * no * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess)
+    return done(AVBD_ERR_HIP);
+  launch_mlp_pack_input(m->stream, xf, n, xAll);
+  MlpTrain T = m->T;
+  T.rowsPad = P;
+  launch_mlp_zero(m->stream, T);
+  const float meanScale = 1.0f / ((float)no * (float)B * (float)batches);
+  // one shuffle per epoch (Fisher-Yates on SplitMix64), made while the epoch before it trains
   std::vector<uint32_t> order((size_t)epochs * n);
   uint64_t s = seed;
   for (int32_t e = 0; e < epochs; e++) {
@@ -253,17 +261,8 @@ extern "C" avbd_status avbd_mlp_train(avbd_mlp* m, const float* x, const float* 
       uint32_t j = (uint32_t)(splitmix(s) % (uint64_t)(i + 1));
       std::swap(o[i], o[j]);
     }
-  }
-  if (hipMemcpyAsync(xf, x, (size_t)n * kMlpIn * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
-      hipMemcpyAsync(tAll, t, (size_t)n * no * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
-      hipMemcpyAsync(perm, order.data(), order.size() * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess)
-    return done(AVBD_ERR_HIP);
-  launch_mlp_pack_input(m->stream, xf, n, xAll);
-  MlpTrain T = m->T;
-  T.rowsPad = P;
-  launch_mlp_zero(m->stream, T);
-  const float meanScale = 1.0f / ((float)no * (float)B * (float)batches);
-  for (int32_t e = 0; e < epochs; e++) {
+    if (hipMemcpyAsync(perm + (size_t)e * n, o, (size_t)n * 4, hipMemcpyHostToDevice, m->stream) != hipSuccess)
+      return done(AVBD_ERR_HIP);
     for (uint32_t k = 0; k < batches; k++) {
       launch_mlp_backprop(m->stream, m->M, T, xAll, tAll, perm + (size_t)e * n + (size_t)k * B, B, m->cus);
       launch_mlp_update(m->stream, m->M, T, lr, ++m->adamStep, losses + e, meanScale);
