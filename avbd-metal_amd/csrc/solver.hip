@@ -1881,6 +1881,7 @@ avbd_status build_static_and_upload(avbd_solver* s, const avbd_scene_desc* d) {
   ALLOC(S.colorFlags, 32) ALLOC(S.counters, CTR_TOTAL)
   ALLOC(S.hashedRigid, std::max<size_t>(1, hashedRigid.size()))
   ALLOC(S.clothSlots, cslots.size())
+  S.numClothSlots = (uint32_t)cslots.size();
   ALLOC(s->rateJointDev, std::max<size_t>(1, s->rateJoints.size()))
   ALLOC(s->rateValueDev, std::max<size_t>(1, s->rateValues.size()))
   ALLOC(s->spinBodyDev, std::max<size_t>(1, s->spinBodies.size()))

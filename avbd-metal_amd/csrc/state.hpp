@@ -97,6 +97,7 @@ struct DeviceState {
   F4 *posLinSnap, *posAngSnap;
   // cloth surfaces
   ClothSlot* clothSlots;      // parallel to sAdjList (membrane / bend / particle-spring entries)
+  uint32_t numClothSlots;     // its length: one where no scene entry has a slot
   U4* tris;                   // collision triangles (vertex ids in xyz)
   U2* edges;                  // unique surface edges (ids ascending)
   uint32_t *nbrStart, *nbrCount, *nbrList;  // sorted topological 1-ring of every body
