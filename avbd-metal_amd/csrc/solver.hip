@@ -2265,6 +2265,25 @@ uint32_t island_threads(const avbd_solver* s) {
   return std::min<uint32_t>(kIslandThreads, std::max<uint32_t>(64u, (want + 63u) / 64u * 64u));
 }
 
+// Lanes per body of a surface scene whose colors hold particles only, from the
+// bodies of its largest color.  A rule and no timing: the split orders a
+// particle's sums, so a create that times near-equal splits may give the next
+// one other bits.  Square sheets (two colors of n^2 / 2, 4 frames of 30
+// sweeps, ms):
+//   n    draped 8 / 16 / 32      folded 8 / 16 / 32
+//   20    5.14  5.01  5.09        7.96  6.48  6.03
+//   64    6.08  5.85  5.96       10.14  8.56  7.91
+//   72    6.46  6.27  6.38       10.34  8.75  8.38
+//   128   7.53  7.45  7.89       14.30 13.81 13.66
+//   165   9.31  9.25 10.47       19.73 19.39 19.62
+//   200  11.48 12.17 13.41       26.91 27.48 26.43
+//   256  14.73 15.81 18.06       42.34 39.20 39.47
+// 32 lanes while a color is at most one wave per SIMD (2048 bodies); 16 while
+// it fits the four waves per SIMD the kernel's registers allow, with a small
+// margin; 8 beyond.  Under 300 bodies 16 stays: sheets that small have always
+// run it, and draped it is the faster one.
+int particle_lanes(uint32_t bodies) { return bodies < 300 ? 16 : bodies <= 2048 ? 32 : bodies <= 16000 ? 16 : 8; }
+
 // Times primal sweeps / iterations for each lane split and sweep mode on the
 // initial state, then restores every buffer the trials touched.
 void autotune(avbd_solver* s) {
@@ -2281,6 +2300,8 @@ void autotune(avbd_solver* s) {
   if (s->dynamicColoring && wantMode == 0) modeCands = {2, 1};
   // cloth: the Planar-DAT passes run between the colors' launches
   if (s->datOn || s->isoOn) modeCands = {1};
+  if ((s->datOn || s->isoOn) && s->allMode == kModeParticle && laneCands.size() > 1)
+    laneCands = {particle_lanes(*std::max_element(s->staticColorCounts.begin(), s->staticColorCounts.end()))};
   // persistent grid size per lane count
   auto pblocks = [&](int L) {
     int maxB = persistent_max_blocks(L, s->allMode);
