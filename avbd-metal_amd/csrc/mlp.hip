@@ -160,14 +160,14 @@ __global__ void __launch_bounds__(64 * kFwdWaves) k_mlp_forward(MlpDevice M, con
 // L = sum_r |y_r - t_r|^2 * lossScale over every 16-row tile of the padded
 // batch (rows >= `rows` carry zero gradient; row r is dataset row perm[r], or
 // r without perm); writes the feature-major operands of the weight-gradient
-// GEMMs and adds the bias gradients and sum |y - t|^2 atomically.
+// GEMMs and the workgroup's parts of the bias gradients and of sum |y - t|^2.
 //
 // A workgroup owns a tile and each of its four waves two of the eight column
 // tiles of every layer, so the weights a wave multiplies fit its registers:
 // they are read once, all loads in flight together, straight from the L2.
 // One wave per tile needs every weight, staged through 86 KB of LDS: at 4096
 // rows that filled 64 CUs, was bound by the staging, and took 21 us (15 us
-// now).
+// with the bias sums added atomically, 11 us writing parts).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_mlp_act_grad(MlpDevice M, MlpTrain T, const bf16* X, const float* Tgt,
                                                       const uint32_t* perm, uint32_t rows, float lossScale) {
@@ -278,7 +278,9 @@ __global__ void __launch_bounds__(256) k_mlp_act_grad(MlpDevice M, MlpTrain T, c
     if (tid >= (uint32_t)kHid) store_transposed(h1, kSH, tid - kHid, T.dz1t, P, r0);
     __syncthreads();  // the next tile overwrites h1 / h2 / dz
   }
-  // bias gradients: the four row groups of each column, then one atomic per column and workgroup
+  // bias gradients: the four row groups of each column, then this workgroup's part
+  float* part = T.gb + blockIdx.x;
+  const uint32_t parts = gridDim.x;
 #pragma unroll
   for (int c = 0; c < kN; c++) {
     float a = db1[c], b = db2[c];
@@ -287,26 +289,28 @@ __global__ void __launch_bounds__(256) k_mlp_act_grad(MlpDevice M, MlpTrain T, c
     b += __shfl_xor(b, 16, 64);
     b += __shfl_xor(b, 32, 64);
     if (lane < 16) {
-      atomicAdd(&T.gb1[(kN * wv + c) * 16 + lane], a);
-      atomicAdd(&T.gb2[(kN * wv + c) * 16 + lane], b);
+      const uint32_t col = (kN * wv + c) * 16 + lane;
+      part[col * parts] = a;
+      part[(kHid + col) * parts] = b;
     }
   }
   if (wv != 0u) return;
   db3 += __shfl_xor(db3, 16, 64);
   db3 += __shfl_xor(db3, 32, 64);
-  if (lane < 16) atomicAdd(&T.gb3[lane], db3);
+  if (lane < 16) part[(2 * kHid + lane) * parts] = db3;
   for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o, 64);
-  if (lane == 0) atomicAdd(T.loss, loss);
+  if (lane == 0) part[(kMlpGb - 1u) * parts] = loss;
 }
 
 // ---------------------------------------------------------------------------
 // training, pass 2: weight gradients as split-K GEMMs over the samples,
 //   gW1 = Xt dZ1t^T (32 x 128), gW2 = H1t dZ2t^T (128 x 128), gW3 = H2t dYt^T (128 x 16);
 // 88 output tiles of 16 x 16, one per wave (blockIdx.y: 22 groups of 4),
-// blockIdx.x owns a range of samples (a multiple of 32); partial sums added
-// atomically (f32)
+// blockIdx.x owns a range of samples (a multiple of 32) and writes part
+// blockIdx.x of the sums
 // ---------------------------------------------------------------------------
 constexpr int kGradTiles = 2 * 8 + 8 * 8 + 8;
+constexpr uint32_t kGw2 = kInPad * kHid, kGw3 = kGw2 + kHid * kHid;  // gW2 and gW3 in a part
 __global__ void __launch_bounds__(256) k_mlp_wgrad(MlpTrain T, uint32_t samplesPerBlock) {
   const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63u;
   const uint32_t ar = lane & 15u, ak = 8u * (lane >> 4), dr = 4u * (lane >> 4);
@@ -316,11 +320,11 @@ __global__ void __launch_bounds__(256) k_mlp_wgrad(MlpTrain T, uint32_t samplesP
   const int tile = blockIdx.y * 4 + wv;
   if (tile >= kGradTiles) return;
   const bf16 *At, *Bt;
-  float* G;
+  float* G = T.gw + (size_t)blockIdx.x * kMlpGw;
   uint32_t mt, nt, ldG;
-  if (tile < 16) { At = T.xt; Bt = T.dz1t; G = T.gw1; mt = tile / 8; nt = tile % 8; ldG = kHid; }
-  else if (tile < 80) { int q = tile - 16; At = T.h1t; Bt = T.dz2t; G = T.gw2; mt = q / 8; nt = q % 8; ldG = kHid; }
-  else { int q = tile - 80; At = T.h2t; Bt = T.dyt; G = T.gw3; mt = q; nt = 0; ldG = kOutPad; }
+  if (tile < 16) { At = T.xt; Bt = T.dz1t; mt = tile / 8; nt = tile % 8; ldG = kHid; }
+  else if (tile < 80) { int q = tile - 16; At = T.h1t; Bt = T.dz2t; G += kGw2; mt = q / 8; nt = q % 8; ldG = kHid; }
+  else { int q = tile - 80; At = T.h2t; Bt = T.dyt; G += kGw3; mt = q; nt = 0; ldG = kOutPad; }
   const bf16* ap = At + (size_t)(mt * 16 + ar) * P + ak;
   const bf16* bp = Bt + (size_t)(nt * 16 + ar) * P + ak;
   f32x4 acc = zero4();
@@ -337,71 +341,81 @@ __global__ void __launch_bounds__(256) k_mlp_wgrad(MlpTrain T, uint32_t samplesP
   }
   for (; k < k1; k += 32) acc = mfma(ld8(ap + k), ld8(bp + k), acc);
 #pragma unroll
-  for (int i = 0; i < 4; i++) atomicAdd(&G[(mt * 16 + dr + i) * ldG + nt * 16 + ar], acc[i]);
+  for (int i = 0; i < 4; i++) G[(mt * 16 + dr + i) * ldG + nt * 16 + ar] = acc[i];
 }
 
-// gradients in the master layout from the GEMM outputs (padding dropped)
-__global__ void __launch_bounds__(256) k_mlp_gather_grad(MlpTrain T, uint32_t nOut) {
-  const uint32_t offB3 = (uint32_t)mlp_off_b3((int)nOut), n = (uint32_t)mlp_params((int)nOut);
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    float g;
-    if (i < (uint32_t)kMlpOffB1) g = T.gw1[i];  // rows 0..23 of gw1 [32][128]
-    else if (i < (uint32_t)kMlpOffW2) g = T.gb1[i - kMlpOffB1];
-    else if (i < (uint32_t)kMlpOffB2) g = T.gw2[i - kMlpOffW2];
-    else if (i < (uint32_t)kMlpOffW3) g = T.gb2[i - kMlpOffB2];
-    else if (i < offB3) {
-      uint32_t q = i - kMlpOffW3;
-      g = T.gw3[(q / nOut) * kOutPad + q % nOut];
-    } else {
-      g = T.gb3[i - offB3];
-    }
-    T.grad[i] = g;
-  }
-}
-
-__global__ void __launch_bounds__(256) k_mlp_zero(MlpTrain T) {
-  constexpr uint32_t n1 = kInPad * kHid, n2 = kHid * kHid, n3 = kHid * kOutPad;
-  constexpr uint32_t total = n1 + n2 + n3 + 2 * kHid + kOutPad + 1;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-    if (i < n1) T.gw1[i] = 0.0f;
-    else if (i < n1 + n2) T.gw2[i - n1] = 0.0f;
-    else if (i < n1 + n2 + n3) T.gw3[i - n1 - n2] = 0.0f;
-    else if (i < n1 + n2 + n3 + kHid) T.gb1[i - n1 - n2 - n3] = 0.0f;
-    else if (i < n1 + n2 + n3 + 2 * kHid) T.gb2[i - n1 - n2 - n3 - kHid] = 0.0f;
-    else if (i < total - 1) T.gb3[i - n1 - n2 - n3 - 2 * kHid] = 0.0f;
-    else T.loss[0] = 0.0f;
-  }
-}
-
-// One training step's tail: Adam (beta1 0.9, beta2 0.999, eps 1e-8) on the f32
-// master parameters, the bf16 operand layouts and f32 biases of the updated
-// values, the batch's share of the epoch's mean loss, and zeros where the
-// next batch adds its gradients.  20099 parameters (3 outputs) are nothing
-// but launches: five of 2.3 to 4.2 us each, one of 3.3 us now.
-__global__ void __launch_bounds__(256) k_mlp_update(MlpDevice M, MlpTrain T, float lr, float b1c, float b2c,
-                                                    float* lossDst, float lossScale) {
+// The tail of a gradient: sums the parts of every gradient entry.  UPDATE: one
+// training step's Adam (beta1 0.9, beta2 0.999, eps 1e-8) on the f32 master
+// parameters, the bf16 operand layouts and f32 biases of the updated values,
+// and the batch's share of the epoch's mean loss; otherwise the gradient in the
+// master layout and the loss.
+//
+// The parts are added in the order of their workgroups, so a training run
+// repeats bit for bit: float atomics added them as they arrived, and the
+// thousand steps of an epoch of small batches amplified the last bits of the
+// bias gradients to 6 percent of the parameters.  A thread owns a weight and a
+// wave a bias (of up to kMlpRowParts parts, or the loss).  4096 rows (16 and 256
+// parts) take 3.6 us, as an update of sums added atomically did (3.3 us): 20099
+// parameters are nothing but a launch, and it replaces five of 2.3 to 4.2 us.
+template <bool UPDATE>
+__global__ void __launch_bounds__(256) k_mlp_sum(MlpDevice M, MlpTrain T, uint32_t weightParts, uint32_t rowParts,
+                                                 uint32_t weightBlocks, float lr, float b1c, float b2c, float* lossDst,
+                                                 float lossScale) {
   const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
   const uint32_t nOut = M.nOut, offB3 = (uint32_t)mlp_off_b3((int)nOut);
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0u) {
-    lossDst[0] += T.loss[0] * lossScale;
-    T.loss[0] = 0.0f;
+  uint32_t i;
+  float g = 0.0f, m0 = 0.0f, v0 = 0.0f, p0 = 0.0f;
+  auto fetch = [&]() {  // in flight beside the parts
+    m0 = T.m[i];
+    v0 = T.v[i];
+    p0 = M.params[i];
+  };
+  if (blockIdx.x < weightBlocks) {
+    constexpr uint32_t n1 = kIn * kHid, n2 = kHid * kHid;  // rows 0..23 of gW1 [32][128]
+    const uint32_t w = blockIdx.x * 256u + threadIdx.x;
+    if (w >= n1 + n2 + kHid * nOut) return;
+    uint32_t q;
+    if (w < n1) {
+      i = q = w;
+    } else if (w < n1 + n2) {
+      i = kMlpOffW2 + (w - n1);
+      q = kGw2 + (w - n1);
+    } else {
+      const uint32_t r = w - n1 - n2;
+      i = kMlpOffW3 + r;
+      q = kGw3 + r / nOut * kOutPad + r % nOut;
+    }
+    if (UPDATE) fetch();
+    const float* p = T.gw + q;
+#pragma unroll 8
+    for (uint32_t k = 0; k < weightParts; k++) g += p[(size_t)k * kMlpGw];
+  } else {
+    const uint32_t c = (blockIdx.x - weightBlocks) * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    if (c > 2u * kHid + nOut) return;
+    const bool isLoss = c == 2u * kHid + nOut;
+    i = c < (uint32_t)kHid ? kMlpOffB1 + c : c < 2u * kHid ? kMlpOffB2 + (c - kHid) : offB3 + (c - 2u * kHid);
+    if (UPDATE && !isLoss) fetch();
+    const float* p = T.gb + (size_t)(isLoss ? kMlpGb - 1u : c) * rowParts;
+#pragma unroll
+    for (uint32_t k = 0; k < kMlpRowParts / 64u; k++)
+      if (lane + 64u * k < rowParts) g += p[lane + 64u * k];
+    for (int o = 32; o > 0; o >>= 1) g += __shfl_xor(g, o, 64);
+    if (lane != 0u) return;
+    if (isLoss) {
+      if (UPDATE) lossDst[0] += g * lossScale;
+      else T.loss[0] = g;
+      return;
+    }
   }
-  if (i >= M.nParams) return;
-  float* gp;
-  if (i < (uint32_t)kMlpOffB1) gp = &T.gw1[i];  // rows 0..23 of gw1 [32][128]
-  else if (i < (uint32_t)kMlpOffW2) gp = &T.gb1[i - kMlpOffB1];
-  else if (i < (uint32_t)kMlpOffB2) gp = &T.gw2[i - kMlpOffW2];
-  else if (i < (uint32_t)kMlpOffW3) gp = &T.gb2[i - kMlpOffB2];
-  else if (i < offB3) gp = &T.gw3[((i - kMlpOffW3) / nOut) * kOutPad + (i - kMlpOffW3) % nOut];
-  else gp = &T.gb3[i - offB3];
-  const float g = *gp;
-  *gp = 0.0f;
-  const float m = beta1 * T.m[i] + (1.0f - beta1) * g;
-  const float v = beta2 * T.v[i] + (1.0f - beta2) * g * g;
+  if (!UPDATE) {
+    T.grad[i] = g;
+    return;
+  }
+  const float m = beta1 * m0 + (1.0f - beta1) * g;
+  const float v = beta2 * v0 + (1.0f - beta2) * g * g;
   T.m[i] = m;
   T.v[i] = v;
-  const float p = M.params[i] - lr * (m / b1c) / (sqrtf(v / b2c) + eps);
+  const float p = p0 - lr * (m / b1c) / (sqrtf(v / b2c) + eps);
   M.params[i] = p;
   // the padding of the operand layouts is zero since k_mlp_pack
   if (i < (uint32_t)kMlpOffB1) {
@@ -478,31 +492,43 @@ void launch_mlp_forward(hipStream_t st, const MlpDevice& M, const void* X, uint3
   if (blocks > cus) blocks = cus;  // one 8-wave block per CU (LDS), tiles strided over the grid
   hipLaunchKernelGGL(k_mlp_forward, dim3(blocks), dim3(64 * kFwdWaves), 0, st, M, (const bf16*)X, rows, Y);
 }
-void launch_mlp_zero(hipStream_t st, const MlpTrain& T) {
-  hipLaunchKernelGGL(k_mlp_zero, dim3(96), dim3(256), 0, st, T);
+// parts of a batch: of its bias sums (workgroups of k_mlp_act_grad) and of its
+// weight sums (ranges of samplesPerBlock).  4096 rows: the weight gradients take
+// 6 us on 352 workgroups of 256 rows with eight loads in flight a wave (11 us
+// on 88 of 1024 rows, two at a time)
+static uint32_t row_parts(uint32_t rowsPad, uint32_t cus) {
+  return std::min(rowsPad / 16u, std::min(2u * cus, kMlpRowParts));
+}
+static uint32_t weight_rows(uint32_t rowsPad) {
+  const uint32_t spb = (rowsPad + kMlpWeightParts - 1) / kMlpWeightParts;
+  return std::max(256u, (spb + 31u) / 32u * 32u);
+}
+static uint32_t weight_parts(uint32_t rowsPad) {
+  return (rowsPad + weight_rows(rowsPad) - 1) / weight_rows(rowsPad);
 }
 void launch_mlp_backprop(hipStream_t st, const MlpDevice& M, const MlpTrain& T, const void* X, const float* Tgt,
                          const uint32_t* perm, uint32_t rows, uint32_t cus) {
-  const uint32_t P = T.rowsPad, tiles = P / 16;
   const float scale = 1.0f / ((float)M.nOut * (float)(rows > 0 ? rows : 1));
-  hipLaunchKernelGGL(k_mlp_act_grad, dim3(std::min(tiles, 2u * cus)), dim3(256), 0, st, M, T, (const bf16*)X, Tgt, perm,
+  hipLaunchKernelGGL(k_mlp_act_grad, dim3(row_parts(T.rowsPad, cus)), dim3(256), 0, st, M, T, (const bf16*)X, Tgt, perm,
                      rows, scale);
-  // split-K: at least 256 samples per block, about one block per CU and tile group; 4096 rows take 5.7 us on
-  // 352 workgroups, with eight loads in flight a wave (11 us on 88 of 1024 samples, two at a time)
-  uint32_t spb = (P + cus - 1) / cus;
-  spb = (spb + 31) / 32 * 32;
-  if (spb < 256) spb = 256;
-  const uint32_t kb = (P + spb - 1) / spb;
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3(kb, (kGradTiles + 3) / 4), dim3(256), 0, st, T, spb);
+  hipLaunchKernelGGL(k_mlp_wgrad, dim3(weight_parts(T.rowsPad), (kGradTiles + 3) / 4), dim3(256), 0, st, T,
+                     weight_rows(T.rowsPad));
 }
-void launch_mlp_gather_grad(hipStream_t st, const MlpDevice& M, const MlpTrain& T) {
-  hipLaunchKernelGGL(k_mlp_gather_grad, dim3(grid_for(M.nParams, 256)), dim3(256), 0, st, T, M.nOut);
+template <bool UPDATE>
+static void launch_sum(hipStream_t st, const MlpDevice& M, const MlpTrain& T, uint32_t cus, float lr, float b1c,
+                       float b2c, float* lossDst, float lossScale) {
+  const uint32_t weights = (kIn + kHid + M.nOut) * kHid, wb = (weights + 255) / 256;
+  const uint32_t waves = 2 * kHid + M.nOut + 1;
+  hipLaunchKernelGGL((k_mlp_sum<UPDATE>), dim3(wb + (waves + 3) / 4), dim3(256), 0, st, M, T, weight_parts(T.rowsPad),
+                     row_parts(T.rowsPad, cus), wb, lr, b1c, b2c, lossDst, lossScale);
 }
-void launch_mlp_update(hipStream_t st, const MlpDevice& M, const MlpTrain& T, float lr, int step, float* lossDst,
-                       float lossScale) {
+void launch_mlp_gather_grad(hipStream_t st, const MlpDevice& M, const MlpTrain& T, uint32_t cus) {
+  launch_sum<false>(st, M, T, cus, 0.0f, 1.0f, 1.0f, nullptr, 0.0f);
+}
+void launch_mlp_update(hipStream_t st, const MlpDevice& M, const MlpTrain& T, uint32_t cus, float lr, int step,
+                       float* lossDst, float lossScale) {
   const float b1c = 1.0f - powf(0.9f, (float)step), b2c = 1.0f - powf(0.999f, (float)step);
-  hipLaunchKernelGGL(k_mlp_update, dim3((M.nParams + 255) / 256), dim3(256), 0, st, M, T, lr, b1c, b2c, lossDst,
-                     lossScale);
+  launch_sum<true>(st, M, T, cus, lr, b1c, b2c, lossDst, lossScale);
 }
 
 }  // namespace avbd

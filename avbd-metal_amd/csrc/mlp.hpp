@@ -30,13 +30,24 @@ struct MlpDevice {
 };
 
 // Training buffers for batches of at most rowsPad rows (a multiple of 32):
-// feature-major activations and gradients, GEMM outputs, Adam moments.
+// feature-major activations and gradients, the workgroups' parts of the
+// gradient sums, Adam moments.
 struct MlpTrain {
   __bf16 *xt, *h1t, *h2t, *dz1t, *dz2t, *dyt;
-  float *gw1, *gw2, *gw3, *gb1, *gb2, *gb3, *loss;
+  float* gw;    // [weight part][kMlpGw]: gW1 [32][128], gW2 [128][128], gW3 [128][16]
+  float* gb;    // [kMlpGb][row part]: gb1, gb2, gb3 (padded to 16), sum |y - t|^2
+  float* loss;  // sum |y - t|^2 of a gradient call
   float *grad, *m, *v;
   uint32_t rowsPad;
 };
+constexpr uint32_t kMlpGw = kMlpInPad * kMlpHidden + kMlpHidden * kMlpHidden + kMlpHidden * kMlpOutPad;
+constexpr uint32_t kMlpGb = 2 * kMlpHidden + kMlpOutPad + 1;
+// most parts of a batch: of the weight sums (ranges of at least 256 rows) and of the bias sums
+constexpr uint32_t kMlpWeightParts = 64, kMlpRowParts = 512;
+inline uint32_t mlp_weight_parts_cap(uint32_t rowsPad) {
+  const uint32_t n = (rowsPad + 255u) / 256u;
+  return n < kMlpWeightParts ? n : kMlpWeightParts;
+}
 
 // The learned stage inside a step: dynamic particles (and rigid bodies) in
 // list order, their 1-ring (body ids; joint partners for rigid bodies), this
@@ -73,18 +84,16 @@ struct WarmState {
 void launch_mlp_pack(hipStream_t st, const MlpDevice& M);
 void launch_mlp_pack_input(hipStream_t st, const float* Xf, uint32_t n, void* X);
 void launch_mlp_forward(hipStream_t st, const MlpDevice& M, const void* X, uint32_t rows, float* Y, uint32_t cus);
-// gradient sums and the batch loss to zero
-void launch_mlp_zero(hipStream_t st, const MlpTrain& T);
-// adds the gradients of L = sum |y - t|^2 / (nOut rows) to T's sums and sum
-// |y - t|^2 to T.loss; row r is row perm[r] of X and Tgt (r without perm)
+// the parts of the gradients of L = sum |y - t|^2 / (nOut rows) and of sum
+// |y - t|^2; row r is row perm[r] of X and Tgt (r without perm)
 void launch_mlp_backprop(hipStream_t st, const MlpDevice& M, const MlpTrain& T, const void* X, const float* Tgt,
                          const uint32_t* perm, uint32_t rows, uint32_t cus);
-// T's sums in the master layout, T.grad
-void launch_mlp_gather_grad(hipStream_t st, const MlpDevice& M, const MlpTrain& T);
-// Adam step number `step` from T's sums, the operand layouts of the new
-// values, lossDst += T.loss lossScale; T's sums and loss are zero afterwards
-void launch_mlp_update(hipStream_t st, const MlpDevice& M, const MlpTrain& T, float lr, int step, float* lossDst,
-                       float lossScale);
+// the sums of T's parts, in the master layout in T.grad and in T.loss
+void launch_mlp_gather_grad(hipStream_t st, const MlpDevice& M, const MlpTrain& T, uint32_t cus);
+// Adam step number `step` from the sums of T's parts, the operand layouts of
+// the new values, lossDst += sum |y - t|^2 lossScale
+void launch_mlp_update(hipStream_t st, const MlpDevice& M, const MlpTrain& T, uint32_t cus, float lr, int step,
+                       float* lossDst, float lossScale);
 
 // learned stage of a step (learned.hip)
 void launch_ws_features(hipStream_t st, const DeviceState& S, const StepParams& P, const WarmState& W);

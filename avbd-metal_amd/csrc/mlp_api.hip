@@ -58,9 +58,8 @@ hipError_t ensure_train(avbd_mlp* m, uint32_t rowsPad) {
   if ((e = grab(L, &T.xt, kMlpInPad * P)) || (e = grab(L, &T.h1t, kMlpHidden * P)) ||
       (e = grab(L, &T.h2t, kMlpHidden * P)) || (e = grab(L, &T.dz1t, kMlpHidden * P)) ||
       (e = grab(L, &T.dz2t, kMlpHidden * P)) || (e = grab(L, &T.dyt, kMlpOutPad * P)) ||
-      (e = grab(L, &T.gw1, kMlpInPad * kMlpHidden)) || (e = grab(L, &T.gw2, kMlpHidden * kMlpHidden)) ||
-      (e = grab(L, &T.gw3, kMlpHidden * kMlpOutPad)) || (e = grab(L, &T.gb1, kMlpHidden)) ||
-      (e = grab(L, &T.gb2, kMlpHidden)) || (e = grab(L, &T.gb3, kMlpOutPad)) || (e = grab(L, &T.loss, 4)))
+      (e = grab(L, &T.gw, (size_t)mlp_weight_parts_cap(rowsPad) * kMlpGw)) ||
+      (e = grab(L, &T.gb, (size_t)kMlpGb * kMlpRowParts)) || (e = grab(L, &T.loss, 4)))
     return e;
   T.rowsPad = rowsPad;
   m->T = T;
@@ -210,9 +209,8 @@ extern "C" avbd_status avbd_mlp_loss_grad(avbd_mlp* m, const float* x, const flo
     return AVBD_ERR_HIP;
   MlpTrain T = m->T;
   T.rowsPad = P;
-  launch_mlp_zero(m->stream, T);
   launch_mlp_backprop(m->stream, m->M, T, m->xb, m->tf, nullptr, n, m->cus);
-  launch_mlp_gather_grad(m->stream, m->M, T);
+  launch_mlp_gather_grad(m->stream, m->M, T, m->cus);
   float l = 0.0f;
   if (hipMemcpyAsync(&l, T.loss, 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
       (grad && hipMemcpyAsync(grad, T.grad, (size_t)m->M.nParams * 4, hipMemcpyDeviceToHost, m->stream) != hipSuccess) ||
@@ -249,7 +247,6 @@ extern "C" avbd_status avbd_mlp_train(avbd_mlp* m, const float* x, const float* 
   launch_mlp_pack_input(m->stream, xf, n, xAll);
   MlpTrain T = m->T;
   T.rowsPad = P;
-  launch_mlp_zero(m->stream, T);
   const float meanScale = 1.0f / ((float)no * (float)B * (float)batches);
   // one shuffle per epoch (Fisher-Yates on SplitMix64), made while the epoch before it trains
   std::vector<uint32_t> order((size_t)epochs * n);
@@ -265,7 +262,7 @@ extern "C" avbd_status avbd_mlp_train(avbd_mlp* m, const float* x, const float* 
       return done(AVBD_ERR_HIP);
     for (uint32_t k = 0; k < batches; k++) {
       launch_mlp_backprop(m->stream, m->M, T, xAll, tAll, perm + (size_t)e * n + (size_t)k * B, B, m->cus);
-      launch_mlp_update(m->stream, m->M, T, lr, ++m->adamStep, losses + e, meanScale);
+      launch_mlp_update(m->stream, m->M, T, m->cus, lr, ++m->adamStep, losses + e, meanScale);
     }
   }
   if (hipGetLastError() != hipSuccess) return done(AVBD_ERR_HIP);

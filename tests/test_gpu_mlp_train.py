@@ -68,3 +68,23 @@ def test_training_steps(outputs, n, batch):
     y = net.forward(x[:100])
     net.params = net.params
     assert np.array_equal(y, net.forward(x[:100]))
+
+
+@pytest.mark.parametrize("outputs,n,batch", [(3, 50, 97), (6, 20000, 97), (3, 9000, 512), (3, 12000, 4096),
+                                             (3, 20000, 17000)])
+def test_training_repeats_bit_for_bit(outputs, n, batch):
+    """Sums over workgroups in a fixed order: one and several parts of the
+    weight and of the bias sums, more row tiles than parts."""
+    flush_print(f"[gpu case] repeated MLP training, {outputs} outputs, {n} rows, batches of {batch}")
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, 24)).astype(np.float32)
+    t = rng.standard_normal((n, outputs)).astype(np.float32)
+    runs = []
+    for _ in range(3):
+        net = WarmStartMLP(seed=4, outputs=outputs)
+        loss = net.train(x, t, epochs=2, batch=batch, lr=1e-3, seed=9)
+        l, g = net.lossGrad(x[:5000], t[:5000])
+        runs.append((net.params, loss, l, g))
+    for r in runs[1:]:
+        for a, b in zip(r, runs[0]):
+            assert np.array_equal(a, b)
