@@ -9,7 +9,6 @@
 #include <string.h>
 #include <stdio.h>
 #include <algorithm>
-#include <atomic>
 #include <array>
 #include <functional>
 #include <map>
@@ -24,6 +23,7 @@
 #include "../../include/avbd.h"
 #include "kernels.hpp"
 #include "lifetime.hpp"
+#include "turns.hpp"
 #include "mlp.hpp"
 
 // upload-time geometry must round exactly as written (radii feed the
@@ -130,11 +130,8 @@ struct avbd_solver {
   bool graphsValid[2] = {false, false};
   bool graphsDisabled = false;
   int64_t graphBaseFrame[2] = {1, 1};  // frame that replays the pair's first graph
-  // kernels that wait for their other workgroups (tiles, grid barriers)
-  bool waits = false;          // this solver's frames may hold such kernels
+  Turn turn;                   // announces frames with kernels that wait (tiles, grid barriers)
   bool cooperative = true;     // how the next frame launches its tile kernel
-  std::atomic<bool> frameOpen{false};          // a frame is being submitted (or iterated to a residual)
-  std::atomic<bool> waitBusy[2] = {false, false};  // per frame slot: submitted and not retired
   // failure latch
   avbd_failure failure{};
   bool failed = false;
@@ -483,63 +480,37 @@ hipError_t build_graphs(avbd_solver* s) {
 
 avbd_status sync_all(avbd_solver* s);
 
-// Kernels that wait for their other workgroups need all of them resident.
-// Cooperative launches are kept apart by the runtime; an ordinary launch of
-// the tile kernel is only safe beside kernels that end by themselves (or one
-// tile kernel more: two of its workgroups fit a CU).  So each solver whose
-// frames hold such kernels announces them here, per process, and a tile frame
-// is launched the ordinary way only while no other solver's is in flight;
-// other waiting kernels hold back until an ordinary tile frame has ended.
-struct WaitingSolvers {
-  std::mutex m;
-  std::vector<avbd_solver*> list;
-};
-WaitingSolvers& waiting_solvers() {
-  static WaitingSolvers* w = new WaitingSolvers();  // outlives every handle
-  return *w;
+Turns& turns() {
+  static Turns* t = new Turns();  // outlives every handle
+  return *t;
 }
-void leave_waiting(avbd_solver* s) {
-  WaitingSolvers& w = waiting_solvers();
-  std::lock_guard<std::mutex> lock(w.m);
-  w.list.erase(std::remove(w.list.begin(), w.list.end(), s), w.list.end());
+// What the kernels of the solver's frames ask of the device.
+Launch frame_launch(const avbd_solver* s) {
+  if (s->numTiles) return Launch::Tiles;
+  const bool grid = (s->dynamicColoring && !s->numIslands) || (s->sweepMode == 2 && !s->islandSolve);
+  return grid ? Launch::Apart : Launch::Ends;
 }
-bool frame_in_flight(avbd_solver* o) {
-  if (o->frameOpen) return true;
-  for (int k = 0; k < 2; k++)
-    if (o->waitBusy[k]) {
-      const hipError_t e = hipEventQuery(o->frameDone[k]);
-      if (e == hipErrorNotReady) {
-        (void)hipGetLastError();
-        return true;
-      }
-    }
-  return false;
-}
-// held from the choice of the launch to the record of the frame's event
+// a frame's announcement, from the choice of its launch to submitted()
 struct FrameTurn {
   avbd_solver* s;
-  explicit FrameTurn(avbd_solver* solver) : s(solver) {
-    if (!s->waits) return;
-    WaitingSolvers& w = waiting_solvers();
-    for (;;) {
-      bool others = false, tile = false;
-      {
-        std::lock_guard<std::mutex> lock(w.m);
-        for (avbd_solver* o : w.list)
-          if (o != s && o->device == s->device && frame_in_flight(o)) {
-            others = true;
-            tile |= o->numTiles && !o->cooperative;
-          }
-        if (s->numTiles || !tile) {
-          s->cooperative = others || !s->numTiles;
-          s->frameOpen = true;
-          return;
-        }
-      }
-      std::this_thread::yield();
-    }
+  Launch launch = Launch::Ends;
+  bool open = false;
+  FrameTurn(avbd_solver* solver, Launch want) : s(solver) {
+    if (want == Launch::Ends) return;
+    while (!turns().begin(&s->turn, want, &launch)) std::this_thread::yield();
+    open = true;
+    s->cooperative = launch != Launch::Tiles;
   }
-  ~FrameTurn() { s->frameOpen = false; }
+  // the frame's completion is recorded in frameDone[slot]
+  void submitted(int slot) {
+    if (open) turns().end(&s->turn, slot);
+    open = false;
+  }
+  ~FrameTurn() {
+    if (!open) return;
+    hipStreamSynchronize(s->stream);  // trials and error paths leave kernels that no event covers
+    turns().end(&s->turn, -1);
+  }
   FrameTurn(const FrameTurn&) = delete;
   FrameTurn& operator=(const FrameTurn&) = delete;
 };
@@ -566,9 +537,8 @@ constexpr uint32_t kTileFill = 8;
 avbd_status retire_slot(avbd_solver* s, int slot) {
   if (!s->slotBusy[slot]) return AVBD_OK;
   s->slotBusy[slot] = false;
-  s->waitBusy[slot] = false;
   int64_t frame = s->slotFrame[slot];
-  hipError_t e = hipEventSynchronize(s->frameDone[slot]);
+  hipError_t e = turns().retire(&s->turn, slot, [&] { return hipEventSynchronize(s->frameDone[slot]); });
   if (e != hipSuccess) {
     char m[160];
     snprintf(m, sizeof(m), "frame %lld did not complete: %s", (long long)frame, hipGetErrorString(e));
@@ -1235,17 +1205,17 @@ extern "C" avbd_status avbd_create(const avbd_scene_desc* d, const avbd_options*
     *out = nullptr;
     return st;
   }
-  s->waits = true;  // the trials may launch grid-wide sweeps
-  {
-    std::lock_guard<std::mutex> lock(waiting_solvers().m);
-    waiting_solvers().list.push_back(s);
-  }
+  s->turn.device = s->device;
+  s->turn.done = [s](int slot) {
+    const hipError_t e = hipEventQuery(s->frameDone[slot]);
+    if (e == hipErrorNotReady) (void)hipGetLastError();
+    return e != hipErrorNotReady;
+  };
+  turns().join(&s->turn);
   autotune(s);
   create_phase(s, "autotune");
   s->stats.lanes_per_body = s->lanes;
-  s->waits = s->numTiles || (s->dynamicColoring && !s->numIslands) || (s->sweepMode == 2 && !s->islandSolve);
-  s->cooperative = !s->numTiles;
-  if (!s->waits) leave_waiting(s);
+  if (frame_launch(s) == Launch::Ends) turns().leave(&s->turn);
   s->stats.sweep_mode = s->numTiles ? 2 : s->sweepMode;
   s->stats.uses_dynamic_coloring = s->dynamicColoring ? 1 : 0;
   return AVBD_OK;
@@ -1261,7 +1231,7 @@ namespace {
 void release_solver(avbd_solver* s) {
   if (!s) return;
   if (s->stream) hipStreamSynchronize(s->stream);
-  leave_waiting(s);
+  turns().leave(&s->turn);
   invalidate_graphs(s);
   for (void* p : s->allocs) hipFree(p);
   for (int i = 0; i < 2; i++)
@@ -2334,7 +2304,7 @@ void autotune(avbd_solver* s) {
     if (s->sweepMode == 2 && s->persistentBlocks <= 0) s->sweepMode = 1;
     return;
   }
-  FrameTurn turn(s);
+  FrameTurn turn(s, Launch::Apart);  // the trials may launch grid-wide sweeps
   // backup
   std::vector<std::pair<void*, size_t>> bufs = {
       {S.posLin, nb * 16}, {S.posLo, nb * 16}, {S.posAng, nb * 16}, {S.initLin, nb * 16}, {S.initAng, nb * 16},
@@ -2449,7 +2419,7 @@ extern "C" avbd_status avbd_submit_step(avbd_solver* s) {
   }
   choose_tile_path(s, slot);
   bool useGraph = s->opts.use_graph && !s->graphsDisabled && !s->profiling;
-  FrameTurn turn(s);
+  FrameTurn turn(s, frame_launch(s));
   if (useGraph && !s->graphsValid[s->cooperative]) {
     hipError_t e = build_graphs(s);
     if (e != hipSuccess) {
@@ -2493,7 +2463,7 @@ extern "C" avbd_status avbd_submit_step(avbd_solver* s) {
                frame);
   HIP_OR_LATCH(s, hipEventRecord(s->frameDone[slot], s->stream), frame);
   s->slotBusy[slot] = true;
-  s->waitBusy[slot] = s->waits;
+  turn.submitted(slot);
   s->slotFrame[slot] = frame;
   s->frameIndex = frame;
   return AVBD_OK;
@@ -2575,7 +2545,7 @@ extern "C" avbd_status avbd_step_to_residual(avbd_solver* s, float tol, int32_t 
   hipStream_t st = s->stream;
   choose_tile_path(s, slot);
   bool useGraph = s->opts.use_graph && !s->graphsDisabled && !s->profiling;
-  FrameTurn turn(s);
+  FrameTurn turn(s, frame_launch(s));
   if (useGraph && !(s->resValid && s->resCheck == check_every && s->resMax == max_iterations && s->resTol == tol)) {
     if (build_residual_graphs(s, tol, max_iterations, check_every) != hipSuccess) {
       (void)hipGetLastError();
@@ -2636,7 +2606,7 @@ extern "C" avbd_status avbd_step_to_residual(avbd_solver* s, float tol, int32_t 
                frame);
   HIP_OR_LATCH(s, hipEventRecord(s->frameDone[slot], st), frame);
   s->slotBusy[slot] = true;
-  s->waitBusy[slot] = s->waits;
+  turn.submitted(slot);
   s->slotFrame[slot] = frame;
   s->frameIndex = frame;
   avbd_status out = sync_all(s);

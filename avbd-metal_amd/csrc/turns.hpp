@@ -1,0 +1,88 @@
+// turns.hpp -- which solvers' frames may be on a device together.
+//
+// Kernels whose workgroups wait for each other (the tile kernel, the grid-wide
+// sweeps and the cooperative color repair) need all of them resident.
+// Cooperative launches of one process are kept apart by the runtime, but one
+// costs 36 to 110 us of gaps, so the tile kernel is launched the ordinary way
+// where that is safe: beside kernels that end by themselves, and beside one
+// tile kernel more (two of its workgroups fit a CU).  Every solver whose frames
+// hold such kernels has an entry here, and a frame stays announced from the
+// choice of its launch until its completion has been seen:
+//   - a tile frame is ordinary while no other solver's waiting frame is
+//     announced, cooperative otherwise;
+//   - a frame of grid-wide kernels is not begun while another solver's
+//     ordinary tile frame is announced.
+//
+// No HIP calls: an entry brings its own completion query.
+#pragma once
+#include <algorithm>
+#include <functional>
+#include <mutex>
+#include <vector>
+
+namespace avbd {
+
+enum class Launch : unsigned char {
+  Ends,   // every kernel of the frame ends by itself
+  Apart,  // kernels that wait, launched cooperatively
+  Tiles,  // the tile kernel, launched the ordinary way
+};
+
+// One solver's entry.  All but `device` and `done` belongs to Turns.
+struct Turn {
+  int device = 0;
+  std::function<bool(int slot)> done;  // has the frame submitted in this slot completed?
+  Launch open = Launch::Ends;          // the frame being submitted (or iterated to a residual)
+  Launch slot[2] = {Launch::Ends, Launch::Ends};  // frames submitted and not seen to complete
+};
+
+class Turns {
+ public:
+  void join(Turn* t) {
+    std::lock_guard<std::mutex> g(m_);
+    list_.push_back(t);
+  }
+  void leave(Turn* t) {
+    std::lock_guard<std::mutex> g(m_);
+    list_.erase(std::remove(list_.begin(), list_.end(), t), list_.end());
+  }
+  // Announces t's next frame, which holds `want`; *got is how to launch it.
+  // False: not now, nothing announced.
+  bool begin(Turn* t, Launch want, Launch* got) {
+    std::lock_guard<std::mutex> g(m_);
+    bool others = false, tiles = false;
+    for (Turn* o : list_) {
+      if (o == t || o->device != t->device) continue;
+      // not while it submits: it may be capturing, which a query of its events would end
+      for (int k = 0; k < 2 && o->open == Launch::Ends; k++)
+        if (o->slot[k] != Launch::Ends && o->done(k)) o->slot[k] = Launch::Ends;
+      for (Launch l : {o->open, o->slot[0], o->slot[1]}) {
+        others |= l != Launch::Ends;
+        tiles |= l == Launch::Tiles;
+      }
+    }
+    if (want == Launch::Apart && tiles) return false;
+    *got = t->open = want == Launch::Tiles && others ? Launch::Apart : want;
+    return true;
+  }
+  // The frame is submitted in `slot`, its completion recorded there; slot < 0: it left nothing on the device.
+  void end(Turn* t, int slot) {
+    std::lock_guard<std::mutex> g(m_);
+    if (slot >= 0) t->slot[slot] = t->open;
+    t->open = Launch::Ends;
+  }
+  // Waits for the slot's frame (`wait`), which stays announced meanwhile.
+  template <typename Wait>
+  auto retire(Turn* t, int slot, Wait&& wait) -> decltype(wait()) {
+    const auto r = wait();
+    std::lock_guard<std::mutex> g(m_);
+    t->slot[slot] = Launch::Ends;
+    return r;
+  }
+
+ private:
+  std::mutex m_;
+  std::vector<Turn*> list_;
+};
+
+}  // namespace avbd
