@@ -131,7 +131,6 @@ struct avbd_solver {
   bool graphsDisabled = false;
   int64_t graphBaseFrame[2] = {1, 1};  // frame that replays the pair's first graph
   Turn turn;                   // announces frames with kernels that wait (tiles, grid barriers)
-  bool cooperative = true;     // how the next frame launches its tile kernel
   // failure latch
   avbd_failure failure{};
   bool failed = false;
@@ -363,15 +362,17 @@ void enqueue_pre_solve(avbd_solver* s, const DeviceState& S, const StepParams& P
 }
 
 // `iterations` sweeps (every color, then the dual); the persistent mode runs
-// them in one cooperative launch whose barrier counter starts at zero
+// them in one cooperative launch whose barrier counter starts at zero;
+// `launch`: what the frame announced
 hipError_t enqueue_iterations(avbd_solver* s, const DeviceState& S, const StepParams& P0, uint32_t iterations,
-                              bool clearBarrier) {
+                              bool clearBarrier, Launch launch) {
   hipStream_t st = s->stream;
   StepParams P = P0;
   P.iterations = iterations;
   if (iterations == 0) return hipSuccess;
   if (s->numTiles && s->tileHold == 0) {
-    return launch_tile_solve(st, S, P, s->numTiles, s->staticUsedColors, s->tileThreads, s->cooperative);
+    return launch_tile_solve(st, S, P, s->numTiles, s->staticUsedColors, s->tileThreads,
+                             launch != Launch::Tiles);
   }
   if (s->islandSolve) {
     launch_island_solve(st, S, P, s->numIslands, s->lanes, s->islandThreads);
@@ -414,13 +415,13 @@ void enqueue_post_solve(avbd_solver* s, const DeviceState& S, const StepParams& 
 }
 
 // Enqueue one frame's kernels on the stream (eagerly or under capture).
-hipError_t enqueue_frame(avbd_solver* s, const DeviceState& S, const StageFn& mark = nullptr) {
+hipError_t enqueue_frame(avbd_solver* s, const DeviceState& S, Launch launch, const StageFn& mark = nullptr) {
   auto stage = [&](const char* name) {
     if (mark) mark(name);
   };
   StepParams P = make_params(s);
   enqueue_pre_solve(s, S, P, stage);
-  hipError_t e = enqueue_iterations(s, S, P, P.iterations, false);
+  hipError_t e = enqueue_iterations(s, S, P, P.iterations, false, launch);
   if (e != hipSuccess) return e;
   stage("solve");
   enqueue_post_solve(s, S, P, stage);
@@ -456,14 +457,17 @@ hipError_t capture_graph(avbd_solver* s, const std::function<hipError_t()>& body
   return e;
 }
 
-hipError_t build_graphs(avbd_solver* s) {
-  const int v = s->cooperative ? 1 : 0;
+// which of the captured forms a frame replays: the tile kernel launched the ordinary way, or any other
+int graph_form(Launch launch) { return launch == Launch::Tiles ? 0 : 1; }
+
+hipError_t build_graphs(avbd_solver* s, Launch launch) {
+  const int v = graph_form(launch);
   DeviceState S = s->S;
   for (int p = 0; p < 2; p++) {
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return e;
-    hipError_t eq = enqueue_frame(s, S);
+    hipError_t eq = enqueue_frame(s, S, launch);
     e = hipStreamEndCapture(s->stream, &g);
     if (eq != hipSuccess) { if (g) hipGraphDestroy(g); return eq; }
     if (e != hipSuccess) return e;
@@ -499,7 +503,6 @@ struct FrameTurn {
     if (want == Launch::Ends) return;
     while (!turns().begin(&s->turn, want, &launch)) std::this_thread::yield();
     open = true;
-    s->cooperative = launch != Launch::Tiles;
   }
   // the frame's completion is recorded in frameDone[slot]
   void submitted(int slot) {
@@ -2420,8 +2423,9 @@ extern "C" avbd_status avbd_submit_step(avbd_solver* s) {
   choose_tile_path(s, slot);
   bool useGraph = s->opts.use_graph && !s->graphsDisabled && !s->profiling;
   FrameTurn turn(s, frame_launch(s));
-  if (useGraph && !s->graphsValid[s->cooperative]) {
-    hipError_t e = build_graphs(s);
+  const int form = graph_form(turn.launch);
+  if (useGraph && !s->graphsValid[form]) {
+    hipError_t e = build_graphs(s, turn.launch);
     if (e != hipSuccess) {
       hipGetLastError();
       invalidate_graphs(s);
@@ -2431,8 +2435,7 @@ extern "C" avbd_status avbd_submit_step(avbd_solver* s) {
   }
   if (useGraph) {
     // the pair's first graph was captured with the buffer roles of frame graphBaseFrame
-    const int v = s->cooperative ? 1 : 0;
-    HIP_OR_LATCH(s, hipGraphLaunch(s->graphs[v][(frame - s->graphBaseFrame[v]) & 1], s->stream), frame);
+    HIP_OR_LATCH(s, hipGraphLaunch(s->graphs[form][(frame - s->graphBaseFrame[form]) & 1], s->stream), frame);
   } else if (s->profiling) {
     // eager, with per-stage events
     hipStream_t st = s->stream;
@@ -2446,14 +2449,14 @@ extern "C" avbd_status avbd_submit_step(avbd_solver* s) {
       if (name) names.push_back(name);
     };
     mark(nullptr);
-    HIP_OR_LATCH(s, enqueue_frame(s, s->S, mark), frame);
+    HIP_OR_LATCH(s, enqueue_frame(s, s->S, turn.launch, mark), frame);
     HIP_OR_LATCH(s, hipStreamSynchronize(st), frame);
     s->profNames = names;
     s->profMs.assign(names.size(), 0.0f);
     for (size_t i = 0; i + 1 < ev.size(); i++) hipEventElapsedTime(&s->profMs[i], ev[i], ev[i + 1]);
     for (auto e : ev) hipEventDestroy(e);
   } else {
-    HIP_OR_LATCH(s, enqueue_frame(s, s->S), frame);
+    HIP_OR_LATCH(s, enqueue_frame(s, s->S, turn.launch), frame);
   }
   std::swap(s->S.manifolds, s->S.prevManifolds);
   std::swap(s->S.soft, s->S.prevSoft);
@@ -2488,10 +2491,10 @@ namespace {
 constexpr uint32_t kChunksInFlight = 3;
 
 hipError_t enqueue_chunk(avbd_solver* s, const DeviceState& S, const StepParams& P, uint32_t n, float tol,
-                         uint32_t maxIt) {
+                         uint32_t maxIt, Launch launch) {
   StepParams Pc = P;
   Pc.convCheck = 1u;  // the chunk's kernels stop once a check has ended the frame
-  hipError_t e = enqueue_iterations(s, S, Pc, n, true);
+  hipError_t e = enqueue_iterations(s, S, Pc, n, true, launch);
   if (e != hipSuccess) return e;
   launch_residual(s->stream, S, Pc, s->residualBlocks, true);
   launch_residual_check(s->stream, S, s->residualBlocks, tol, maxIt, n, s->convDev);
@@ -2511,14 +2514,11 @@ hipError_t build_residual_graphs(avbd_solver* s, float tol, int32_t maxIt, int32
   for (int p = 0; p < 2; p++) {
     hipError_t e = capture_graph(s, [&]() { enqueue_pre_solve(s, S, P, none); return hipGetLastError(); },
                                  &s->resPre[p]);
-    const bool now = s->cooperative;
-    for (int v = 0; v < 2 && e == hipSuccess; v++) {
-      if (v != (now ? 1 : 0) && !s->numTiles) continue;
-      s->cooperative = v == 1;
-      e = capture_graph(s, [&]() { return enqueue_chunk(s, S, P, (uint32_t)check, tol, (uint32_t)maxIt); },
-                        &s->resChunk[v][p]);
+    for (Launch l : {Launch::Tiles, Launch::Apart}) {
+      if (e != hipSuccess || (l == Launch::Tiles && !s->numTiles)) continue;
+      e = capture_graph(s, [&]() { return enqueue_chunk(s, S, P, (uint32_t)check, tol, (uint32_t)maxIt, l); },
+                        &s->resChunk[graph_form(l)][p]);
     }
-    s->cooperative = now;
     if (e == hipSuccess)
       e = capture_graph(s, [&]() { enqueue_post_solve(s, S, P, none); return hipGetLastError(); }, &s->resPost[p]);
     if (e != hipSuccess) return e;
@@ -2569,10 +2569,10 @@ extern "C" avbd_status avbd_step_to_residual(avbd_solver* s, float tol, int32_t 
   for (;;) {
     while (launched < total && launched - seen < kChunksInFlight) {
       if (launched < full && useGraph) {
-        HIP_OR_LATCH(s, hipGraphLaunch(s->resChunk[s->cooperative][parity], st), frame);
+        HIP_OR_LATCH(s, hipGraphLaunch(s->resChunk[graph_form(turn.launch)][parity], st), frame);
       } else {
         const uint32_t n = launched < full ? (uint32_t)check_every : tail;
-        HIP_OR_LATCH(s, enqueue_chunk(s, S, P, n, tol, (uint32_t)max_iterations), frame);
+        HIP_OR_LATCH(s, enqueue_chunk(s, S, P, n, tol, (uint32_t)max_iterations, turn.launch), frame);
       }
       launched++;
     }

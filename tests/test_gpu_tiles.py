@@ -115,3 +115,42 @@ def test_tiles_beside_other_solvers():
             assert g.runtimeFailure is None
             for x, y in zip(g.bodyStates(), want):
                 assert np.array_equal(x, y)
+
+
+def test_residual_frames_beside_grid_sweeps():
+    """Frames of tile solvers iterated to a residual, their graphs captured anew
+    for every frame (another chunk length each), while grid-wide sweeps step in
+    other threads: every solver ends where it ends alone, and none times out."""
+    import threading
+
+    flush_print("[gpu case] residual frames beside grid sweeps")
+    rigid = demos.stack_scene(height=140)
+
+    def solvers():
+        return [GPUSolver(_pair(cells=2, bottom=0.02)), GPUSolver(_pair(cells=9, bottom=0.02)),
+                GPUSolver(rigid, lanesPerBody=8, sweepMode=2), GPUSolver(rigid, lanesPerBody=4, sweepMode=2)]
+
+    def run(k, g):
+        for i in range(5):
+            if k < 2:
+                g.stepToResidual(1e-9, 40, 8 + 2 * (i % 2))
+            else:
+                g.step(8)
+                g.synchronize()
+
+    alone = []
+    for k, g in enumerate(solvers()):
+        with g:
+            run(k, g)
+            alone.append(g.bodyStates())
+    together = solvers()
+    threads = [threading.Thread(target=run, args=(k, g)) for k, g in enumerate(together)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g, want in zip(together, alone):
+        with g:
+            assert g.runtimeFailure is None
+            for x, y in zip(g.bodyStates(), want):
+                assert np.array_equal(x, y)
