@@ -48,6 +48,8 @@ struct HostBody {
 
 }  // namespace
 
+constexpr int kGraphForms = 3;  // of a frame's graphs, one for each Launch
+
 struct avbd_solver {
   avbd_settings settings{};
   avbd_options opts{};
@@ -123,13 +125,12 @@ struct avbd_solver {
   bool slotBusy[2] = {false, false};
   int64_t frameIndex = 0;
   int64_t pairCountsFrom = 1;  // first frame whose pair count is in pinnedCounters
-  // graphs (even / odd frame: manifold buffers alternate)
-  // one pair for ordinary launches, one with the waiting kernels launched
-  // cooperatively (scenes on the tile path only)
-  hipGraphExec_t graphs[2][2] = {};
-  bool graphsValid[2] = {false, false};
+  // graphs (even / odd frame: manifold buffers alternate), a pair for each
+  // form that the solver's frames have taken (graph_form)
+  hipGraphExec_t graphs[kGraphForms][2] = {};
+  bool graphsValid[kGraphForms] = {};
   bool graphsDisabled = false;
-  int64_t graphBaseFrame[2] = {1, 1};  // frame that replays the pair's first graph
+  int64_t graphBaseFrame[kGraphForms] = {};  // frame that replays the pair's first graph
   Turn turn;                   // announces frames with kernels that wait (tiles, grid barriers)
   // failure latch
   avbd_failure failure{};
@@ -155,7 +156,7 @@ struct avbd_solver {
   // even and odd frame roles, for one (chunk, tolerance, cap) key
   ConvHost* convHost = nullptr;
   ConvHost* convDev = nullptr;
-  hipGraphExec_t resPre[2] = {nullptr, nullptr}, resChunk[2][2] = {}, resPost[2] = {nullptr, nullptr};
+  hipGraphExec_t resPre[2] = {nullptr, nullptr}, resChunk[kGraphForms][2] = {}, resPost[2] = {nullptr, nullptr};
   bool resValid = false;
   int32_t resCheck = 0, resMax = 0;
   float resTol = 0.0f;
@@ -370,7 +371,7 @@ hipError_t enqueue_iterations(avbd_solver* s, const DeviceState& S, const StepPa
   StepParams P = P0;
   P.iterations = iterations;
   if (iterations == 0) return hipSuccess;
-  if (s->numTiles && s->tileHold == 0) {
+  if (s->numTiles && launch != Launch::Ends) {
     return launch_tile_solve(st, S, P, s->numTiles, s->staticUsedColors, s->tileThreads,
                              launch != Launch::Tiles);
   }
@@ -428,16 +429,24 @@ hipError_t enqueue_frame(avbd_solver* s, const DeviceState& S, Launch launch, co
   return hipGetLastError();
 }
 
-void invalidate_graphs(avbd_solver* s) {
+void drop_graph(hipGraphExec_t* g) {
+  if (*g) hipGraphExecDestroy(*g);
+  *g = nullptr;
+}
+void invalidate_residual_graphs(avbd_solver* s) {
   for (int i = 0; i < 2; i++) {
-    for (hipGraphExec_t* g : {&s->graphs[0][i], &s->graphs[1][i], &s->resPre[i], &s->resChunk[0][i], &s->resChunk[1][i],
-                              &s->resPost[i]}) {
-      if (*g) hipGraphExecDestroy(*g);
-      *g = nullptr;
-    }
+    drop_graph(&s->resPre[i]);
+    drop_graph(&s->resPost[i]);
+    for (int f = 0; f < kGraphForms; f++) drop_graph(&s->resChunk[f][i]);
   }
-  s->graphsValid[0] = s->graphsValid[1] = false;
   s->resValid = false;
+}
+void invalidate_graphs(avbd_solver* s) {
+  for (int f = 0; f < kGraphForms; f++) {
+    for (int i = 0; i < 2; i++) drop_graph(&s->graphs[f][i]);
+    s->graphsValid[f] = false;
+  }
+  invalidate_residual_graphs(s);
 }
 
 // captures what `body` enqueues on the solver stream into an executable graph
@@ -457,8 +466,8 @@ hipError_t capture_graph(avbd_solver* s, const std::function<hipError_t()>& body
   return e;
 }
 
-// which of the captured forms a frame replays: the tile kernel launched the ordinary way, or any other
-int graph_form(Launch launch) { return launch == Launch::Tiles ? 0 : 1; }
+// which captured form a frame replays: one for each launch that a frame may announce
+int graph_form(Launch launch) { return (int)launch; }
 
 hipError_t build_graphs(avbd_solver* s, Launch launch) {
   const int v = graph_form(launch);
@@ -482,15 +491,13 @@ hipError_t build_graphs(avbd_solver* s, Launch launch) {
   return hipSuccess;
 }
 
-avbd_status sync_all(avbd_solver* s);
-
 Turns& turns() {
   static Turns* t = new Turns();  // outlives every handle
   return *t;
 }
 // What the kernels of the solver's frames ask of the device.
 Launch frame_launch(const avbd_solver* s) {
-  if (s->numTiles) return Launch::Tiles;
+  if (s->numTiles) return s->tileHold == 0 ? Launch::Tiles : Launch::Ends;
   const bool grid = (s->dynamicColoring && !s->numIslands) || (s->sweepMode == 2 && !s->islandSolve);
   return grid ? Launch::Apart : Launch::Ends;
 }
@@ -526,12 +533,8 @@ struct FrameTurn {
 constexpr int kTileHold = 120;
 void choose_tile_path(avbd_solver* s, int slot) {
   if (!s->numTiles) return;
-  const bool was = s->tileHold == 0;
   if (s->dynContact[slot]) s->tileHold = kTileHold;
   else if (s->tileHold > 0) s->tileHold--;
-  if (was == (s->tileHold == 0)) return;
-  sync_all(s);  // the graphs of the other path may be running
-  invalidate_graphs(s);
 }
 // Bodies a tile is filled to before a further CU takes some: 8, 16 and 36
 // measured 0.59, 0.61 and 0.63 ms a frame on 125 vertices (9261: no difference).
@@ -2502,23 +2505,13 @@ hipError_t enqueue_chunk(avbd_solver* s, const DeviceState& S, const StepParams&
 }
 
 hipError_t build_residual_graphs(avbd_solver* s, float tol, int32_t maxIt, int32_t check) {
-  for (int i = 0; i < 2; i++)
-    for (hipGraphExec_t* g : {&s->resPre[i], &s->resChunk[0][i], &s->resChunk[1][i], &s->resPost[i]}) {
-      if (*g) hipGraphExecDestroy(*g);
-      *g = nullptr;
-    }
-  s->resValid = false;
+  invalidate_residual_graphs(s);
   DeviceState S = s->S;
   const StepParams P = make_params(s);
   auto none = [](const char*) {};
   for (int p = 0; p < 2; p++) {
     hipError_t e = capture_graph(s, [&]() { enqueue_pre_solve(s, S, P, none); return hipGetLastError(); },
                                  &s->resPre[p]);
-    for (Launch l : {Launch::Tiles, Launch::Apart}) {
-      if (e != hipSuccess || (l == Launch::Tiles && !s->numTiles)) continue;
-      e = capture_graph(s, [&]() { return enqueue_chunk(s, S, P, (uint32_t)check, tol, (uint32_t)maxIt, l); },
-                        &s->resChunk[graph_form(l)][p]);
-    }
     if (e == hipSuccess)
       e = capture_graph(s, [&]() { enqueue_post_solve(s, S, P, none); return hipGetLastError(); }, &s->resPost[p]);
     if (e != hipSuccess) return e;
@@ -2530,6 +2523,25 @@ hipError_t build_residual_graphs(avbd_solver* s, float tol, int32_t maxIt, int32
   s->resMax = maxIt;
   s->resTol = tol;
   s->resBase = s->frameIndex + 1;
+  return hipSuccess;
+}
+
+// the chunk graphs of one form, for the frame roles of resPre / resPost
+hipError_t build_chunk_graphs(avbd_solver* s, Launch launch) {
+  DeviceState S = s->S;
+  if ((s->frameIndex + 1 - s->resBase) & 1) {
+    std::swap(S.manifolds, S.prevManifolds);
+    std::swap(S.soft, S.prevSoft);
+  }
+  const StepParams P = make_params(s);
+  for (int p = 0; p < 2; p++) {
+    const hipError_t e = capture_graph(
+        s, [&]() { return enqueue_chunk(s, S, P, (uint32_t)s->resCheck, s->resTol, (uint32_t)s->resMax, launch); },
+        &s->resChunk[graph_form(launch)][p]);
+    if (e != hipSuccess) return e;
+    std::swap(S.manifolds, S.prevManifolds);
+    std::swap(S.soft, S.prevSoft);
+  }
   return hipSuccess;
 }
 
@@ -2546,8 +2558,13 @@ extern "C" avbd_status avbd_step_to_residual(avbd_solver* s, float tol, int32_t 
   choose_tile_path(s, slot);
   bool useGraph = s->opts.use_graph && !s->graphsDisabled && !s->profiling;
   FrameTurn turn(s, frame_launch(s));
-  if (useGraph && !(s->resValid && s->resCheck == check_every && s->resMax == max_iterations && s->resTol == tol)) {
-    if (build_residual_graphs(s, tol, max_iterations, check_every) != hipSuccess) {
+  const int form = graph_form(turn.launch);
+  if (useGraph) {
+    hipError_t e = hipSuccess;
+    if (!(s->resValid && s->resCheck == check_every && s->resMax == max_iterations && s->resTol == tol))
+      e = build_residual_graphs(s, tol, max_iterations, check_every);
+    if (e == hipSuccess && !s->resChunk[form][1]) e = build_chunk_graphs(s, turn.launch);
+    if (e != hipSuccess) {
       (void)hipGetLastError();
       invalidate_graphs(s);
       s->graphsDisabled = true;
@@ -2569,7 +2586,7 @@ extern "C" avbd_status avbd_step_to_residual(avbd_solver* s, float tol, int32_t 
   for (;;) {
     while (launched < total && launched - seen < kChunksInFlight) {
       if (launched < full && useGraph) {
-        HIP_OR_LATCH(s, hipGraphLaunch(s->resChunk[graph_form(turn.launch)][parity], st), frame);
+        HIP_OR_LATCH(s, hipGraphLaunch(s->resChunk[form][parity], st), frame);
       } else {
         const uint32_t n = launched < full ? (uint32_t)check_every : tail;
         HIP_OR_LATCH(s, enqueue_chunk(s, S, P, n, tol, (uint32_t)max_iterations, turn.launch), frame);

@@ -154,3 +154,50 @@ def test_residual_frames_beside_grid_sweeps():
             assert g.runtimeFailure is None
             for x, y in zip(g.bodyStates(), want):
                 assert np.array_equal(x, y)
+
+
+def _floating():
+    """A block next to weightless whose inner particles stand 4 % apart, and its middle one."""
+    s = demos.soft_block_scene(cells=4, bottom=0.5, radius_factor=0.48, vel_sigma=0.0, iterations=10)
+    s.settings.gravity = -0.01
+    return s, np.array([1 + (2 * 5 + 2) * 5 + 2], np.uint32)
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_inner_contacts_come_and_go(graph):
+    """A particle pushed into its neighbour, then apart for longer than the 120
+    frames that the tile path stays off, twice: each path's frames continue the
+    other's.  A frame may add the bound of _close to the displacements."""
+    flush_print(f"[gpu case] contacts inside a block come and go, graphs {graph}")
+    scene, middle = _floating()
+    with GPUSolver(scene, lanesPerBody=32, useGraph=graph) as a, \
+            GPUSolver(scene, lanesPerBody=32, sweepMode=1, useGraph=graph) as b:
+        frames = 0
+
+        def step(contacts):
+            nonlocal frames
+            for want in contacts:
+                a.step()
+                b.step()
+                assert a.stats().num_active_manifolds == b.stats().num_active_manifolds == want
+            frames += len(contacts)
+            pa, ra, va, wa = a.bodyStates()
+            pb, rb, vb, wb = b.bodyStates()
+            bound = 8 * (1 + frames) * float(np.abs(pb[1:]).max()) * 2.0 ** -23
+            assert np.abs(pa - pb).max() <= bound and np.abs(va - vb).max() <= 60 * bound
+
+        def push():
+            p, r, v, w = (x[middle] for x in b.bodyStates())
+            for g in (a, b):
+                g.setBodyStates(middle, p + np.float32([0.04, 0, 0]), r, v, w)
+
+        step([0] * 3)
+        for _ in range(2):
+            push()
+            step([1, 1] + [0] * 126)
+        for tol in (1e-9, 0.5):
+            push()
+            for g in (a, b):
+                g.stepToResidual(tol, 20, 10)
+            frames += 1
+            step([1] + [0] * 2)
