@@ -102,6 +102,9 @@ struct avbd_solver {
   uint32_t tileThreads = 0;
   int tileHold = 0;              // frames the tile path still stays off after contacts between dynamic bodies
   bool dynContact[2] = {false, false};  // per frame slot: the retired frame had contacts between dynamic bodies
+  uint32_t numDynamic = 0;       // dynamic bodies of a scene with tiles
+  std::vector<uint32_t> writeMark;  // per body: the last state write that held it
+  uint32_t writeCount = 0;
   uint32_t numIslands = 0;       // island workgroups that color the dynamic palette (0: grid-wide coloring)
   bool islandSolve = false;      // they also run the sweeps
   uint32_t islandThreads = 64;   // their workgroup size
@@ -289,12 +292,16 @@ bool stage_denied(const avbd_solver* s, const char* stage, int64_t frame) {
 // called after each stage with its name.
 using StageFn = std::function<void(const char*)>;
 
-void enqueue_pre_solve(avbd_solver* s, const DeviceState& S, const StepParams& P, const StageFn& stage) {
-  hipStream_t st = s->stream;
+void zero_frame_counts(avbd_solver* s, const DeviceState& S) {
   uint32_t* zp[6] = {S.counters, S.cellCount, S.cellRigid, S.dAdjCount, S.fineCount, S.colorFlags};
   uint32_t zn[6] = {CTR_TOTAL, s->gridHashSize, s->gridHashSize, s->nb, s->fineCellSize > 0.0f ? s->gridHashSize : 0u,
                     s->numIslands ? kColorPasses : 0u};
-  launch_zero_multi(st, zp, zn, 6);
+  launch_zero_multi(s->stream, zp, zn, 6);
+}
+
+void enqueue_pre_solve(avbd_solver* s, const DeviceState& S, const StepParams& P, const StageFn& stage) {
+  hipStream_t st = s->stream;
+  zero_frame_counts(s, S);
   if (s->datOn) launch_fill_u32(st, S.datT, s->nb, 0x3F800000u);  // 1.0f: no pass has lowered a fraction
   if (!s->rateJoints.empty())
     launch_rate_motors(st, S, s->rateJointDev, s->rateValueDev, (uint32_t)s->rateJoints.size(), P.dt);
@@ -527,14 +534,34 @@ struct FrameTurn {
 
 // Which path the next frame takes: after a frame with contacts between
 // dynamic bodies, which the tile kernel leaves to the grid-wide sweep, the
-// next kTileHold frames run one launch per color.  Frame f decides for frame
-// f + 2, whose submission has always seen f retired, so the choice does not
-// depend on when the caller synchronizes.
+// next kTileHold frames run one launch per color (a block of 12^3 cells with
+// such contacts in every frame 2.71 against 1.35 ms a frame, of 20^3 3.58
+// against 1.65, of 28^3 4.49 against 2.32).  Frame f decides for frame f + 2,
+// whose submission has always seen f retired, so the choice does not depend on
+// when the caller synchronizes; and a write of every dynamic body's state
+// forgets it (forget_contacts), so that it does not depend on what ran before.
 constexpr int kTileHold = 120;
 void choose_tile_path(avbd_solver* s, int slot) {
   if (!s->numTiles) return;
   if (s->dynContact[slot]) s->tileHold = kTileHold;
   else if (s->tileHold > 0) s->tileHold--;
+}
+// The two paths round differently: the same states written again have to take
+// the path they took the first time.
+void forget_contacts(avbd_solver* s, const uint32_t* idx, uint32_t n) {
+  if (!s->numTiles) return;
+  s->writeCount++;
+  uint32_t dynamic = 0;
+  for (uint32_t k = 0; k < n; k++) {
+    const uint32_t b = idx ? idx[k] : k;
+    if (s->mass[b] > 0.0f && s->writeMark[b] != s->writeCount) {
+      s->writeMark[b] = s->writeCount;
+      dynamic++;
+    }
+  }
+  if (dynamic < s->numDynamic) return;
+  s->tileHold = 0;
+  s->dynContact[0] = s->dynContact[1] = false;
 }
 // Bodies a tile is filled to before a further CU takes some: 8, 16 and 36
 // measured 0.59, 0.61 and 0.63 ms a frame on 125 vertices (9261: no difference).
@@ -2010,11 +2037,30 @@ avbd_status build_static_and_upload(avbd_solver* s, const avbd_scene_desc* d) {
   return islands;
 }
 
+// Whether dynamic bodies touch each other as uploaded: the first frame's
+// broadphase, narrow phase and contact adjacency, which the frame repeats.
+avbd_status touches_at_upload(avbd_solver* s, bool* touches) {
+  DeviceState& S = s->S;
+  const StepParams P = make_params(s);
+  zero_frame_counts(s, S);
+  launch_broadphase(s->stream, S, P);
+  launch_narrowphase(s->stream, S, P, s->gridCap);
+  launch_contact_adjacency(s->stream, S, P, s->gridCap);
+  uint32_t flag = 0;
+  if (hipMemcpyAsync(&flag, S.counters + CTR_DYN_CONTACT, 4, hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
+      hipStreamSynchronize(s->stream) != hipSuccess)
+    return AVBD_ERR_HIP;
+  *touches = flag != 0u;
+  launch_fill_u32(s->stream, S.counters, CTR_TOTAL, 0u);
+  return AVBD_OK;
+}
+
 // Tiles of a scene whose dynamic bodies are all particles of tets only:
 // bodies in Morton order of their positions, an equal share each, one
 // workgroup per tile and at most one per CU (all of them resident).  Scenes
 // past kTileOwn bodies a CU stay with one launch per color, which by then is
-// bound by memory and not by the launches.
+// bound by memory and not by the launches, and so do scenes whose dynamic
+// bodies touch each other as uploaded (see kTileHold).
 avbd_status build_tiles(avbd_solver* s, const std::vector<uint32_t>& colors, const std::vector<uint32_t>& sStart) {
   DeviceState& S = s->S;
   if (s->dynamicColoring || s->allMode != kModeTet || s->datOn || s->isoOn || s->opts.sweep_mode != 0 ||
@@ -2025,6 +2071,9 @@ avbd_status build_tiles(avbd_solver* s, const std::vector<uint32_t>& colors, con
     if (s->mass[b] > 0.0f) order.push_back(b);
   const uint32_t nd = (uint32_t)order.size(), C = s->staticUsedColors;
   if (nd == 0 || nd > kTileOwn * s->cus) return AVBD_OK;
+  bool touches = false;
+  if (const avbd_status st = touches_at_upload(s, &touches)) return st;
+  if (touches) return AVBD_OK;
   std::vector<F4> pos(s->nb);
   if (hipMemcpy(pos.data(), S.posLin, 16 * (size_t)s->nb, hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
   V3 lo = xyz(pos[order[0]]), hi = lo;
@@ -2115,6 +2164,8 @@ avbd_status build_tiles(avbd_solver* s, const std::vector<uint32_t>& colors, con
       upload(S.tileHaloBody, hb) || upload(S.tileIdx, idx))
     return AVBD_ERR_HIP;
   s->numTiles = T;
+  s->numDynamic = nd;
+  s->writeMark.assign(s->nb, 0u);
   s->tileThreads = (threads + 63u) / 64u * 64u;
   return AVBD_OK;
 }
@@ -2807,6 +2858,7 @@ extern "C" avbd_status avbd_set_body_states(avbd_solver* s, const uint32_t* idx,
   hipLaunchKernelGGL(k_write_states, dim3((n + 255) / 256), dim3(256), 0, s->stream, s->S, dIdx, n, dBuf,
                      dBuf + 3 * n, dBuf + 7 * n, dBuf + 10 * n);
   launch_reset_incident(s, dFlag);
+  forget_contacts(s, idx, n);
   // written states invalidate the learned stage's correction history
   if (s->wsBuilt) {
     hipMemsetAsync(s->W.corr, 0, 16 * (size_t)s->nb, s->stream);
@@ -2869,6 +2921,7 @@ extern "C" avbd_status avbd_set_body_states_noalloc(avbd_solver* s, const uint32
   hipLaunchKernelGGL(k_write_states, dim3((n + 255) / 256), dim3(256), 0, q, s->S, dIdx, n, dBuf,
                      dBuf + 3 * n, dBuf + 7 * n, dBuf + 10 * n);
   launch_reset_incident(s, dFlag);
+  forget_contacts(s, idx, n);
   if (s->wsBuilt) {
     launch_fill_u32(q, (uint32_t*)s->W.corr, 4 * s->nb, 0u);
     launch_fill_u32(q, (uint32_t*)s->W.corrPrev, 4 * s->nb, 0u);

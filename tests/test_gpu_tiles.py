@@ -10,10 +10,12 @@ compiler fuses multiply-adds differently in each: an update may differ by one
 rounding, 2^-24 of its step, which Gauss-Seidel contracts.  The bound is eight
 units in the last place of the scene's extent on positions, and sixty times
 that (1 / dt) on velocities."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from avbd_amd import GPUSolver, demos
+from avbd_amd import GPUSolver, _capi, demos
 from conftest import flush_print
 
 pytestmark = pytest.mark.gpu
@@ -201,3 +203,53 @@ def test_inner_contacts_come_and_go(graph):
                 g.stepToResidual(tol, 20, 10)
             frames += 1
             step([1] + [0] * 2)
+
+
+@pytest.mark.parametrize("write", ["all", "shuffled", "noalloc"])
+def test_states_written_again_take_the_same_path(write):
+    """The same start state three times in one solver, and in a new one, with a
+    contact between inner particles and frames after it: the same bits each time,
+    although the frame path stays changed for 120 frames after such a contact."""
+    flush_print(f"[gpu case] the same states again, {write}")
+    scene, middle = _floating()
+    runs = []
+    rng = np.random.default_rng(5)
+
+    def interval(g):
+        order = np.arange(len(p), dtype=np.uint32)
+        if write == "shuffled":
+            order = rng.permutation(len(p)).astype(np.uint32)
+        if write == "noalloc":
+            arrays = [np.ascontiguousarray(x[order]) for x in (p, r, v, w)]
+            assert g._lib.avbd_set_body_states_noalloc(
+                g._h, order.ctypes.data_as(C.POINTER(C.c_uint32)), len(order),
+                *[x.ctypes.data_as(C.POINTER(C.c_float)) for x in arrays]) == _capi.OK
+        else:
+            g.setBodyStates(order, p[order], r[order], v[order], w[order])
+        g.step(7)
+        runs.append(g.bodyStates())
+
+    with GPUSolver(scene) as g:
+        p, r, v, w = g.bodyStates()
+        p[middle] += np.float32([0.04, 0, 0])
+        v[1:] = rng.normal(0, 0.1, v[1:].shape).astype(np.float32)
+        for _ in range(3):
+            interval(g)
+    with GPUSolver(scene) as g:
+        interval(g)
+    for x in runs[1:]:
+        for i, j in zip(x, runs[0]):
+            assert np.array_equal(i, j)
+
+
+def test_touching_as_uploaded_keeps_color_launches():
+    """A block whose inner particles overlap at rest ends where one launch per
+    color ends, bit for bit (the same lanes), from its first frame."""
+    flush_print("[gpu case] inner particles touching as uploaded")
+    scene = _pair(cells=7, bottom=0.02, radius_factor=0.7)
+    with GPUSolver(scene, lanesPerBody=32) as a, GPUSolver(scene, lanesPerBody=32, sweepMode=1) as b:
+        a.step(5)
+        b.step(5)
+        assert a.stats().sweep_mode == 1
+        for x, y in zip(a.bodyStates(), b.bodyStates()):
+            assert np.array_equal(x, y)
