@@ -502,7 +502,7 @@ Turns& turns() {
   static Turns* t = new Turns();  // outlives every handle
   return *t;
 }
-// What the kernels of the solver's frames ask of the device.
+// What the kernels of the solver's next frame ask of the device.
 Launch frame_launch(const avbd_solver* s) {
   if (s->numTiles) return s->tileHold == 0 ? Launch::Tiles : Launch::Ends;
   const bool grid = (s->dynamicColoring && !s->numIslands) || (s->sweepMode == 2 && !s->islandSolve);
@@ -513,9 +513,11 @@ struct FrameTurn {
   avbd_solver* s;
   Launch launch = Launch::Ends;
   bool open = false;
-  FrameTurn(avbd_solver* solver, Launch want) : s(solver) {
+  // lasting: the frame stays announced as open while it runs
+  FrameTurn(avbd_solver* solver, Launch want, bool lasting) : s(solver) {
     if (want == Launch::Ends) return;
-    while (!turns().begin(&s->turn, want, &launch)) std::this_thread::yield();
+    auto after = [&](Turn* o, int slot) { hipStreamWaitEvent(s->stream, (hipEvent_t)o->event[slot], 0); };
+    while (!turns().begin(&s->turn, want, lasting, &launch, after)) std::this_thread::yield();
     open = true;
   }
   // the frame's completion is recorded in frameDone[slot]
@@ -1244,6 +1246,8 @@ extern "C" avbd_status avbd_create(const avbd_scene_desc* d, const avbd_options*
     if (e == hipErrorNotReady) (void)hipGetLastError();
     return e != hipErrorNotReady;
   };
+  for (int k = 0; k < 2; k++) s->turn.event[k] = s->frameDone[k];
+  s->turn.grid = s->numTiles == 0;  // the trials may launch grid-wide sweeps
   turns().join(&s->turn);
   autotune(s);
   create_phase(s, "autotune");
@@ -2361,7 +2365,8 @@ void autotune(avbd_solver* s) {
     if (s->sweepMode == 2 && s->persistentBlocks <= 0) s->sweepMode = 1;
     return;
   }
-  FrameTurn turn(s, Launch::Apart);  // the trials may launch grid-wide sweeps
+  const bool grid = s->dynamicColoring || std::find(modeCands.begin(), modeCands.end(), 2) != modeCands.end();
+  FrameTurn turn(s, grid ? Launch::Apart : Launch::Ends, false);
   // backup
   std::vector<std::pair<void*, size_t>> bufs = {
       {S.posLin, nb * 16}, {S.posLo, nb * 16}, {S.posAng, nb * 16}, {S.initLin, nb * 16}, {S.initAng, nb * 16},
@@ -2476,7 +2481,7 @@ extern "C" avbd_status avbd_submit_step(avbd_solver* s) {
   }
   choose_tile_path(s, slot);
   bool useGraph = s->opts.use_graph && !s->graphsDisabled && !s->profiling;
-  FrameTurn turn(s, frame_launch(s));
+  FrameTurn turn(s, frame_launch(s), false);
   const int form = graph_form(turn.launch);
   if (useGraph && !s->graphsValid[form]) {
     hipError_t e = build_graphs(s, turn.launch);
@@ -2608,7 +2613,7 @@ extern "C" avbd_status avbd_step_to_residual(avbd_solver* s, float tol, int32_t 
   hipStream_t st = s->stream;
   choose_tile_path(s, slot);
   bool useGraph = s->opts.use_graph && !s->graphsDisabled && !s->profiling;
-  FrameTurn turn(s, frame_launch(s));
+  FrameTurn turn(s, frame_launch(s), true);
   const int form = graph_form(turn.launch);
   if (useGraph) {
     hipError_t e = hipSuccess;

@@ -10,8 +10,11 @@
 // choice of its launch until its completion has been seen:
 //   - a tile frame is ordinary while no other solver's waiting frame is
 //     announced, cooperative otherwise;
-//   - a frame of grid-wide kernels is not begun while another solver's
-//     ordinary tile frame is announced.
+//   - a frame of grid-wide kernels is ordered, on the device, after the
+//     ordinary tile frames of other solvers.  It has to wait on the host only
+//     for one that is still being submitted, and a frame that its solver
+//     iterates to a residual, which stays open for as long as it runs, is
+//     ordinary only where no other solver has grid-wide kernels at all.
 //
 // No HIP calls: an entry brings its own completion query.
 #pragma once
@@ -28,10 +31,12 @@ enum class Launch : unsigned char {
   Tiles,  // the tile kernel, launched the ordinary way
 };
 
-// One solver's entry.  All but `device` and `done` belongs to Turns.
+// One solver's entry.  Up to `event` all is set before it joins; the rest belongs to Turns.
 struct Turn {
   int device = 0;
+  bool grid = false;                   // some of its frames hold grid-wide kernels
   std::function<bool(int slot)> done;  // has the frame submitted in this slot completed?
+  void* event[2] = {};                 // what its owner records behind a frame, for the frames ordered after it
   Launch open = Launch::Ends;          // the frame being submitted (or iterated to a residual)
   Launch slot[2] = {Launch::Ends, Launch::Ends};  // frames submitted and not seen to complete
 };
@@ -47,21 +52,25 @@ class Turns {
     list_.erase(std::remove(list_.begin(), list_.end(), t), list_.end());
   }
   // Announces t's next frame, which holds `want`; *got is how to launch it.
-  // False: not now, nothing announced.
-  bool begin(Turn* t, Launch want, Launch* got) {
+  // after(o, k): the frame has to run after the one in o's slot k.  `lasting`:
+  // it stays open while it runs.  False: not now, nothing announced.
+  template <typename After>
+  bool begin(Turn* t, Launch want, bool lasting, Launch* got, After&& after) {
     std::lock_guard<std::mutex> g(m_);
-    bool others = false, tiles = false;
+    bool others = false;
     for (Turn* o : list_) {
       if (o == t || o->device != t->device) continue;
       // not while it submits: it may be capturing, which a query of its events would end
       for (int k = 0; k < 2 && o->open == Launch::Ends; k++)
         if (o->slot[k] != Launch::Ends && o->done(k)) o->slot[k] = Launch::Ends;
-      for (Launch l : {o->open, o->slot[0], o->slot[1]}) {
-        others |= l != Launch::Ends;
-        tiles |= l == Launch::Tiles;
-      }
+      if (want == Launch::Apart && o->open == Launch::Tiles) return false;
+      for (Launch l : {o->open, o->slot[0], o->slot[1]}) others |= l != Launch::Ends;
+      others |= lasting && o->grid;
     }
-    if (want == Launch::Apart && tiles) return false;
+    if (want == Launch::Apart)
+      for (Turn* o : list_)
+        for (int k = 0; k < 2; k++)
+          if (o != t && o->device == t->device && o->slot[k] == Launch::Tiles) after(o, k);
     *got = t->open = want == Launch::Tiles && others ? Launch::Apart : want;
     return true;
   }

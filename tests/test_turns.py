@@ -11,6 +11,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 PROGRAM = r"""
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <thread>
@@ -22,8 +23,9 @@ struct Solver {
   Turn t;
   bool complete[2] = {false, false};
   Turns& all;
-  explicit Solver(Turns& a, int device = 0) : all(a) {
+  explicit Solver(Turns& a, int device = 0, bool grid = false) : all(a) {
     t.device = device;
+    t.grid = grid;
     t.done = [this](int k) {
       CHECK(t.open == Launch::Ends);  // a query may end the capture of a frame being submitted
       return complete[k];
@@ -31,45 +33,62 @@ struct Solver {
     all.join(&t);
   }
   ~Solver() { all.leave(&t); }
-  bool begin(Launch want, Launch expect) {
+  std::vector<std::pair<Turn*, int>> after;  // what the last frame begun has to run after
+  bool begin(Launch want, Launch expect, bool lasting = false) {
     Launch got = Launch::Ends;
-    return all.begin(&t, want, &got) && got == expect;
+    after.clear();
+    return all.begin(&t, want, lasting, &got, [&](Turn* o, int k) { after.push_back({o, k}); }) && got == expect;
+  }
+  bool behind(std::vector<std::pair<Turn*, int>> frames) {  // a grid-wide frame may begin, behind these
+    const bool ok = begin(Launch::Apart, Launch::Apart) && after == frames;
+    all.end(&t, -1);
+    return ok;
   }
   bool refused(Launch want) {
     Launch got;
-    return !all.begin(&t, want, &got);
+    return !all.begin(&t, want, false, &got, [](Turn*, int) { CHECK(false); });
   }
   void submit(int k) {
     complete[k] = false;
     all.end(&t, k);
   }
+  void finish(int k) {
+    submit(k);
+    complete[k] = true;
+    all.retire(&t, k, [] { return 0; });
+  }
 };
 
-// a frame alone is ordinary; others beside it are cooperative or wait
+// a frame alone is ordinary; others beside it are cooperative or come after it
 void announced() {
   Turns all;
   Solver a(all), b(all), grid(all);
   CHECK(a.begin(Launch::Tiles, Launch::Tiles));
   CHECK(b.begin(Launch::Tiles, Launch::Apart));
   b.all.end(&b.t, -1);
-  CHECK(grid.refused(Launch::Apart));
+  CHECK(grid.refused(Launch::Apart));  // its completion is not recorded yet
   a.submit(1);
-  CHECK(grid.refused(Launch::Apart));
+  CHECK(grid.behind({{&a.t, 1}}));
   CHECK(a.begin(Launch::Tiles, Launch::Tiles));  // its own frame before it is in the same stream
   CHECK(grid.refused(Launch::Apart));
   a.submit(0);
+  CHECK(grid.behind({{&a.t, 0}, {&a.t, 1}}));
   a.complete[1] = true;
-  CHECK(grid.refused(Launch::Apart));
-  a.complete[0] = true;
+  CHECK(grid.behind({{&a.t, 0}}));
   CHECK(grid.begin(Launch::Apart, Launch::Apart));
-  CHECK(a.begin(Launch::Tiles, Launch::Apart));
+  CHECK(a.begin(Launch::Tiles, Launch::Apart));  // the grid-wide frame is still to come
   a.submit(1);
+  a.complete[0] = true;
   CHECK(b.begin(Launch::Tiles, Launch::Apart));
-  b.all.end(&b.t, -1);
+  b.submit(0);
   grid.submit(0);
+  CHECK(grid.behind({}));  // cooperative frames are kept apart by the runtime
   grid.complete[0] = a.complete[1] = true;
-  CHECK(b.begin(Launch::Tiles, Launch::Tiles));
-  b.all.end(&b.t, -1);
+  CHECK(a.begin(Launch::Tiles, Launch::Apart));
+  a.all.end(&a.t, -1);
+  b.complete[0] = true;
+  CHECK(a.begin(Launch::Tiles, Launch::Tiles));
+  a.all.end(&a.t, -1);
 }
 
 // while its owner waits for a frame, the others still see it
@@ -79,14 +98,33 @@ void waited_for() {
   CHECK(a.begin(Launch::Tiles, Launch::Tiles));
   a.submit(0);
   const int r = all.retire(&a.t, 0, [&] {
-    CHECK(grid.refused(Launch::Apart));
+    CHECK(grid.behind({{&a.t, 0}}));
     CHECK(b.begin(Launch::Tiles, Launch::Apart));
     b.all.end(&b.t, -1);
     a.complete[0] = true;
     return 7;
   });
   CHECK(r == 7);
-  CHECK(grid.begin(Launch::Apart, Launch::Apart));
+  CHECK(grid.behind({}));
+}
+
+// a frame that stays open while it runs never keeps a grid-wide solver waiting that joined before it
+void lasting() {
+  Turns all;
+  Solver a(all), b(all);
+  CHECK(a.begin(Launch::Tiles, Launch::Tiles, true));
+  a.finish(0);
+  {
+    Solver far(all, 1, true), grid(all, 0, true);
+    CHECK(a.begin(Launch::Tiles, Launch::Apart, true));
+    CHECK(grid.behind({}));
+    a.finish(1);
+    CHECK(a.begin(Launch::Tiles, Launch::Tiles, false));
+    a.finish(0);
+  }
+  Solver far(all, 1, true);
+  CHECK(a.begin(Launch::Tiles, Launch::Tiles, true));
+  a.finish(1);
 }
 
 // devices are apart, and a solver that left is not seen
@@ -94,43 +132,52 @@ void apart() {
   Turns all;
   Solver other(all, 1), grid(all);
   CHECK(other.begin(Launch::Tiles, Launch::Tiles));
-  CHECK(grid.begin(Launch::Apart, Launch::Apart));
-  all.end(&grid.t, -1);
+  CHECK(grid.behind({}));
+  other.submit(0);
+  CHECK(grid.behind({}));
   {
     Solver a(all);
     CHECK(a.begin(Launch::Tiles, Launch::Tiles));
     CHECK(grid.refused(Launch::Apart));
   }
-  CHECK(grid.begin(Launch::Apart, Launch::Apart));
+  CHECK(grid.behind({}));
 }
 
-// four threads, every choice checked against what is on the device
+// four threads, every choice checked against what is on the device: a
+// completed frame's event is set, a frame ordered behind others waits for theirs
 void threads() {
   Turns all;
-  std::mutex m;
-  int ordinary = 0, cooperative = 0, grids = 0;
+  std::atomic<int> ordinary{0}, grids{0};
   auto run = [&](bool tiles) {
-    Solver s(all);
-    for (int i = 0; i < 4000; i++) {
+    Turn t;
+    std::atomic<bool> complete[2] = {{true}, {true}};
+    t.grid = !tiles;
+    t.done = [&](int k) { return complete[k].load(); };
+    all.join(&t);
+    for (int i = 0; i < 3000; i++) {
+      const int k = i & 1;
       Launch got;
-      if (!all.begin(&s.t, tiles ? Launch::Tiles : Launch::Apart, &got)) {
+      while (!all.begin(&t, tiles ? Launch::Tiles : Launch::Apart, i % 7 == 0, &got, [](Turn*, int) {}))
         std::this_thread::yield();
-        i--;
-        continue;
+      complete[k] = false;
+      if (got == Launch::Tiles) {
+        CHECK(++ordinary == 1);
+        CHECK(grids == 0);
       }
-      {
-        std::lock_guard<std::mutex> g(m);
-        (got == Launch::Tiles ? ordinary : tiles ? cooperative : grids)++;
-        CHECK(ordinary <= 1);
-        CHECK(!(ordinary && grids));
-      }
-      all.end(&s.t, i & 1);
-      all.retire(&s.t, i & 1, [&] {
-        std::lock_guard<std::mutex> g(m);
-        (got == Launch::Tiles ? ordinary : tiles ? cooperative : grids)--;
+      all.end(&t, k);
+      all.retire(&t, k, [&] {
+        if (!tiles) {  // the device runs it once the frames before it have ended
+          while (ordinary) std::this_thread::yield();
+          ++grids;
+          CHECK(ordinary == 0);
+          --grids;
+        }
+        if (got == Launch::Tiles) --ordinary;
+        complete[k] = true;
         return 0;
       });
     }
+    all.leave(&t);
   };
   std::thread a(run, true), b(run, true), c(run, false), d(run, false);
   a.join(), b.join(), c.join(), d.join();
@@ -140,6 +187,7 @@ int main(int, char** argv) {
   const std::string name = argv[1];
   if (name == "announced") announced();
   else if (name == "waited_for") waited_for();
+  else if (name == "lasting") lasting();
   else if (name == "apart") apart();
   else if (name == "threads") threads();
   else return 2;
@@ -156,7 +204,7 @@ def program(tmp_path_factory):
     return str(d / "turns")
 
 
-@pytest.mark.parametrize("name", ["announced", "waited_for", "apart", "threads"])
+@pytest.mark.parametrize("name", ["announced", "waited_for", "lasting", "apart", "threads"])
 def test_turns(program, name):
     r = subprocess.run([program, name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
