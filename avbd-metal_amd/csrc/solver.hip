@@ -502,9 +502,13 @@ Turns& turns() {
   static Turns* t = new Turns();  // outlives every handle
   return *t;
 }
+// Whether frames run the tile kernel (as far as the frames retired so far decide)
+bool tiles_on(const avbd_solver* s) { return s->numTiles && s->tileHold == 0; }
+int32_t sweep_mode_in_use(const avbd_solver* s) { return tiles_on(s) ? 2 : s->sweepMode; }
+
 // What the kernels of the solver's next frame ask of the device.
 Launch frame_launch(const avbd_solver* s) {
-  if (s->numTiles) return s->tileHold == 0 ? Launch::Tiles : Launch::Ends;
+  if (s->numTiles) return tiles_on(s) ? Launch::Tiles : Launch::Ends;
   const bool grid = (s->dynamicColoring && !s->numIslands) || (s->sweepMode == 2 && !s->islandSolve);
   return grid ? Launch::Apart : Launch::Ends;
 }
@@ -1253,7 +1257,7 @@ extern "C" avbd_status avbd_create(const avbd_scene_desc* d, const avbd_options*
   create_phase(s, "autotune");
   s->stats.lanes_per_body = s->lanes;
   if (frame_launch(s) == Launch::Ends) turns().leave(&s->turn);
-  s->stats.sweep_mode = s->numTiles ? 2 : s->sweepMode;
+  s->stats.sweep_mode = sweep_mode_in_use(s);
   s->stats.uses_dynamic_coloring = s->dynamicColoring ? 1 : 0;
   return AVBD_OK;
 }
@@ -3085,7 +3089,7 @@ extern "C" avbd_status avbd_get_stats(avbd_solver* s, avbd_stats* out) {
   if (!s || !out) return AVBD_ERR_INVALID_ARGUMENT;
   sync_all(s);
   s->stats.lanes_per_body = s->lanes;
-  s->stats.sweep_mode = s->numTiles ? 2 : s->sweepMode;
+  s->stats.sweep_mode = sweep_mode_in_use(s);
   s->stats.uses_dynamic_coloring = s->dynamicColoring ? 1 : 0;
   *out = s->stats;
   return AVBD_OK;

@@ -321,7 +321,8 @@ typedef struct avbd_stats {
     int32_t color_conflicts;
     int32_t uses_dynamic_coloring;
     int32_t lanes_per_body;        /* primal lane split in use */
-    int32_t sweep_mode;            /* 1 per-color launches, 2 persistent (the whole grid, or one workgroup per island) */
+    int32_t sweep_mode;            /* of the last frame: 1 one launch per color, 2 all sweeps in one launch (grid-wide,
+                                    * one workgroup per group of islands, or one per tile of a tetrahedral scene) */
     int32_t dat_pairs;             /* lastPlanarDATPairs: V-T + E-E pair demand */
     int32_t dat_vt_pairs;          /* lastPlanarDATVertexTrianglePairs */
     int32_t dat_ee_pairs;          /* lastPlanarDATEdgeEdgePairs */

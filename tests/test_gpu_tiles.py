@@ -78,7 +78,15 @@ def test_tiles_equal_the_color_launches(name):
         a.step(3)
         b.step(3)
         _close(a, b)
-        flush_print(f"  {a.stats().num_active_manifolds} contacts")
+        m = a.manifolds()["header"]
+        m = m[m[:, 2] > 0]  # active: bodies, contacts
+        static = a.bodyMass() <= 0
+        between = int((~static[m[:, 0]] & ~static[m[:, 1]]).sum())
+        _, touching = np.unique(m[:, :2][~static[m[:, :2]]], return_counts=True)
+        flush_print(f"  {len(m)} contacts, {between} between particles, at most {touching.max(initial=0)} of one")
+        assert len(m) or name == "pinned_6"
+        assert name == "too_large_33" or (between > 0) == (name == "self_contact_7")
+        assert name != "corner_4" or touching.max() == 2
 
 
 def test_tiles_beside_other_solvers():
@@ -92,8 +100,8 @@ def test_tiles_beside_other_solvers():
     def solvers():
         rigid = demos.stack_scene(height=140)
         return [GPUSolver(_pair(cells=1, bottom=0.02)), GPUSolver(_pair(cells=2, bottom=0.02)),
-                GPUSolver(_pair(cells=14, bottom=0.02)), GPUSolver(rigid), GPUSolver(rigid, sweepMode=2),
-                GPUSolver(demos.stack_scene(height=6))]
+                GPUSolver(_pair(cells=14, bottom=0.02)), GPUSolver(rigid, lanesPerBody=4),
+                GPUSolver(rigid, lanesPerBody=8, sweepMode=2), GPUSolver(demos.stack_scene(height=6))]
 
     alone = []
     for g in solvers():
@@ -176,12 +184,14 @@ def test_inner_contacts_come_and_go(graph):
             GPUSolver(scene, lanesPerBody=32, sweepMode=1, useGraph=graph) as b:
         frames = 0
 
-        def step(contacts):
+        def step(contacts, modes):
             nonlocal frames
-            for want in contacts:
+            for want, mode in zip(contacts, modes, strict=True):
                 a.step()
                 b.step()
-                assert a.stats().num_active_manifolds == b.stats().num_active_manifolds == want
+                sa = a.stats()
+                assert sa.num_active_manifolds == b.stats().num_active_manifolds == want
+                assert sa.sweep_mode == mode
             frames += len(contacts)
             pa, ra, va, wa = a.bodyStates()
             pb, rb, vb, wb = b.bodyStates()
@@ -193,16 +203,16 @@ def test_inner_contacts_come_and_go(graph):
             for g in (a, b):
                 g.setBodyStates(middle, p + np.float32([0.04, 0, 0]), r, v, w)
 
-        step([0] * 3)
+        step([0] * 3, [2] * 3)
         for _ in range(2):
             push()
-            step([1, 1] + [0] * 126)
+            step([1, 1] + [0] * 126, [2, 2] + [1] * 121 + [2] * 5)
         for tol in (1e-9, 0.5):
             push()
             for g in (a, b):
                 g.stepToResidual(tol, 20, 10)
             frames += 1
-            step([1] + [0] * 2)
+            step([1] + [0] * 2, [2, 1, 1] if tol == 1e-9 else [1, 1, 1])
 
 
 @pytest.mark.parametrize("write", ["all", "shuffled", "noalloc"])
