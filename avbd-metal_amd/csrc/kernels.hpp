@@ -70,7 +70,8 @@ void launch_contact_adjacency(hipStream_t st, const DeviceState& S, const StepPa
 // static palette: one Jacobi pass of c_v = mex{c_u : u < v, u ~ v}; sets CTR_COLOR_CHANGED when any color moved
 void launch_static_color_pass(hipStream_t st, const DeviceState& S, const StepParams& P, const uint32_t* in,
                               uint32_t* out);
-void launch_dynamic_coloring(hipStream_t st, const DeviceState& S, const StepParams& P);
+// gridWide: the repair may use a kernel with grid barriers
+void launch_dynamic_coloring(hipStream_t st, const DeviceState& S, const StepParams& P, bool gridWide);
 // colorStart / colorList of `colors` (CTR_COLOR_BASE counts zero on entry)
 void launch_color_buckets(hipStream_t st, const DeviceState& S, const StepParams& P, const uint32_t* colors);
 // primal specialisations of a color's bodies

@@ -264,7 +264,7 @@ __global__ void __launch_bounds__(256) k_color_repair_coop(DeviceState S, StepPa
   }
 }
 
-// Serial form, used only when cooperative launch is unavailable.
+// Serial form, used only when cooperative launch is unavailable or not wanted.
 __global__ void k_color_repair(DeviceState S, StepParams P, uint32_t* colors, uint32_t finalPass) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   if (S.colorFlags[finalPass] == 0u) return;
@@ -352,7 +352,7 @@ __global__ void k_color_starts(DeviceState S, StepParams P) {
   S.colorStart[kMaxColors + 1] = used;
 }
 
-void launch_dynamic_coloring(hipStream_t st, const DeviceState& S, const StepParams& P) {
+void launch_dynamic_coloring(hipStream_t st, const DeviceState& S, const StepParams& P, bool gridWide) {
   const uint32_t passes = kColorPasses;
   uint32_t bb = (P.numBodies + 255) / 256;
   launch_fill_u32(st, S.colorFlags, passes + 4, 0u);
@@ -363,7 +363,7 @@ void launch_dynamic_coloring(hipStream_t st, const DeviceState& S, const StepPar
     uint32_t* t = src; src = dst; dst = t;
   }
   // after an even number of passes the final colors are back in S.colors
-  int rb = repair_coop_blocks(P.numBodies);
+  int rb = gridWide ? repair_coop_blocks(P.numBodies) : 0;
   bool coop = false;
   if (rb > 0) {
     DeviceState s2 = S;

@@ -24,6 +24,7 @@
 #include "kernels.hpp"
 #include "lifetime.hpp"
 #include "turns.hpp"
+#include "claims.hpp"
 #include "mlp.hpp"
 
 // upload-time geometry must round exactly as written (radii feed the
@@ -100,6 +101,11 @@ struct avbd_solver {
   int lanes = 8, sweepMode = 1;
   uint32_t numTiles = 0;         // tiles of a tetrahedral scene (0: no tile path)
   uint32_t tileThreads = 0;
+  // locks against other processes' waiting kernels (claims.hpp)
+  std::string bus;               // the device's PCI bus id
+  Claim claim = Claim::None;     // what this solver holds
+  bool tilesElsewhere = false;   // tiles refused: one launch per color instead
+  bool gridElsewhere = false;    // grid-wide kernels refused: launches that end by themselves instead
   int tileHold = 0;              // frames the tile path still stays off after contacts between dynamic bodies
   bool dynContact[2] = {false, false};  // per frame slot: the retired frame had contacts between dynamic bodies
   uint32_t numDynamic = 0;       // dynamic bodies of a scene with tiles
@@ -341,7 +347,7 @@ void enqueue_pre_solve(avbd_solver* s, const DeviceState& S, const StepParams& P
   if (s->numIslands) {
     launch_island_coloring(st, S, s->numIslands, s->islandThreads);
     if (!s->islandSolve) launch_color_buckets(st, S, P, S.colors);
-  } else if (s->dynamicColoring) launch_dynamic_coloring(st, S, P);
+  } else if (s->dynamicColoring) launch_dynamic_coloring(st, S, P, !s->gridElsewhere);
   stage("coloring");
   // learned warm start: features, then (with a network) the learned start
   // and the residual comparison against the plain guess
@@ -498,6 +504,19 @@ hipError_t build_graphs(avbd_solver* s, Launch launch) {
   return hipSuccess;
 }
 
+Claims& claims() {
+  static Claims* c = new Claims();  // outlives every handle
+  return *c;
+}
+bool take_claim(avbd_solver* s, Claim what) {
+  if (!claims().take(s->bus, what)) return false;
+  s->claim = what;
+  return true;
+}
+void give_claim(avbd_solver* s) {
+  if (s->claim != Claim::None) claims().give(s->bus, s->claim);
+  s->claim = Claim::None;
+}
 Turns& turns() {
   static Turns* t = new Turns();  // outlives every handle
   return *t;
@@ -509,7 +528,8 @@ int32_t sweep_mode_in_use(const avbd_solver* s) { return tiles_on(s) ? 2 : s->sw
 // What the kernels of the solver's next frame ask of the device.
 Launch frame_launch(const avbd_solver* s) {
   if (s->numTiles) return tiles_on(s) ? Launch::Tiles : Launch::Ends;
-  const bool grid = (s->dynamicColoring && !s->numIslands) || (s->sweepMode == 2 && !s->islandSolve);
+  const bool grid =
+      (s->dynamicColoring && !s->numIslands && !s->gridElsewhere) || (s->sweepMode == 2 && !s->islandSolve);
   return grid ? Launch::Apart : Launch::Ends;
 }
 // a frame's announcement, from the choice of its launch to submitted()
@@ -1215,6 +1235,9 @@ extern "C" avbd_status avbd_create(const avbd_scene_desc* d, const avbd_options*
   avbd_solver* s = new avbd_solver();
   s->phaseT0 = std::chrono::steady_clock::now();
   hipGetDevice(&s->device);
+  char bus[32] = {};
+  if (hipDeviceGetPCIBusId(bus, (int)sizeof(bus), s->device) == hipSuccess) s->bus = bus;
+  else (void)hipGetLastError();
   if (resolve_fixed_scratch(s->device, &s->fixedScratch) != hipSuccess) {
     (void)hipGetLastError();
     delete s;
@@ -1256,7 +1279,10 @@ extern "C" avbd_status avbd_create(const avbd_scene_desc* d, const avbd_options*
   autotune(s);
   create_phase(s, "autotune");
   s->stats.lanes_per_body = s->lanes;
-  if (frame_launch(s) == Launch::Ends) turns().leave(&s->turn);
+  if (frame_launch(s) == Launch::Ends) {
+    turns().leave(&s->turn);
+    give_claim(s);
+  }
   s->stats.sweep_mode = sweep_mode_in_use(s);
   s->stats.uses_dynamic_coloring = s->dynamicColoring ? 1 : 0;
   return AVBD_OK;
@@ -1273,6 +1299,7 @@ void release_solver(avbd_solver* s) {
   if (!s) return;
   if (s->stream) hipStreamSynchronize(s->stream);
   turns().leave(&s->turn);
+  give_claim(s);
   invalidate_graphs(s);
   for (void* p : s->allocs) hipFree(p);
   for (int i = 0; i < 2; i++)
@@ -2068,7 +2095,8 @@ avbd_status touches_at_upload(avbd_solver* s, bool* touches) {
 // workgroup per tile and at most one per CU (all of them resident).  Scenes
 // past kTileOwn bodies a CU stay with one launch per color, which by then is
 // bound by memory and not by the launches, and so do scenes whose dynamic
-// bodies touch each other as uploaded (see kTileHold).
+// bodies touch each other as uploaded (see kTileHold), and those of a process
+// that another one keeps from launching tiles the ordinary way.
 avbd_status build_tiles(avbd_solver* s, const std::vector<uint32_t>& colors, const std::vector<uint32_t>& sStart) {
   DeviceState& S = s->S;
   if (s->dynamicColoring || s->allMode != kModeTet || s->datOn || s->isoOn || s->opts.sweep_mode != 0 ||
@@ -2163,6 +2191,10 @@ avbd_status build_tiles(avbd_solver* s, const std::vector<uint32_t>& colors, con
     for (uint32_t b = x; b < T; b += 8) torder[b] = next++;
   const uint32_t threads = std::min<uint32_t>(kTileThreads, std::max<uint32_t>(64u, widest * 32u));
   if (!tile_fits(threads)) return AVBD_OK;
+  if (!take_claim(s, Claim::Alone)) {
+    s->tilesElsewhere = true;
+    return AVBD_OK;
+  }
   if (hb.empty()) hb.push_back(U2{0u, 0u});
   if (dev_alloc(s, &S.tileOrder, T) || dev_alloc(s, &S.tileOwn, own.size()) || dev_alloc(s, &S.tileHalo, halo.size()) ||
       dev_alloc(s, &S.tileWork, work.size()) || dev_alloc(s, &S.tileHaloBody, hb.size()) ||
@@ -2350,8 +2382,8 @@ void autotune(avbd_solver* s) {
     return (int)std::min<uint32_t>(want, (uint32_t)maxB);
   };
   s->islandThreads = island_threads(s);
-  if (s->numTiles) {
-    s->lanes = 32;
+  if (s->numTiles || s->tilesElsewhere) {
+    s->lanes = 32;     // the tiles' order of a body's sums
     s->sweepMode = 1;  // while the tile path is off
     return;
   }
@@ -2359,6 +2391,12 @@ void autotune(avbd_solver* s) {
     s->lanes = laneCands.size() == 1 ? laneCands[0] : kIslandLanes;
     s->sweepMode = 2;
     return;
+  }
+  const bool grid = (s->dynamicColoring && !s->numIslands) ||
+                    std::find(modeCands.begin(), modeCands.end(), 2) != modeCands.end();
+  if (grid && !take_claim(s, Claim::Shared)) {
+    s->gridElsewhere = true;
+    modeCands = {1};
   }
   if (laneCands.size() == 1 && modeCands.size() == 1) {
     s->lanes = laneCands[0];
@@ -2369,8 +2407,7 @@ void autotune(avbd_solver* s) {
     if (s->sweepMode == 2 && s->persistentBlocks <= 0) s->sweepMode = 1;
     return;
   }
-  const bool grid = s->dynamicColoring || std::find(modeCands.begin(), modeCands.end(), 2) != modeCands.end();
-  FrameTurn turn(s, grid ? Launch::Apart : Launch::Ends, false);
+  FrameTurn turn(s, grid && !s->gridElsewhere ? Launch::Apart : Launch::Ends, false);
   // backup
   std::vector<std::pair<void*, size_t>> bufs = {
       {S.posLin, nb * 16}, {S.posLo, nb * 16}, {S.posAng, nb * 16}, {S.initLin, nb * 16}, {S.initAng, nb * 16},
@@ -2396,7 +2433,7 @@ void autotune(avbd_solver* s) {
   launch_fill_u32(st, S.dAdjStart, nb, 0u);
   if (s->dynamicColoring) {
     StepParams P = make_params(s);
-    launch_dynamic_coloring(st, S, P);
+    launch_dynamic_coloring(st, S, P, !s->gridElsewhere);
   }
   StepParams P = make_params(s);
   P.iterations = 2;

@@ -210,7 +210,13 @@ void avbd_scene_free(avbd_scene_desc* d);
 typedef struct avbd_options {
     int32_t max_pairs_per_body;        /* 16; maxPairs = max(4096, colliders * this), negative -> 16 */
     int32_t lanes_per_body;            /* 0 = automatic; else 4, 8, 16 or 32 lanes per body in the primal sweep */
-    int32_t sweep_mode;                /* 0 = automatic, 1 = one launch per color, 2 = persistent cooperative sweep */
+    int32_t sweep_mode;                /* 0 = automatic, 1 = one launch per color, 2 = persistent cooperative sweep.
+                                        * Automatic sweeps of tetrahedral scenes may launch, the ordinary way, a kernel
+                                        * whose workgroups wait for each other.  A process does so only while no other
+                                        * process has solvers of this or of grid-wide sweeps on the device, and then
+                                        * keeps others from both (a file in /dev/shm is locked; who is refused takes 1,
+                                        * also where 2 was asked for).  Processes on one device that do not share
+                                        * /dev/shm pass 1 themselves. */
     int32_t use_graph;                 /* 1 = capture each step in a hipGraph (default), 0 = eager launches */
     int32_t pair_capacity_override;    /* test hook (planarDATPairCapacityForTesting analogue): >0 caps rigid pairs */
     int32_t dat_pair_capacity_override;  /* test hook, planarDATPairCapacityForTesting (GPUSolver.swift:2119): >0 caps the V-T/E-E stream */

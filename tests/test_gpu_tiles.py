@@ -267,3 +267,48 @@ def test_touching_as_uploaded_keeps_color_launches():
         assert a.stats().sweep_mode == 1
         for x, y in zip(a.bodyStates(), b.bodyStates()):
             assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("kind", ["LOCK_EX", "LOCK_SH"])
+def test_another_process_holds_the_device(kind):
+    """While another process has the device's lock, a tetrahedral scene runs one
+    launch per color at the tiles' lanes, and while it has it alone a rigid scene
+    too large for island workgroups does so too, with the same bits; afterwards
+    both are as before."""
+    import gc
+    import glob
+    import subprocess
+    import sys
+
+    flush_print(f"[gpu case] tile and grid-wide scenes beside another process, {kind}")
+    soft, rigid = _pair(cells=4, bottom=0.02), demos.stack_scene(height=520)
+    hold = ("import fcntl, sys\n"
+            "files = [open(p, 'r+') for p in sys.argv[2:]]\n"
+            "for f in files: fcntl.lockf(f, getattr(fcntl, sys.argv[1]) | fcntl.LOCK_NB)\n"
+            "print('held', flush=True)\n"
+            "sys.stdin.read()\n")
+
+    def ends(scene, mode, lanes, **kw):
+        with GPUSolver(scene, lanesPerBody=lanes, **kw) as g:
+            g.step(6)
+            assert g.stats().sweep_mode == mode
+            return g.bodyStates()
+
+    def same(a, b):
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y)
+
+    gc.collect()  # solvers that earlier tests left open hold the lock for this process
+    tiles, grid = ends(soft, 2, 32), ends(rigid, 2, 4, sweepMode=2)
+    other = subprocess.Popen([sys.executable, "-c", hold, kind, *glob.glob("/dev/shm/avbd_device_*")],
+                             stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True)
+    try:
+        assert other.stdout.readline().strip() == "held"
+        same(ends(soft, 1, 0), ends(soft, 1, 32, sweepMode=1))
+        same(ends(rigid, 1 if kind == "LOCK_EX" else 2, 4, sweepMode=2), grid)
+    finally:
+        other.stdin.close()
+        other.wait(timeout=30)
+        other.stdout.close()
+    same(ends(soft, 2, 0), tiles)
+    same(ends(rigid, 2, 4, sweepMode=2), grid)
