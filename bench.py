@@ -10,9 +10,12 @@ GPU; the timed region is K steps bracketed by device synchronisation.
 value = dynamic vertices x iterations x steps / wall time.
 
 The same JSON line carries:
-  * roofline: the primal color sweep (the dominant kernel) timed live with
-    HIP events on the solver stream, algorithmic bytes per launch from the
-    per-stamp record model, DRAM traffic from the committed PMC summary;
+  * roofline: the kernel that runs the step's sweeps (the tile kernel, all
+    sweeps of a frame in one launch; one color's primal launch for scenes and
+    options that sweep so), timed live with HIP events on the solver stream,
+    algorithmic bytes per launch from the per-stamp record model, DRAM traffic
+    from the committed PMC summary; beside one-launch sweeps, one color's
+    launch of the same scene as per_color_launch;
   * config.residual_1e-4: frames of the block iterated until the residual is
     <= 1e-4 (sweep cap --res-cap, default 1000: the FP32 and FP64 oracles need
     110-370 sweeps per frame on this block, beyond the metric's 200), with
@@ -121,6 +124,31 @@ def primal_roofline(solver, pmc):
             "kernel": f"k_primal<{st.lanes_per_body}>", "avg_launch_us": round(tp["avg_launch_us"], 3),
             "algorithmic_bytes_per_launch": round(bytes_per_launch),
             "launches_per_sweep": tp["launches_per_sweep"]}
+
+
+def sweep_roofline(solver, iterations, kernel, pmc, color_pmc):
+    """The kernel that runs the frames' sweeps: `kernel` where one launch does
+    (its time from the events around the solve stage of eager frames), else one
+    color's primal launch."""
+    import numpy as np
+
+    per_color = primal_roofline(solver, color_pmc)
+    if solver.stats().sweep_mode != 2 or kernel is None:
+        return per_color
+    solver.setProfiling(True)
+    ms = []
+    for _ in range(20):
+        solver.step()
+        solver.synchronize()
+        ms.append(solver.profile()["solve"])
+    solver.setProfiling(False)
+    us = float(np.median(ms)) * 1e3
+    size = per_color["algorithmic_bytes_per_launch"] * per_color["launches_per_sweep"] * iterations
+    achieved = size / (us * 1e-6) / 1e9
+    return {"bound": "hbm", "limited_by": "latency of the color chain", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic_from_profiles(pmc), "kernel": kernel,
+            "avg_launch_us": round(us, 3), "algorithmic_bytes_per_launch": round(size), "launches_per_step": 1,
+            "per_color_launch": per_color}
 
 
 def timed_steps(solver, steps, warmup):
@@ -322,14 +350,14 @@ def config_batched(args, threads):
     with GPUSolver(s) as g:
         wall = timed_steps(g, args.side_steps, 5)
         st = g.stats()
-        roof = primal_roofline(g, None)
+        roof = sweep_roofline(g, s.settings.iterations, "k_island_solve", None, None)
     it = s.settings.iterations
     out = {"workload": f"4096 batched uneven rigid scenes ({s.numDynamic} bodies, {len(s.joints)} hinges), "
                        f"{it} iterations, dt 1/60, contact-aware dynamic coloring",
            "ms_per_step": round(wall * 1e3 / args.side_steps, 4),
            "body_iters_per_s": round(s.numDynamic * it * args.side_steps / wall, 1),
            "colors": st.num_colors, "lanes_per_body": st.lanes_per_body,
-           "sweep_mode": "persistent" if st.sweep_mode == 2 else "per-color launches", "roofline": roof}
+           "sweep_mode": "one launch" if st.sweep_mode == 2 else "per-color launches", "roofline": roof}
     small, _ = demos.batched_scene(64)
     out["error_vs_fp64"] = dict(error_vs_fp64(small, args.fp64_batched_steps, threads),
                                 scenes="the first 64 of the 4096 scenes")
@@ -429,6 +457,7 @@ def main():
 
     model, nproc, allowed, threads = cpu_info()
     unit, pmc = "vertex-iters/s", f"primal_soft_block_{args.cells + 1}_pmc.json"
+    kernel, solve_pmc = None, None  # of scenes whose sweeps are one launch
     if args.workload == "cloth":
         scene = demos.cloth_scene()
         desc = (f"cloth drape 256^2 ({scene.numDynamic} vertices, {len(scene.tris)} triangles) onto a fixed "
@@ -438,11 +467,12 @@ def main():
         scene = demos.batched_scene()[0]
         desc = (f"4096 batched uneven rigid scenes ({scene.numDynamic} bodies, {len(scene.joints)} hinges), "
                 f"{scene.settings.iterations} iterations, dt 1/60, contact-aware dynamic coloring")
-        unit, pmc = "body-iters/s", None
+        unit, pmc, kernel = "body-iters/s", None, "k_island_solve"
     else:
         scene = demos.soft_block_scene(cells=args.cells)
         desc = (f"soft block {args.cells}^3 cells, {scene.numDynamic} vertices, {len(scene.tets)} SNH tets, "
                 f"{scene.settings.iterations} iterations, dt 1/60, static coloring")
+        kernel, solve_pmc = "k_tile_solve", f"tile_soft_block_{args.cells + 1}_pmc.json"
     iters, nv = scene.settings.iterations, scene.numDynamic
     if args.workload != "soft_block":
         args.quick, args.no_learned, args.res_frames, args.fp64_steps = True, True, 0, 0
@@ -456,11 +486,11 @@ def main():
         st = solver.stats()
         cfg = {"workload": desc, "dynamic_bodies": nv, "iterations": iters, "colors": st.num_colors,
                "lanes_per_body": st.lanes_per_body,
-               "sweep_mode": "persistent" if st.sweep_mode == 2 else "per-color launches",
+               "sweep_mode": "one launch" if st.sweep_mode == 2 else "per-color launches",
                "end_residual": solver.residual()}
-        out["roofline"] = primal_roofline(solver, pmc)
+        out["roofline"] = sweep_roofline(solver, iters, kernel if args.sweep == 0 else None, solve_pmc, pmc)
     out["config"] = cfg
-    log(f"headline {out['ms_per_step']} ms/step, primal frac {out['roofline']['frac']}")
+    log(f"headline {out['ms_per_step']} ms/step, {out['roofline']['kernel']} {out['roofline']['frac']} of the peak")
     if args.fp64_steps > 0:
         cfg["error_vs_fp64"] = error_vs_fp64(scene, args.fp64_steps, threads)
 
