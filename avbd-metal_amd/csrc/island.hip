@@ -177,8 +177,9 @@ void launch_island_coloring(hipStream_t st, const DeviceState& S, uint32_t numIs
 // against 1.81), 64 bodies a workgroup as good as 32 or 128; splitting the
 // listed contacts over the threads took the dual of 128 bodies from 20 us
 // (eight lanes per body, its manifolds in turn) to the time of a color.
-// 4096 batched scenes: this kernel 0.67 ms, the frame 3.35 -> 1.84 ms with the
-// coloring above; 64 scenes 1.18 -> 0.64 ms, a 10-cube stack 0.48 -> 0.29 ms.
+// 4096 batched scenes: this kernel 0.65 ms, the frame 3.35 -> 1.84 ms with the
+// coloring above; 64 scenes 0.30, the frame 1.18 -> 0.64 ms; a 10-cube stack
+// 0.144 (20 colors and 10 duals, 4.8 us each), the frame 0.48 -> 0.29 ms.
 // ---------------------------------------------------------------------------
 // f(manifold, contacts) for every active manifold of the workgroup's bodies,
 // split over its threads; one of two dynamic bodies belongs to its first

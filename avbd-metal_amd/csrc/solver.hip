@@ -2325,7 +2325,11 @@ avbd_status static_coloring(avbd_solver* s) {
 
 // Workgroup size of the island kernels: enough lane groups for the larger
 // color of the largest island (two colors share a stack or chain about
-// evenly), at most kIslandThreads.
+// evenly), at most kIslandThreads.  Four lanes a body with many islands and
+// with few; the solve of a frame with 4, 8, 16 and 32 lanes, us:
+//   a stack of 10 cubes 146 149 263 372, of 64 222 333 735 1297, of 128 266 448
+//   903 1764; 64 scenes 367 382 786 1435, 512 487 447 646 1178, 4096 783 985
+//   1610 2830
 constexpr int kIslandLanes = 4;
 uint32_t island_threads(const avbd_solver* s) {
   const uint32_t want = (s->largestIsland + 1) / 2 * (uint32_t)kIslandLanes;

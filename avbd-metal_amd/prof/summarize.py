@@ -1,5 +1,4 @@
-"""Summaries of the profiling recipes (profile_soft_block.sh,
-profile_learned.sh): per-kernel
+"""Summaries of the profiling recipes (profile_*.sh): per-kernel
 durations of the benchmark and HBM bytes per launch of the primal kernel
 from the FETCH_SIZE / WRITE_SIZE passes, calibrated on a plain copy of known
 size.  Writes kernels_soft_block_<side>.txt and primal_soft_block_<side>_pmc.json
@@ -44,9 +43,28 @@ def kernels_only(stats_csv, dest, title, cmd):
     print("\n".join(lines[:12]))
 
 
+def bytes_only(out, kernel, dest, cmd):
+    """HBM bytes per launch of one kernel from the FETCH_SIZE / WRITE_SIZE
+    passes on it and on the copy, in <out>/prof_<counter>."""
+    res = {"command": cmd, "kernel": kernel, "hbm_bytes_per_launch": 0.0}
+    for c in ("FETCH_SIZE", "WRITE_SIZE"):
+        b, n = counter_avg(os.path.join(out, f"prof_{c}", "bench_counter_collection.csv"), c, kernel)
+        k, _ = counter_avg(os.path.join(out, f"prof_{c}", "copy_counter_collection.csv"), c, "k_copy")
+        res[c] = {"avg_kib": b, "dispatches": n, "copy_avg_kib": k, "copy_bytes": COPY_BYTES,
+                  "bytes": b * COPY_BYTES / k}
+        res["hbm_bytes_per_launch"] += res[c]["bytes"]
+    os.makedirs(os.path.dirname(dest), exist_ok=True)
+    with open(dest, "w") as f:
+        json.dump(res, f, indent=1)
+    print(json.dumps(res))
+
+
 def main():
     if sys.argv[1] == "--kernels-only":
         kernels_only(*sys.argv[2:6])
+        return
+    if sys.argv[1] == "--bytes-only":
+        bytes_only(*sys.argv[2:6])
         return
     out, bench_cmd = sys.argv[1], sys.argv[2]
     side = int(sys.argv[3]) if len(sys.argv) > 3 else 21
