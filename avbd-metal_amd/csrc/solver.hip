@@ -539,7 +539,7 @@ struct FrameTurn {
   bool open = false;
   // lasting: the frame stays announced as open while it runs
   FrameTurn(avbd_solver* solver, Launch want, bool lasting) : s(solver) {
-    if (want == Launch::Ends) return;
+    if (want == Launch::Ends && !s->numTiles) return;  // no entry
     auto after = [&](Turn* o, int slot) { hipStreamWaitEvent(s->stream, (hipEvent_t)o->event[slot], 0); };
     while (!turns().begin(&s->turn, want, lasting, &launch, after)) std::this_thread::yield();
     open = true;

@@ -12,7 +12,7 @@
 //     announced, cooperative otherwise;
 //   - a frame of grid-wide kernels is ordered, on the device, after the
 //     ordinary tile frames of other solvers.  It has to wait on the host only
-//     for one that is still being submitted, and a frame that its solver
+//     while such a solver is submitting, and a frame that its solver
 //     iterates to a residual, which stays open for as long as it runs, is
 //     ordinary only where no other solver has grid-wide kernels at all.
 //
@@ -37,7 +37,8 @@ struct Turn {
   bool grid = false;                   // some of its frames hold grid-wide kernels
   std::function<bool(int slot)> done;  // has the frame submitted in this slot completed?
   void* event[2] = {};                 // what its owner records behind a frame, for the frames ordered after it
-  Launch open = Launch::Ends;          // the frame being submitted (or iterated to a residual)
+  bool submitting = false;             // a frame is being submitted (or iterated to a residual)
+  Launch open = Launch::Ends;          // what that frame holds
   Launch slot[2] = {Launch::Ends, Launch::Ends};  // frames submitted and not seen to complete
 };
 
@@ -51,7 +52,8 @@ class Turns {
     std::lock_guard<std::mutex> g(m_);
     list_.erase(std::remove(list_.begin(), list_.end(), t), list_.end());
   }
-  // Announces t's next frame, which holds `want`; *got is how to launch it.
+  // Announces t's next frame, which holds `want`; *got is how to launch it.  A
+  // solver with an entry announces frames that end by themselves too.
   // after(o, k): the frame has to run after the one in o's slot k.  `lasting`:
   // it stays open while it runs.  False: not now, nothing announced.
   template <typename After>
@@ -60,10 +62,12 @@ class Turns {
     bool others = false;
     for (Turn* o : list_) {
       if (o == t || o->device != t->device) continue;
-      // not while it submits: it may be capturing, which a query of its events would end
-      for (int k = 0; k < 2 && o->open == Launch::Ends; k++)
+      // its events are left alone while it submits: it may be capturing, which a query of them would end
+      for (int k = 0; k < 2 && !o->submitting; k++)
         if (o->slot[k] != Launch::Ends && o->done(k)) o->slot[k] = Launch::Ends;
-      if (want == Launch::Apart && o->open == Launch::Tiles) return false;
+      if (want == Launch::Apart && o->submitting)
+        for (Launch l : {o->open, o->slot[0], o->slot[1]})
+          if (l == Launch::Tiles) return false;
       for (Launch l : {o->open, o->slot[0], o->slot[1]}) others |= l != Launch::Ends;
       others |= lasting && o->grid;
     }
@@ -72,6 +76,7 @@ class Turns {
         for (int k = 0; k < 2; k++)
           if (o != t && o->device == t->device && o->slot[k] == Launch::Tiles) after(o, k);
     *got = t->open = want == Launch::Tiles && others ? Launch::Apart : want;
+    t->submitting = true;
     return true;
   }
   // The frame is submitted in `slot`, its completion recorded there; slot < 0: it left nothing on the device.
@@ -79,6 +84,7 @@ class Turns {
     std::lock_guard<std::mutex> g(m_);
     if (slot >= 0) t->slot[slot] = t->open;
     t->open = Launch::Ends;
+    t->submitting = false;
   }
   // Waits for the slot's frame (`wait`), which stays announced meanwhile.
   template <typename Wait>

@@ -129,21 +129,36 @@ def test_tiles_beside_other_solvers():
 
 def test_residual_frames_beside_grid_sweeps():
     """Frames of tile solvers iterated to a residual, their graphs captured anew
-    for every frame (another chunk length each), while grid-wide sweeps step in
-    other threads: every solver ends where it ends alone, and none times out."""
+    for every frame (another chunk length each), and frames that change between
+    the tiles and launches per color, captured while a tile frame is in flight,
+    while grid-wide sweeps step in other threads: every solver ends where it ends
+    alone, and none times out."""
     import threading
 
     flush_print("[gpu case] residual frames beside grid sweeps")
     rigid = demos.stack_scene(height=140)
+    floating, middle = _floating()
+    with GPUSolver(floating) as g:
+        states = g.bodyStates()
+    everything = np.arange(len(states[0]), dtype=np.uint32)
 
     def solvers():
         return [GPUSolver(_pair(cells=2, bottom=0.02)), GPUSolver(_pair(cells=9, bottom=0.02)),
-                GPUSolver(rigid, lanesPerBody=8, sweepMode=2), GPUSolver(rigid, lanesPerBody=4, sweepMode=2)]
+                GPUSolver(rigid, lanesPerBody=8, sweepMode=2), GPUSolver(rigid, lanesPerBody=4, sweepMode=2),
+                GPUSolver(floating)]
 
     def run(k, g):
         for i in range(5):
             if k < 2:
                 g.stepToResidual(1e-9, 40, 8 + 2 * (i % 2))
+            elif k == 4:
+                p, r, v, w = states
+                q = p.copy()
+                q[middle] += np.float32([0.04, 0, 0])
+                g.settings = g.settings  # drops the graphs
+                g.setBodyStates(everything, q, r, v, w)
+                g.step(8)
+                g.synchronize()
             else:
                 g.step(8)
                 g.synchronize()

@@ -27,7 +27,7 @@ struct Solver {
     t.device = device;
     t.grid = grid;
     t.done = [this](int k) {
-      CHECK(t.open == Launch::Ends);  // a query may end the capture of a frame being submitted
+      CHECK(!t.submitting);  // a query may end the capture of a frame being submitted
       return complete[k];
     };
     all.join(&t);
@@ -89,6 +89,29 @@ void announced() {
   b.complete[0] = true;
   CHECK(a.begin(Launch::Tiles, Launch::Tiles));
   a.all.end(&a.t, -1);
+}
+
+// a solver whose frame ends by itself, with a tile frame before it in flight, may be capturing
+void mixed() {
+  Turns all;
+  Solver a(all), b(all), grid(all);
+  CHECK(a.begin(Launch::Tiles, Launch::Tiles));
+  a.submit(0);
+  CHECK(a.begin(Launch::Ends, Launch::Ends));
+  CHECK(grid.refused(Launch::Apart));
+  CHECK(b.begin(Launch::Tiles, Launch::Apart));
+  b.all.end(&b.t, -1);
+  a.submit(1);
+  CHECK(grid.behind({{&a.t, 0}}));
+  a.complete[0] = true;
+  CHECK(a.begin(Launch::Ends, Launch::Ends));
+  CHECK(grid.refused(Launch::Apart));  // not asked while it submits
+  a.finish(0);
+  CHECK(a.begin(Launch::Ends, Launch::Ends));
+  CHECK(grid.behind({}));
+  CHECK(b.begin(Launch::Tiles, Launch::Tiles));
+  b.finish(0);
+  a.finish(1);
 }
 
 // while its owner waits for a frame, the others still see it
@@ -186,6 +209,7 @@ void threads() {
 int main(int, char** argv) {
   const std::string name = argv[1];
   if (name == "announced") announced();
+  else if (name == "mixed") mixed();
   else if (name == "waited_for") waited_for();
   else if (name == "lasting") lasting();
   else if (name == "apart") apart();
@@ -204,7 +228,7 @@ def program(tmp_path_factory):
     return str(d / "turns")
 
 
-@pytest.mark.parametrize("name", ["announced", "waited_for", "lasting", "apart", "threads"])
+@pytest.mark.parametrize("name", ["announced", "mixed", "waited_for", "lasting", "apart", "threads"])
 def test_turns(program, name):
     r = subprocess.run([program, name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
