@@ -1401,15 +1401,19 @@ avbd_status build_islands(avbd_solver* s, const avbd_scene_desc* d) {
   csr(s->nj, [&](uint32_t i) { return island(d->joint_body_a[i], d->joint_body_b[i]); }, jstart, jlist);
   csr(s->ns, [&](uint32_t i) { return island(d->spring_body_a[i], d->spring_body_b[i]); }, pstart, plist);
   DeviceState& S = s->S;
-  if (dev_alloc(s, &S.islandStart, start.size()) || dev_alloc(s, &S.islandBody, body.size()) ||
-      dev_alloc(s, &S.islandLocal, local.size()) || dev_alloc(s, &S.islandJointStart, jstart.size()) ||
-      dev_alloc(s, &S.islandJoint, jlist.size()) || dev_alloc(s, &S.islandSpringStart, pstart.size()) ||
-      dev_alloc(s, &S.islandSpring, plist.size()))
-    return AVBD_ERR_ALLOC;
-  if (upload(S.islandStart, start) || upload(S.islandBody, body) || upload(S.islandLocal, local) ||
-      upload(S.islandJointStart, jstart) || upload(S.islandJoint, jlist) || upload(S.islandSpringStart, pstart) ||
-      upload(S.islandSpring, plist))
-    return AVBD_ERR_HIP;
+  // one block: seven allocations and copies took longer than the rest of this
+  const std::vector<uint32_t>* parts[7] = {&start, &body, &local, &jstart, &jlist, &pstart, &plist};
+  uint32_t** to[7] = {&S.islandStart, &S.islandBody, &S.islandLocal, &S.islandJointStart, &S.islandJoint,
+                      &S.islandSpringStart, &S.islandSpring};
+  std::vector<uint32_t> all;
+  for (const auto* p : parts) all.insert(all.end(), p->begin(), p->end());
+  uint32_t* block = nullptr;
+  if (dev_alloc(s, &block, all.size())) return AVBD_ERR_ALLOC;
+  if (upload(block, all)) return AVBD_ERR_HIP;
+  for (int k = 0; k < 7; k++) {
+    *to[k] = block;
+    block += parts[k]->size();
+  }
   s->numIslands = n;
   s->islandSolve = widest <= kIslandSolveMax;
   for (uint32_t k = 0; k < n; k++) s->largestIsland = std::max(s->largestIsland, start[k + 1] - start[k]);
