@@ -8,6 +8,7 @@
 
 #include "../../include/avbd.h"
 #include "lifetime.hpp"
+#include "gate.hpp"
 #include "mlp.hpp"
 
 using namespace avbd;
@@ -32,15 +33,15 @@ template <typename T>
 hipError_t grab(std::vector<void*>& list, T** p, size_t count) {
   void* q = nullptr;
   size_t bytes = std::max<size_t>(16, count * sizeof(T));
-  hipError_t e = hipMalloc(&q, bytes);
+  hipError_t e = alloc_now(&q, bytes);
   if (e != hipSuccess) return e;
   list.push_back(q);
   *p = (T*)q;
-  return hipMemset(q, 0, bytes);
+  return fill_now(q, 0, bytes);
 }
 
 void release(std::vector<void*>& list) {
-  for (void* p : list) hipFree(p);
+  for (void* p : list) free_now(p);
   list.clear();
 }
 
@@ -166,7 +167,7 @@ extern "C" avbd_status avbd_mlp_info(const avbd_mlp* m, int32_t* outputs, int32_
 extern "C" avbd_status avbd_mlp_get_params(avbd_mlp* m, float* params) {
   if (!m || !params) return AVBD_ERR_INVALID_ARGUMENT;
   if (hipStreamSynchronize(m->stream) != hipSuccess) return AVBD_ERR_HIP;
-  if (hipMemcpy(params, m->M.params, (size_t)m->M.nParams * 4, hipMemcpyDeviceToHost) != hipSuccess)
+  if (copy_now(params, m->M.params, (size_t)m->M.nParams * 4, hipMemcpyDeviceToHost) != hipSuccess)
     return AVBD_ERR_HIP;
   return AVBD_OK;
 }
@@ -177,8 +178,8 @@ extern "C" avbd_status avbd_mlp_set_params(avbd_mlp* m, const float* params) {
   for (size_t i = 0; i < np; i++)
     if (!std::isfinite(params[i])) return AVBD_ERR_INVALID_ARGUMENT;
   if (hipStreamSynchronize(m->stream) != hipSuccess) return AVBD_ERR_HIP;
-  if (hipMemcpy(m->M.params, params, np * 4, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemset(m->T.m, 0, np * 4) != hipSuccess || hipMemset(m->T.v, 0, np * 4) != hipSuccess)
+  if (copy_now(m->M.params, params, np * 4, hipMemcpyHostToDevice) != hipSuccess ||
+      fill_now(m->T.m, 0, np * 4) != hipSuccess || fill_now(m->T.v, 0, np * 4) != hipSuccess)
     return AVBD_ERR_HIP;
   m->adamStep = 0;
   launch_mlp_pack(m->stream, m->M);

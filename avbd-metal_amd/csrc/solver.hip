@@ -25,6 +25,7 @@
 #include "lifetime.hpp"
 #include "turns.hpp"
 #include "claims.hpp"
+#include "gate.hpp"
 #include "mlp.hpp"
 
 // upload-time geometry must round exactly as written (radii feed the
@@ -212,9 +213,9 @@ hipError_t dev_alloc(avbd_solver* s, T** p, size_t count) {
   size_t bytes = count * sizeof(T);
   if (bytes < 16) bytes = 16;
   void* q = nullptr;
-  hipError_t e = hipMalloc(&q, bytes);
+  hipError_t e = alloc_now(&q, bytes);
   if (e != hipSuccess) return e;
-  e = hipMemset(q, 0, bytes);
+  e = fill_now(q, 0, bytes);
   s->allocs.push_back(q);
   *p = (T*)q;
   return e;
@@ -223,7 +224,7 @@ hipError_t dev_alloc(avbd_solver* s, T** p, size_t count) {
 template <typename T>
 hipError_t upload(T* dst, const std::vector<T>& src) {
   if (src.empty()) return hipSuccess;
-  return hipMemcpy(dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice);
+  return copy_now(dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice);
 }
 
 StepParams make_params(const avbd_solver* s) {
@@ -465,10 +466,14 @@ void invalidate_graphs(avbd_solver* s) {
 // captures what `body` enqueues on the solver stream into an executable graph
 hipError_t capture_graph(avbd_solver* s, const std::function<hipError_t()>& body, hipGraphExec_t* out) {
   hipGraph_t g = nullptr;
-  hipError_t e = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
-  if (e != hipSuccess) return e;
-  hipError_t eq = body();
-  e = hipStreamEndCapture(s->stream, &g);
+  hipError_t e, eq;
+  {
+    CaptureApart apart;
+    e = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
+    if (e != hipSuccess) return e;
+    eq = body();
+    e = hipStreamEndCapture(s->stream, &g);
+  }
   if (eq != hipSuccess) {
     if (g) hipGraphDestroy(g);
     return eq;
@@ -486,15 +491,7 @@ hipError_t build_graphs(avbd_solver* s, Launch launch) {
   const int v = graph_form(launch);
   DeviceState S = s->S;
   for (int p = 0; p < 2; p++) {
-    hipGraph_t g = nullptr;
-    hipError_t e = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
-    if (e != hipSuccess) return e;
-    hipError_t eq = enqueue_frame(s, S, launch);
-    e = hipStreamEndCapture(s->stream, &g);
-    if (eq != hipSuccess) { if (g) hipGraphDestroy(g); return eq; }
-    if (e != hipSuccess) return e;
-    e = hipGraphInstantiate(&s->graphs[v][p], g, nullptr, nullptr, 0);
-    hipGraphDestroy(g);
+    const hipError_t e = capture_graph(s, [&]() { return enqueue_frame(s, S, launch); }, &s->graphs[v][p]);
     if (e != hipSuccess) return e;
     std::swap(S.manifolds, S.prevManifolds);
     std::swap(S.soft, S.prevSoft);
@@ -1301,12 +1298,12 @@ void release_solver(avbd_solver* s) {
   turns().leave(&s->turn);
   give_claim(s);
   invalidate_graphs(s);
-  for (void* p : s->allocs) hipFree(p);
+  for (void* p : s->allocs) free_now(p);
   for (int i = 0; i < 2; i++)
     if (s->frameDone[i]) hipEventDestroy(s->frameDone[i]);
-  if (s->pinnedCounters) hipHostFree(s->pinnedCounters);
-  if (s->residualPartialHost) hipHostFree(s->residualPartialHost);
-  if (s->convHost) hipHostFree(s->convHost);
+  if (s->pinnedCounters) free_host_now(s->pinnedCounters);
+  if (s->residualPartialHost) free_host_now(s->residualPartialHost);
+  if (s->convHost) free_host_now(s->convHost);
   if (s->stream) hipStreamDestroy(s->stream);
   delete s;
 }
@@ -2051,14 +2048,14 @@ avbd_status build_static_and_upload(avbd_solver* s, const avbd_scene_desc* d) {
   }
 
   create_phase(s, "uploads");
-  if (hipHostMalloc((void**)&s->pinnedCounters, 2 * CTR_TOTAL * sizeof(uint32_t), hipHostMallocDefault) !=
+  if (alloc_host_now(&s->pinnedCounters, 2 * CTR_TOTAL * sizeof(uint32_t), hipHostMallocDefault) !=
       hipSuccess)
     return AVBD_ERR_ALLOC;
   memset(s->pinnedCounters, 0, 2 * CTR_TOTAL * sizeof(uint32_t));
-  if (hipHostMalloc((void**)&s->residualPartialHost, 2 * bb * sizeof(double), hipHostMallocDefault) != hipSuccess)
+  if (alloc_host_now(&s->residualPartialHost, 2 * bb * sizeof(double), hipHostMallocDefault) != hipSuccess)
     return AVBD_ERR_ALLOC;
   // written by the device's residual checks, read by the host while kernels run
-  if (hipHostMalloc((void**)&s->convHost, sizeof(ConvHost), hipHostMallocMapped | hipHostMallocCoherent) !=
+  if (alloc_host_now(&s->convHost, sizeof(ConvHost), hipHostMallocMapped | hipHostMallocCoherent) !=
           hipSuccess ||
       hipHostGetDevicePointer((void**)&s->convDev, s->convHost, 0) != hipSuccess)
     return AVBD_ERR_ALLOC;
@@ -2115,7 +2112,7 @@ avbd_status build_tiles(avbd_solver* s, const std::vector<uint32_t>& colors, con
   if (const avbd_status st = touches_at_upload(s, &touches)) return st;
   if (touches) return AVBD_OK;
   std::vector<F4> pos(s->nb);
-  if (hipMemcpy(pos.data(), S.posLin, 16 * (size_t)s->nb, hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
+  if (copy_now(pos.data(), S.posLin, 16 * (size_t)s->nb, hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
   V3 lo = xyz(pos[order[0]]), hi = lo;
   for (uint32_t b : order) {
     lo = v3(fminf(lo.x, pos[b].x), fminf(lo.y, pos[b].y), fminf(lo.z, pos[b].z));
@@ -2243,8 +2240,8 @@ avbd_status static_coloring(avbd_solver* s) {
   // synchronize with the null stream)
   if (hipStreamSynchronize(st) != hipSuccess) return AVBD_ERR_HIP;
   std::vector<uint32_t> colors(s->nb);
-  if (hipMemcpy(colors.data(), in, 4 * s->nb, hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
-  if (in != S.colors && hipMemcpy(S.colors, in, 4 * s->nb, hipMemcpyDeviceToDevice) != hipSuccess)
+  if (copy_now(colors.data(), in, 4 * s->nb, hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
+  if (in != S.colors && copy_now(S.colors, in, 4 * s->nb, hipMemcpyDeviceToDevice) != hipSuccess)
     return AVBD_ERR_HIP;
   uint32_t maxColor = 0;
   std::vector<std::vector<uint32_t>> buckets(kMaxColors);
@@ -2427,7 +2424,7 @@ void autotune(avbd_solver* s) {
   std::vector<void*> backups;
   for (auto& b : bufs) {
     void* q = nullptr;
-    if (hipMalloc(&q, b.second) != hipSuccess) { backups.push_back(nullptr); continue; }
+    if (alloc_now(&q, b.second) != hipSuccess) { backups.push_back(nullptr); continue; }
     hipMemcpyAsync(q, b.first, b.second, hipMemcpyDeviceToDevice, st);
     backups.push_back(q);
   }
@@ -2480,7 +2477,7 @@ void autotune(avbd_solver* s) {
       hipEventRecord(e1, st);
       if (!ok || hipEventSynchronize(e1) != hipSuccess) { hipGetLastError(); continue; }
       uint32_t fail = 0;
-      hipMemcpy(&fail, S.counters + CTR_GBAR_FAIL, 4, hipMemcpyDeviceToHost);
+      copy_now(&fail, S.counters + CTR_GBAR_FAIL, 4, hipMemcpyDeviceToHost);
       if (fail) continue;
       float ms = 0.0f;
       hipEventElapsedTime(&ms, e0, e1);
@@ -2495,7 +2492,7 @@ void autotune(avbd_solver* s) {
   }
   hipStreamSynchronize(st);
   for (void* q : backups)
-    if (q) hipFree(q);
+    if (q) free_now(q);
   s->lanes = bestL;
   s->sweepMode = bestM;
   s->persistentBlocks = bestBlocks ? bestBlocks : pblocks(bestL);
@@ -2770,7 +2767,7 @@ template <typename T>
 avbd_status read_dev(avbd_solver* s, std::vector<T>& out, const T* src, size_t n) {
   out.resize(n);
   if (n == 0) return AVBD_OK;
-  if (hipMemcpy(out.data(), src, n * sizeof(T), hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
+  if (copy_now(out.data(), src, n * sizeof(T), hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
   return AVBD_OK;
 }
 }  // namespace
@@ -2889,7 +2886,7 @@ extern "C" avbd_status avbd_set_body_states(avbd_solver* s, const uint32_t* idx,
   const size_t fl = (size_t)n * 13;
   const size_t words = (size_t)n + s->nb + fl;
   void* block = nullptr;
-  if (hipMalloc(&block, 4 * words) != hipSuccess) {
+  if (alloc_now(&block, 4 * words) != hipSuccess) {
     (void)hipGetLastError();
     return AVBD_ERR_ALLOC;
   }
@@ -2901,10 +2898,10 @@ extern "C" avbd_status avbd_set_body_states(avbd_solver* s, const uint32_t* idx,
   memcpy(buf.data() + 3 * (size_t)n, rot4, 16 * (size_t)n);
   memcpy(buf.data() + 7 * (size_t)n, vel3, 12 * (size_t)n);
   memcpy(buf.data() + 10 * (size_t)n, angvel3, 12 * (size_t)n);
-  if (hipMemcpy(dIdx, ids.data(), 4 * (size_t)n, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(dFlag, flag.data(), 4 * (size_t)s->nb, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(dBuf, buf.data(), 4 * fl, hipMemcpyHostToDevice) != hipSuccess) {
-    hipFree(block);
+  if (copy_now(dIdx, ids.data(), 4 * (size_t)n, hipMemcpyHostToDevice) != hipSuccess ||
+      copy_now(dFlag, flag.data(), 4 * (size_t)s->nb, hipMemcpyHostToDevice) != hipSuccess ||
+      copy_now(dBuf, buf.data(), 4 * fl, hipMemcpyHostToDevice) != hipSuccess) {
+    free_now(block);
     return AVBD_ERR_HIP;
   }
   // the incident joints get back the penalties stored at upload
@@ -2920,7 +2917,7 @@ extern "C" avbd_status avbd_set_body_states(avbd_solver* s, const uint32_t* idx,
     hipMemsetAsync(s->W.corrAng, 0, 16 * (size_t)s->nb, s->stream);
   }
   hipError_t e = hipStreamSynchronize(s->stream);
-  hipFree(block);
+  free_now(block);
   if (e != hipSuccess) return latch(s, AVBD_FAIL_COMMAND_EXECUTION, s->frameIndex, 0, 0, (int)e, "set_body_states");
   return AVBD_OK;
 }
@@ -2999,19 +2996,19 @@ __global__ void k_set_joint_field(DeviceState S, const uint32_t* j, const float*
 avbd_status set_joint_field(avbd_solver* s, const uint32_t* joints, uint32_t n, const float* v, int field) {
   const uint32_t width = field == 2 ? 3u : 1u;
   void* block = nullptr;  // joint ids [n], then values [width n]
-  if (hipMalloc(&block, 4 * (size_t)n * (1 + width)) != hipSuccess) {
+  if (alloc_now(&block, 4 * (size_t)n * (1 + width)) != hipSuccess) {
     (void)hipGetLastError();
     return AVBD_ERR_ALLOC;
   }
   uint32_t* dj = (uint32_t*)block;
   float* dv = (float*)(dj + n);
-  hipError_t e = hipMemcpy(dj, joints, 4 * (size_t)n, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(dv, v, 4 * (size_t)width * n, hipMemcpyHostToDevice);
+  hipError_t e = copy_now(dj, joints, 4 * (size_t)n, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = copy_now(dv, v, 4 * (size_t)width * n, hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_set_joint_field, dim3((n + 255) / 256), dim3(256), 0, s->stream, s->S, dj, dv, n, field);
     e = hipStreamSynchronize(s->stream);
   }
-  hipFree(block);
+  free_now(block);
   return e == hipSuccess ? AVBD_OK : AVBD_ERR_HIP;
 }
 // the preconditions of GPUSolver.swift:2496-2590 as argument errors; kept
@@ -3143,7 +3140,7 @@ extern "C" avbd_status avbd_get_stats(avbd_solver* s, avbd_stats* out) {
 extern "C" avbd_status avbd_get_colors(avbd_solver* s, uint32_t n, uint32_t* colors) {
   if (!s || !colors || n > s->nb) return AVBD_ERR_INVALID_ARGUMENT;
   sync_all(s);
-  if (hipMemcpy(colors, s->S.colors, 4 * n, hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
+  if (copy_now(colors, s->S.colors, 4 * n, hipMemcpyDeviceToHost) != hipSuccess) return AVBD_ERR_HIP;
   return AVBD_OK;
 }
 
@@ -3154,11 +3151,11 @@ extern "C" avbd_status avbd_get_cell_lists(avbd_solver* s, uint32_t* hash_size, 
   if (hash_size) *hash_size = s->gridHashSize;
   if (num_hashed) *num_hashed = s->nHashed;
   if (cell_size) *cell_size = s->cellSize;
-  if (cell_start && hipMemcpy(cell_start, s->S.cellStart, 4 * s->gridHashSize, hipMemcpyDeviceToHost))
+  if (cell_start && copy_now(cell_start, s->S.cellStart, 4 * s->gridHashSize, hipMemcpyDeviceToHost))
     return AVBD_ERR_HIP;
-  if (cell_count && hipMemcpy(cell_count, s->S.cellCount, 4 * s->gridHashSize, hipMemcpyDeviceToHost))
+  if (cell_count && copy_now(cell_count, s->S.cellCount, 4 * s->gridHashSize, hipMemcpyDeviceToHost))
     return AVBD_ERR_HIP;
-  if (cell_bodies && s->nHashed && hipMemcpy(cell_bodies, s->S.cellBodies, 4 * s->nHashed, hipMemcpyDeviceToHost))
+  if (cell_bodies && s->nHashed && copy_now(cell_bodies, s->S.cellBodies, 4 * s->nHashed, hipMemcpyDeviceToHost))
     return AVBD_ERR_HIP;
   return AVBD_OK;
 }
@@ -3167,10 +3164,10 @@ extern "C" avbd_status avbd_get_pairs(avbd_solver* s, uint32_t capacity, uint32_
   if (!s || !n) return AVBD_ERR_INVALID_ARGUMENT;
   sync_all(s);
   uint32_t cnt = 0;
-  if (hipMemcpy(&cnt, s->S.counters + CTR_PAIRS, 4, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (copy_now(&cnt, s->S.counters + CTR_PAIRS, 4, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
   *n = cnt;
   uint32_t m = std::min(cnt, capacity);
-  if (pairs && m && hipMemcpy(pairs, s->S.pairs, 8 * m, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (pairs && m && copy_now(pairs, s->S.pairs, 8 * m, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
   return AVBD_OK;
 }
 
@@ -3178,11 +3175,11 @@ extern "C" avbd_status avbd_get_manifolds(avbd_solver* s, uint32_t capacity, uin
   if (!s || !n) return AVBD_ERR_INVALID_ARGUMENT;
   sync_all(s);
   uint32_t cnt = 0;
-  if (hipMemcpy(&cnt, s->S.counters + CTR_PAIRS, 4, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (copy_now(&cnt, s->S.counters + CTR_PAIRS, 4, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
   *n = cnt;
   uint32_t m = std::min(cnt, capacity);
   // the frame just retired wrote into what is now prevManifolds
-  if (records && m && hipMemcpy(records, s->S.prevManifolds, sizeof(ManifoldRec) * m, hipMemcpyDeviceToHost))
+  if (records && m && copy_now(records, s->S.prevManifolds, sizeof(ManifoldRec) * m, hipMemcpyDeviceToHost))
     return AVBD_ERR_HIP;
   return AVBD_OK;
 }
@@ -3209,10 +3206,10 @@ extern "C" avbd_status avbd_get_cloth_info(avbd_solver* s, avbd_cloth_info* info
     info->dat_on = s->datOn ? 1u : 0u;
     info->iso_on = s->isoOn ? 1u : 0u;
   }
-  if (edges && s->nEdges && hipMemcpy(edges, s->S.edges, 8 * (size_t)s->nEdges, hipMemcpyDeviceToHost))
+  if (edges && s->nEdges && copy_now(edges, s->S.edges, 8 * (size_t)s->nEdges, hipMemcpyDeviceToHost))
     return AVBD_ERR_HIP;
   if (particles && s->nParticles &&
-      hipMemcpy(particles, s->S.particleIdx, 4 * (size_t)s->nParticles, hipMemcpyDeviceToHost))
+      copy_now(particles, s->S.particleIdx, 4 * (size_t)s->nParticles, hipMemcpyDeviceToHost))
     return AVBD_ERR_HIP;
   return AVBD_OK;
 }
@@ -3221,7 +3218,7 @@ extern "C" avbd_status avbd_get_motor_targets(avbd_solver* s, uint32_t n, float*
   if (!s || (n && !targets) || n > s->nj) return AVBD_ERR_INVALID_ARGUMENT;
   sync_all(s);
   std::vector<JointRec> j(n);
-  if (n && hipMemcpy(j.data(), s->S.joints, sizeof(JointRec) * n, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (n && copy_now(j.data(), s->S.joints, sizeof(JointRec) * n, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
   for (uint32_t i = 0; i < n; i++) targets[i] = j[i].motor.x;
   return AVBD_OK;
 }
@@ -3232,7 +3229,7 @@ extern "C" avbd_status avbd_get_collision_tris(avbd_solver* s, uint32_t capacity
   uint32_t m = std::min(s->nTris, capacity);
   if (!tris || !m) return AVBD_OK;
   std::vector<U4> tmp(m);
-  if (hipMemcpy(tmp.data(), s->S.tris, sizeof(U4) * m, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (copy_now(tmp.data(), s->S.tris, sizeof(U4) * m, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
   for (uint32_t i = 0; i < m; i++) {
     tris[3 * i] = tmp[i].x;
     tris[3 * i + 1] = tmp[i].y;
@@ -3248,13 +3245,13 @@ extern "C" avbd_status avbd_get_dat_pairs(avbd_solver* s, uint32_t capacity, uin
   if (!s->pairStream) return AVBD_OK;
   uint32_t cnt = 0;
   // the stream of the accepted predictor pose (its demand is the working count)
-  if (hipMemcpy(&cnt, s->S.datStart + s->nParticles + s->nEdges, 4, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (copy_now(&cnt, s->S.datStart + s->nParticles + s->nEdges, 4, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
   cnt = std::min(cnt, s->maxDatPairs);
   *n = cnt;
   uint32_t m = std::min(cnt, capacity);
   if (pairs && m) {
     std::vector<U4> tmp(m);
-    if (hipMemcpy(tmp.data(), s->S.datPairs, sizeof(U4) * m, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+    if (copy_now(tmp.data(), s->S.datPairs, sizeof(U4) * m, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
     for (uint32_t i = 0; i < m; i++) {
       pairs[3 * i] = tmp[i].x;
       pairs[3 * i + 1] = tmp[i].y;
@@ -3270,11 +3267,11 @@ extern "C" avbd_status avbd_get_soft_contacts(avbd_solver* s, uint32_t capacity,
   *n = 0;
   if (!s->nTris) return AVBD_OK;
   uint32_t cnt = 0;
-  if (hipMemcpy(&cnt, s->S.counters + CTR_SOFT, 4, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (copy_now(&cnt, s->S.counters + CTR_SOFT, 4, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
   *n = cnt;
   uint32_t m = std::min(cnt, capacity);
   // the frame just retired wrote into what is now prevSoft
-  if (records && m && hipMemcpy(records, s->S.prevSoft, sizeof(SoftRec) * m, hipMemcpyDeviceToHost))
+  if (records && m && copy_now(records, s->S.prevSoft, sizeof(SoftRec) * m, hipMemcpyDeviceToHost))
     return AVBD_ERR_HIP;
   return AVBD_OK;
 }
@@ -3293,12 +3290,12 @@ extern "C" avbd_status avbd_get_iso_state(avbd_solver* s, uint32_t* vt_track, ui
   avbd_status st = sync_all(s);
   if (st != AVBD_OK) return st;
   const size_t nb = s->nb, ne = s->numContactEdges;
-  if (vt_track && hipMemcpy(vt_track, s->S.vtTrack, 16 * nb, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
-  if (ee_track && ne && hipMemcpy(ee_track, s->S.eeTrack, 16 * ne, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
-  if (bound && hipMemcpy(bound, s->S.ogcBound, 4 * nb, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (vt_track && copy_now(vt_track, s->S.vtTrack, 16 * nb, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (ee_track && ne && copy_now(ee_track, s->S.eeTrack, 16 * ne, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+  if (bound && copy_now(bound, s->S.ogcBound, 4 * nb, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
   if (anchor) {
     std::vector<F4> tmp(nb);
-    if (hipMemcpy(tmp.data(), s->S.ogcPrev, 16 * nb, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
+    if (copy_now(tmp.data(), s->S.ogcPrev, 16 * nb, hipMemcpyDeviceToHost)) return AVBD_ERR_HIP;
     for (size_t i = 0; i < nb; i++) {
       anchor[3 * i] = tmp[i].x;
       anchor[3 * i + 1] = tmp[i].y;
@@ -3319,25 +3316,25 @@ static avbd_status map_query(avbd_solver* s, const uint32_t* pairs, uint32_t n, 
   sync_all(s);
   U2* dq = nullptr;
   int32_t* dout = nullptr;
-  if (hipMalloc(&dq, 8ull * n) != hipSuccess) return AVBD_ERR_ALLOC;
-  if (hipMalloc(&dout, 4ull * n) != hipSuccess) {
-    hipFree(dq);
+  if (alloc_now(&dq, 8ull * n) != hipSuccess) return AVBD_ERR_ALLOC;
+  if (alloc_now(&dout, 4ull * n) != hipSuccess) {
+    free_now(dq);
     return AVBD_ERR_ALLOC;
   }
-  hipError_t e = hipMemcpy(dq, pairs, 8ull * n, hipMemcpyHostToDevice);
+  hipError_t e = copy_now(dq, pairs, 8ull * n, hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     StepParams P = make_params(s);
     if (soft) {
       if (P.softMapCapacity && s->S.softMapKeyA) launch_soft_map_find(s->stream, s->S, P, dq, dout, n);
-      else e = hipMemset(dout, 0xFF, 4ull * n);  // no element contacts: every key is absent
+      else e = fill_now(dout, 0xFF, 4ull * n);  // no element contacts: every key is absent
     } else {
       launch_map_find(s->stream, s->S, P, dq, dout, n);
     }
   }
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-  if (e == hipSuccess) e = hipMemcpy(out, dout, 4ull * n, hipMemcpyDeviceToHost);
-  hipFree(dq);
-  hipFree(dout);
+  if (e == hipSuccess) e = copy_now(out, dout, 4ull * n, hipMemcpyDeviceToHost);
+  free_now(dq);
+  free_now(dout);
   return e == hipSuccess ? AVBD_OK : AVBD_ERR_HIP;
 }
 
@@ -3433,7 +3430,7 @@ extern "C" avbd_status avbd_time_primal(avbd_solver* s, int32_t reps, float* avg
   if (read_dev(s, dlist, S.dAdjList, dtotal)) return AVBD_ERR_HIP;
   std::vector<ManifoldRec> mf;
   uint32_t npairs = 0;
-  hipMemcpy(&npairs, S.counters + CTR_PAIRS, 4, hipMemcpyDeviceToHost);
+  copy_now(&npairs, S.counters + CTR_PAIRS, 4, hipMemcpyDeviceToHost);
   if (read_dev(s, mf, (const ManifoldRec*)S.manifolds, npairs)) return AVBD_ERR_HIP;
   double bytes = 0.0;
   std::vector<uint32_t> sStart(s->nb);
@@ -3487,15 +3484,11 @@ extern "C" avbd_status avbd_time_primal(avbd_solver* s, int32_t reps, float* avg
     launch_fill_u32(s->stream, S.counters + CTR_COLOR_BASE, kMaxColors, 0u);
     launch_color_buckets(s->stream, S, P, S.colors);
   }
-  hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  hipError_t he = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
-  if (he == hipSuccess) {
+  hipError_t he = capture_graph(s, [&]() {
     sweeps();
-    he = hipStreamEndCapture(s->stream, &graph);
-  }
-  if (he == hipSuccess) he = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-  if (graph) hipGraphDestroy(graph);
+    return hipGetLastError();
+  }, &exec);
   if (he != hipSuccess) {
     hipGetLastError();
     return AVBD_ERR_HIP;
@@ -3504,7 +3497,7 @@ extern "C" avbd_status avbd_time_primal(avbd_solver* s, int32_t reps, float* avg
   // frame starts, and every sweep kernel returns at entry while it is set:
   // clear it for the timed sweeps and put it back afterwards
   uint32_t convDone = 0;
-  he = hipMemcpy(&convDone, s->S.counters + CTR_CONV_DONE, 4, hipMemcpyDeviceToHost);
+  he = copy_now(&convDone, s->S.counters + CTR_CONV_DONE, 4, hipMemcpyDeviceToHost);
   if (he == hipSuccess) he = hipMemsetAsync(s->S.counters + CTR_CONV_DONE, 0, 4, s->stream);
   if (he != hipSuccess) {
     hipGraphExecDestroy(exec);
@@ -3518,7 +3511,7 @@ extern "C" avbd_status avbd_time_primal(avbd_solver* s, int32_t reps, float* avg
   hipGraphLaunch(exec, s->stream);
   hipEventRecord(e1, s->stream);
   he = hipEventSynchronize(e1);
-  if (he == hipSuccess) he = hipMemcpy(s->S.counters + CTR_CONV_DONE, &convDone, 4, hipMemcpyHostToDevice);
+  if (he == hipSuccess) he = copy_now(s->S.counters + CTR_CONV_DONE, &convDone, 4, hipMemcpyHostToDevice);
   float ms = 0.0f;
   hipEventElapsedTime(&ms, e0, e1);
   hipEventDestroy(e0);
@@ -3649,9 +3642,9 @@ extern "C" avbd_status avbd_set_warm_start(avbd_solver* s, avbd_mlp* m, int32_t 
   }
   // a fresh attachment starts without correction history
   if (mode && !s->wsMode &&
-      (hipMemset(s->W.corr, 0, 16 * (size_t)s->nb) != hipSuccess ||
-       hipMemset(s->W.corrPrev, 0, 16 * (size_t)s->nb) != hipSuccess ||
-       hipMemset(s->W.corrAng, 0, 16 * (size_t)s->nb) != hipSuccess))
+      (fill_now(s->W.corr, 0, 16 * (size_t)s->nb) != hipSuccess ||
+       fill_now(s->W.corrPrev, 0, 16 * (size_t)s->nb) != hipSuccess ||
+       fill_now(s->W.corrAng, 0, 16 * (size_t)s->nb) != hipSuccess))
     return AVBD_ERR_HIP;
   s->wsMode = mode;
   if (!mode) {
@@ -3674,9 +3667,9 @@ extern "C" avbd_status avbd_get_warm_start_samples_rigid(avbd_solver* s, uint32_
   *n = s->W.nR;
   const size_t c = std::min(capacity, s->W.nR);
   if (c == 0) return AVBD_OK;
-  if ((x && hipMemcpy(x, s->W.logXR, c * kMlpIn * 4, hipMemcpyDeviceToHost)) ||
-      (t && hipMemcpy(t, s->W.logTR, c * kMlpOutRigid * 4, hipMemcpyDeviceToHost)) ||
-      (idx && hipMemcpy(idx, s->W.ridx, c * 4, hipMemcpyDeviceToHost)))
+  if ((x && copy_now(x, s->W.logXR, c * kMlpIn * 4, hipMemcpyDeviceToHost)) ||
+      (t && copy_now(t, s->W.logTR, c * kMlpOutRigid * 4, hipMemcpyDeviceToHost)) ||
+      (idx && copy_now(idx, s->W.ridx, c * 4, hipMemcpyDeviceToHost)))
     return AVBD_ERR_HIP;
   return AVBD_OK;
 }
@@ -3690,9 +3683,9 @@ extern "C" avbd_status avbd_get_warm_start_samples(avbd_solver* s, uint32_t capa
   *n = s->W.n;
   const size_t c = std::min(capacity, s->W.n);
   if (c == 0) return AVBD_OK;
-  if ((x && hipMemcpy(x, s->W.logX, c * kMlpIn * 4, hipMemcpyDeviceToHost)) ||
-      (t && hipMemcpy(t, s->W.logT, c * kMlpOut * 4, hipMemcpyDeviceToHost)) ||
-      (idx && hipMemcpy(idx, s->W.idx, c * 4, hipMemcpyDeviceToHost)))
+  if ((x && copy_now(x, s->W.logX, c * kMlpIn * 4, hipMemcpyDeviceToHost)) ||
+      (t && copy_now(t, s->W.logT, c * kMlpOut * 4, hipMemcpyDeviceToHost)) ||
+      (idx && copy_now(idx, s->W.idx, c * 4, hipMemcpyDeviceToHost)))
     return AVBD_ERR_HIP;
   return AVBD_OK;
 }
@@ -3767,10 +3760,10 @@ extern "C" avbd_status avbd_capture_speculation_snapshot(avbd_solver* s, avbd_sn
     return AVBD_ERR_INVALID_ARGUMENT;
   }
   if (snap->bytes != bytes) {  // grows when a learned warm start was attached since
-    if (snap->block) hipFree(snap->block);
+    if (snap->block) free_now(snap->block);
     snap->block = nullptr;
     snap->bytes = 0;
-    if (hipMalloc(&snap->block, bytes) != hipSuccess) {
+    if (alloc_now(&snap->block, bytes) != hipSuccess) {
       hipGetLastError();
       if (fresh) delete snap;
       return AVBD_ERR_ALLOC;
@@ -3832,7 +3825,7 @@ extern "C" avbd_status avbd_restore_speculation_snapshot(avbd_solver* s, const a
 namespace {
 
 void release_snapshot(avbd_snapshot* snap) {
-  if (snap->block) hipFree(snap->block);
+  if (snap->block) free_now(snap->block);
   delete snap;
 }
 

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "kernels.hpp"
+#include "gate.hpp"
 
 #pragma clang fp contract(off)
 
@@ -77,9 +78,9 @@ template <typename T>
 struct DevBuf {
   T* p = nullptr;
   ~DevBuf() {
-    if (p) (void)hipFree(p);
+    if (p) (void)free_now(p);
   }
-  hipError_t alloc(size_t n) { return hipMalloc((void**)&p, sizeof(T) * (n ? n : 1)); }
+  hipError_t alloc(size_t n) { return alloc_now(&p, sizeof(T) * (n ? n : 1)); }
 };
 
 }  // namespace
