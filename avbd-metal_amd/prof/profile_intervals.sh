@@ -6,11 +6,12 @@
 # known size.  Not traced by default: intervals iterated to a residual, and
 # block_55 and pile_300, whose creates launch cooperatively (the profiler then
 # ends with a segmentation fault of its own, after its results are written).
-# Run from the repo root on the GPU host; raw output under gpurun_out/prof_*.
+# Run from the repo root on a machine with the GPU; raw output under $OUT/prof_*.
 set -u
 cd "$(dirname "$0")/../.."
 export TMPDIR=/tmp
-OUT=gpurun_out
+OUT=${OUT:-/tmp/avbd_prof}
+mkdir -p "$OUT"
 if [ -z "${CASES:-}" ]; then
   /opt/rocm/bin/hipcc -O2 --offload-arch=gfx950 -o avbd-metal_amd/lib/copy_calib avbd-metal_amd/prof/copy_calib.hip || exit 1
   RUN="avbd-metal_amd/prof/interval.py block_20 1"

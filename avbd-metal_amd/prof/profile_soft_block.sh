@@ -4,12 +4,13 @@
 # benchmark, then one rocprofv3 PMC pass per counter (FETCH_SIZE, WRITE_SIZE)
 # on the benchmark and on the copy calibration kernel, then one pass of wave,
 # occupancy and LDS counters.  Run from the repo
-# root on the GPU host; writes raw output under gpurun_out/prof_* and the
+# root on a machine with the GPU; writes raw output under $OUT/prof_* and the
 # summaries via summarize.py.
 set -u
 cd "$(dirname "$0")/../.."
 export TMPDIR=/tmp
-OUT=gpurun_out
+OUT=${OUT:-/tmp/avbd_prof}
+mkdir -p "$OUT"
 CELLS=${CELLS:-20}
 BENCH="bench.py --cells $CELLS --steps 4 --warmup 2 --no-cpu --no-learned --quick --res-frames 0 --fp64-steps 0 --lanes ${LANES:-32} --sweep ${SWEEP:-1}"
 /opt/rocm/bin/hipcc -O2 --offload-arch=gfx950 -o avbd-metal_amd/lib/copy_calib avbd-metal_amd/prof/copy_calib.hip || exit 1
